@@ -218,6 +218,25 @@ int pdipc_debug_narrow_stage_layout(pdipc_handle* h, long long* sizes, int* tile
  * indices; taken by default wherever the narrow tiles fit). */
 int pdipc_sweep_staging(pdipc_handle* h, int* path);
 
+/* Tile solves: where a scene's system fits the registers of the device (8 lanes
+ * per row, sell_stage 1, about 130,000 rows at most) a whole Chebyshev solve is
+ * one launch whose workgroups exchange the iterates; the results are those of
+ * the streamed sweeps bit for bit.  info: [0] 1 if this handle has the tables,
+ * [1] / [2] 1 if its FP32 / FP64 solves run as tiles, [3] tiles, [4] rows per
+ * tile, [5] outer iterations repeated with the streamed sweeps because a tile
+ * gave up waiting for its neighbours.  request_abort != 0 makes the next tile
+ * solve give up (tests). */
+int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort);
+/* The tile tables for at most max_tiles tiles from the host precompute alone
+ * (after pdipc_host_setup; no device).  sizes: [0] 1 if the scene tiles, [1]
+ * tiles, [2] rows per tile, [3] halo rows in total, [4] threads per tile, [5]
+ * threads per row, [6] entries per lane, [7] LDS rows.  Then the tables, each
+ * skipped if null: rows (tiles x rows per tile, -1 past the last), halo_off
+ * (tiles + 1), halo, loc (per tile: an LDS index per thread and entry, 8-entry
+ * chunks by thread). */
+int pdipc_debug_tile_layout(pdipc_handle* h, int max_tiles, long long* sizes, int* rows, int* halo_off, int* halo,
+                            unsigned short* loc);
+
 /* --- no counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  The same minimum time of impact as pdipc_debug_toi over

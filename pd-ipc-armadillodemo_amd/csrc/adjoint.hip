@@ -117,6 +117,7 @@ struct AdjointState {
   bool lastKept = false;  // seg holds the last checkpoint segment, recorded by the rollout
   std::vector<double*> ckX, ckV;
   double *endX = nullptr, *endV = nullptr;
+  pdipc_handle* h = nullptr;  // the owner: its stream clears and fills the buffers below
   Pool tape;
   std::vector<StepTape> seg;
   double *ax = nullptr, *axo = nullptr, *asol = nullptr, *uA = nullptr, *uB = nullptr, *uC = nullptr, *uc = nullptr;
@@ -134,15 +135,16 @@ struct AdjointState {
   double* colRacc = nullptr;
   // local/global loops of the recorded forward and of the reverse pass,
   // captured once per collision flag
-  hipGraphExec_t fwdGraph[2] = {nullptr, nullptr};
+  hipGraphExec_t fwdGraph[2][2] = {};  // [tile solves][collision flag]
   hipGraphExec_t revGraph[2] = {nullptr, nullptr};
   double stats[4] = {0, 0, 0, 0};  // recorded outer iterations, tape bytes, segments, steps
 };
 
 void adjoint_free(AdjointState* a) {
   if (!a) return;
-  for (auto& g : a->fwdGraph)
-    if (g) (void)hipGraphExecDestroy(g);
+  for (auto& tiles : a->fwdGraph)
+    for (auto& g : tiles)
+      if (g) (void)hipGraphExecDestroy(g);
   for (auto& g : a->revGraph)
     if (g) (void)hipGraphExecDestroy(g);
   for (void* p : a->allocs) (void)hipFree(p);
@@ -158,14 +160,14 @@ template <class T>
 int dalloc(AdjointState* A, T** p, size_t n) {
   HIPCHK(hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T)));
   A->allocs.push_back(*p);
-  HIPCHK(hipMemset(*p, 0, std::max<size_t>(n, 1) * sizeof(T)));
+  HIPCHK(hipMemsetAsync(*p, 0, std::max<size_t>(n, 1) * sizeof(T), A->h->stream));
   return PDIPC_OK;
 }
 template <class T>
 int dupload(AdjointState* A, T** p, const std::vector<T>& v) {
   int rc = dalloc(A, p, v.size());
   if (rc) return rc;
-  if (!v.empty()) HIPCHK(hipMemcpy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+  if (!v.empty()) HIPCHK(A->h->copy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   return PDIPC_OK;
 }
 
@@ -173,6 +175,7 @@ int ensure_state(pdipc_handle* h) {
   if (h->adj) return PDIPC_OK;
   auto* A = new AdjointState();
   h->adj = A;
+  A->h = h;
   const HostSetup& hs = h->hs;
   const DeviceMesh& m = h->m;
   size_t V3 = 3 * (size_t)m.ld;
@@ -301,7 +304,7 @@ int adjoint_refresh_values(pdipc_handle* h) {
   std::vector<double> midA(A->midQ.size());
   for (size_t at = 0; at < midA.size(); at++) midA[at] = L.pA[A->midQ[at]];
   HIPCHK(hipStreamSynchronize(h->stream));
-  HIPCHK(hipMemcpy(A->am.midA, midA.data(), midA.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(h->copy(A->am.midA, midA.data(), midA.size() * sizeof(double), hipMemcpyHostToDevice));
   return PDIPC_OK;
 }
 
@@ -343,12 +346,13 @@ void enqueue_taped_lg(pdipc_handle* h, int withCol) {
   launch_diag(m, withCol, s);
   launch_copy(L.D(b), m.sysDiag, m.nSim, s);
   launch_operators(m, p.omega, PDIPC_FP64, s);
+  if (m.tile.use(PDIPC_FP64)) launch_tile_reset(m, s);
   std::vector<double*> outs(p.cheb_iters + 1);
   for (int l = 0; l < p.lg_iters; l++) {
     launch_local(m, PDIPC_FP64, p.sigma_lo, p.sigma_hi, withCol, s);
     launch_copy(L.rhs(b, l), m.sysRhs, (int64_t)L.V3, s);
     for (int k = 0; k <= p.cheb_iters; k++) outs[k] = L.it(b, l, k);
-    launch_solve_taped(m, p.omega, p.rho, p.cheb_iters, outs.data(), s);
+    launch_solve_taped(m, p.omega, p.rho, p.cheb_iters, outs.data(), s, l & 1);
   }
 }
 
@@ -376,30 +380,35 @@ int taped_step(pdipc_handle* h, StepTape& st) {
   for (; outer < p.max_outer; outer++) {
     OuterTape ot;
     ot.withCol = activeCol ? 1 : 0;
-    if ((rc = run_captured(h, A->fwdGraph[ot.withCol], [&]() { enqueue_taped_lg(h, ot.withCol); }))) return rc;
-    if ((rc = A->tape.alloc(A->lay.bytes(), (void**)&ot.blob))) return rc;
-    HIPCHK(hipMemcpyAsync(ot.blob, A->stage, A->lay.bytes(), hipMemcpyDeviceToDevice, s));
-    launch_direction(m, s);
-    if (outer == 0) {
-      if ((rc = broad_phase(h, m.Xold, m.Dir))) return rc;
-      st.nRecs = h->lastRecs;
-      if ((rc = A->tape.alloc((size_t)std::max(1, st.nRecs) * sizeof(int4), (void**)&st.recs))) return rc;
-      if (st.nRecs > 0)
-        HIPCHK(hipMemcpyAsync(st.recs, m.recs, (size_t)st.nRecs * sizeof(int4), hipMemcpyDeviceToDevice, s));
-      if (st.nRecs > A->recToiCap) {
-        if (A->recToi) {
-          (void)hipFree(A->recToi);
-          A->allocs.erase(std::find(A->allocs.begin(), A->allocs.end(), (void*)A->recToi));
+    auto iteration = [&]() -> int {
+      if ((rc = run_captured(h, A->fwdGraph[m.tile.use(PDIPC_FP64) ? 1 : 0][ot.withCol], [&]() { enqueue_taped_lg(h, ot.withCol); }))) return rc;
+      if ((rc = A->tape.alloc(A->lay.bytes(), (void**)&ot.blob))) return rc;
+      HIPCHK(hipMemcpyAsync(ot.blob, A->stage, A->lay.bytes(), hipMemcpyDeviceToDevice, s));
+      launch_direction(m, s);
+      if (outer == 0) {
+        if ((rc = broad_phase(h, m.Xold, m.Dir))) return rc;
+        st.nRecs = h->lastRecs;
+        if ((rc = A->tape.alloc((size_t)std::max(1, st.nRecs) * sizeof(int4), (void**)&st.recs))) return rc;
+        if (st.nRecs > 0)
+          HIPCHK(hipMemcpyAsync(st.recs, m.recs, (size_t)st.nRecs * sizeof(int4), hipMemcpyDeviceToDevice, s));
+        if (st.nRecs > A->recToiCap) {
+          if (A->recToi) {
+            (void)hipFree(A->recToi);
+            A->allocs.erase(std::find(A->allocs.begin(), A->allocs.end(), (void*)A->recToi));
+          }
+          A->recToiCap = st.nRecs + st.nRecs / 2 + 1024;
+          if ((rc = dalloc(A, &A->recToi, (size_t)A->recToiCap))) return rc;
         }
-        A->recToiCap = st.nRecs + st.nRecs / 2 + 1024;
-        if ((rc = dalloc(A, &A->recToi, (size_t)A->recToiCap))) return rc;
       }
-    }
-    HIPCHK(hipMemsetAsync(m.counters + 4, 0x7f, sizeof(int), s));  // (launch_direction reset the TOI minimum)
-    launch_ccd_records(m, m.recs, h->lastRecs, m.Xold, m.X, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
-                       p.touch_policy, A->recToi, m.counters + 4, s);
-    launch_clamp_residual(m, p.toi_scale, s);
-    if ((rc = collision(h))) return rc;  // reads the scalars back
+      HIPCHK(hipMemsetAsync(m.counters + 4, 0x7f, sizeof(int), s));  // (launch_direction reset the TOI minimum)
+      launch_ccd_records(m, m.recs, h->lastRecs, m.Xold, m.X, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
+                         p.touch_policy, A->recToi, m.counters + 4, s);
+      launch_clamp_residual(m, p.toi_scale, s);
+      return collision(h);  // reads the scalars back
+    };
+    rc = iteration();
+    if (rc == kTileAborted && !(rc = tile_recover(h, outer))) rc = iteration();
+    if (rc) return rc;
     activeCol = true;
     ot.nAct = h->hCounters()[2];
     if ((rc = A->tape.alloc((size_t)std::max(1, ot.nAct) * sizeof(int), (void**)&ot.act))) return rc;
@@ -525,6 +534,7 @@ int pdipc_rollout(pdipc_handle* h, int nsteps, int every) {
   if (h->prm.cheb_iters > kMaxCheb) return fail(PDIPC_E_ARG, "the adjoint supports at most 32 Chebyshev sweeps");
   if (h->prm.precision != PDIPC_FP64) return fail(PDIPC_E_ARG, "the adjoint runs on FP64 steps");
   if ((rc = ensure_state(h))) return rc;
+  TileTurn turn(h);
   AdjointState* A = h->adj;
   DeviceMesh& m = h->m;
   size_t V3 = 3 * (size_t)m.ld;
@@ -590,6 +600,7 @@ int pdipc_backward(pdipc_handle* h, const double* dx, const double* dv, double* 
   if (!A || A->nSteps < 1) return fail(PDIPC_E_ARG, "pdipc_backward needs a pdipc_rollout first");
   if (h->prm.precision != PDIPC_FP64) return fail(PDIPC_E_ARG, "the adjoint runs on FP64 steps");
   if (dk && nk < h->hs.nClothTris) return fail(PDIPC_E_ARG, "dL/dk holds fewer entries than the cloth triangles");
+  TileTurn turn(h);
   DeviceMesh& m = h->m;
   const HostSetup& hs = h->hs;
   hipStream_t s = h->stream;
@@ -645,9 +656,9 @@ int pdipc_backward(pdipc_handle* h, const double* dx, const double* dv, double* 
   if (dv0 && (rc = get_soa(h, vin, dv0, m.nSim))) return rc;
   if (dk) {
     std::vector<double> sb(hs.cNbr.size()), rb(hs.r1Col.size()), de(m.nSim);
-    HIPCHK(hipMemcpy(sb.data(), A->sbar, sb.size() * sizeof(double), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(rb.data(), A->R1bar, rb.size() * sizeof(double), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(de.data(), A->DbarEl, de.size() * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(h->copy(sb.data(), A->sbar, sb.size() * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(h->copy(rb.data(), A->R1bar, rb.size() * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(h->copy(de.data(), A->DbarEl, de.size() * sizeof(double), hipMemcpyDeviceToHost));
     // spring weight of a slot enters: the local step (sbar), R1(i, nbr) and the diagonal D_i
     std::vector<double> eg(hs.edgeTriOff.size(), 0.0);
     for (size_t c = 0; c < hs.cCenter.size(); c++) {
@@ -746,7 +757,7 @@ int pdipc_debug_tape(pdipc_handle* h, int step, int outer, int which, int l, int
   }
   if (!src) return fail(PDIPC_E_ARG, "no such recorded vector");
   if (which == 2) {
-    HIPCHK(hipMemcpy(out, src, h->m.nSim * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(h->copy(out, src, h->m.nSim * sizeof(double), hipMemcpyDeviceToHost));
     return PDIPC_OK;
   }
   return get_soa(h, src, out, h->m.nSim);

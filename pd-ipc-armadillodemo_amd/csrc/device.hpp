@@ -19,6 +19,12 @@ struct __align__(32) Row64 {
   double x, y, z, w;
 };
 
+// c = (w^2 sum_j R1_ij b_j / D_j + (2 - w) w b_i) / D_i of one component, given
+// the sum: one rounding sequence for every kernel that forms it
+__device__ __forceinline__ double first_term(double w, double sum, double b, double d) {
+  return __builtin_fma(w * w, sum, (2.0 - w) * w * b) / d;
+}
+
 // LBVH node for the stackless traversal: box rounded outward to float (a
 // superset of the exact box, used only to prune), the left child (internal
 // nodes) or the patch id (leaves), and the next node in depth-first preorder
@@ -50,6 +56,7 @@ enum TimerClass {
 struct KernelTimer {
   std::vector<hipEvent_t> pool;  // (start, stop) pairs
   std::vector<int> cls;          // class of each pair in use
+  std::vector<int> weight;       // launches each pair counts as (a tile solve: its sweeps)
   size_t used = 0;
   double us[TC_COUNT] = {};
   long long count[TC_COUNT] = {};
@@ -68,8 +75,13 @@ struct KernelTimer {
     *e0 = pool[2 * used];
     *e1 = pool[2 * used + 1];
     if (cls.size() <= used) cls.resize(used + 1);
+    if (weight.size() <= used) weight.resize(used + 1);
+    weight[used] = 1;
     cls[used++] = c;
     return true;
+  }
+  void weigh(int launches) {  // the last pair taken stands for this many launches
+    if (used) weight[used - 1] = launches;
   }
   ~KernelTimer() {
     for (hipEvent_t e : pool) (void)hipEventDestroy(e);
@@ -86,6 +98,28 @@ inline void launch_t(KernelTimer* t, int cls, void (*kernel)(KA...), dim3 grid, 
   else
     hipLaunchKernelGGL(kernel, grid, block, shm, s, args...);
 }
+
+// How the tile solves (k_tiles.hip) map a tile's rows to a workgroup: `tpr`
+// threads per row, each holding 8 / tpr lanes of `width` entries
+struct TileConfig {
+  int threads = 0, tpr = 0, width = 0;
+  bool laneMajor = false;
+};
+// Tables of the tile solves (host_setup.hpp, SolveTiles) on the device
+struct TileMesh {
+  bool built = false;               // tables present
+  bool ok32 = false, ok64 = false;  // every tile of the FP32 / FP64 solve is resident at once
+  bool on = false;                  // this handle may launch them now (it holds the device's turn)
+  TileConfig cfg;
+  int nTiles = 0, rowsPerTile = 0, uCap = 0;
+  int4* rows = nullptr;
+  int *haloOff = nullptr, *halo = nullptr;
+  uint16_t* loc = nullptr;
+  unsigned long long* slots = nullptr;  // two sets of four publication slots
+  double* cheb = nullptr;               // W_1 .. of the Chebyshev recurrence
+  int* abort = nullptr;                 // set by a tile that gave up waiting
+  bool use(int precision) const { return on && (precision == 0 ? ok64 : ok32); }
+};
 
 struct DeviceMesh {
   KernelTimer* timer = nullptr;  // in-step kernel timing (null: off)
@@ -151,6 +185,7 @@ struct DeviceMesh {
   uint16_t* ntileCol = nullptr;
   uint8_t* m2Loc8 = nullptr;
   int narrowStride = 0;
+  TileMesh tile;
   // collision topology
   int nFaces = 0, nEdges = 0, nPatches = 0;
   int3* bFaces = nullptr;
@@ -221,10 +256,18 @@ void launch_copy(double* dst, const double* src, int64_t n, hipStream_t s);
 // launched with residualReady
 void launch_local(const DeviceMesh& m, int precision, double sigLo, double sigHi, int withCollision, hipStream_t s,
                   double residualOmega = -1.0);
+// k_tiles.hip: one launch per Chebyshev solve (launch_solve picks them while
+// m.tile.use(); launch_tile_reset before the first of a sequence, whose
+// launches then alternate parity 0, 1, 0, ...)
+void tile_check(DeviceMesh& m, int cus, int iters);
+void launch_tile_reset(const DeviceMesh& m, hipStream_t s);
+void launch_tile_solve32(const DeviceMesh& m, int iters, int parity, hipStream_t s);
+void launch_tile_solve64(const DeviceMesh& m, double w, int iters, int parity, double* out, int64_t outStride,
+                         hipStream_t s);
 // k_solve.hip
 void launch_operators(const DeviceMesh& m, double omega, int precision, hipStream_t s);
 void launch_solve(const DeviceMesh& m, double omega, double rho, int chebIters, int precision, hipStream_t s,
-                  bool residualReady = false);
+                  bool residualReady = false, int parity = 0);
 // one Chebyshev sweep of the given precision (measurement support)
 void launch_one_sweep(const DeviceMesh& m, int precision, hipStream_t s);
 // k_contact.hip
@@ -249,7 +292,8 @@ struct AdjMesh {
   int *uOff = nullptr, *uCol = nullptr;
   uint16_t* uPos = nullptr;
 };
-void launch_solve_taped(const DeviceMesh& m, double omega, double rho, int iters, double* const* outs, hipStream_t s);
+void launch_solve_taped(const DeviceMesh& m, double omega, double rho, int iters, double* const* outs, hipStream_t s,
+                        int parity = 0);
 // the whole reverse of one K-sweep solve: u[k] for k = K-1 .. 0 from u[K] (given)
 // and u[K+1] (zero), then one SELL pass adding sum_k W_k u_{k+1} x_k^T to Gbar,
 // with the forward iterates x_0 and x_k = x1 + (k-1) xStride (k >= 1)

@@ -41,11 +41,12 @@ struct pdipc_handle {
   DeviceMesh m;
   hipStream_t stream = nullptr;
   int device = 0;  // the HIP device current at pdipc_init
-  // local/global loop captured once per (collision flag, precision) and replayed
-  hipGraphExec_t lgGraph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+  // local/global loop captured once per (tile solves, collision flag, precision) and replayed
+  hipGraphExec_t lgGraph[2][2][2] = {};
+  int tileAborts = 0;  // outer iterations repeated with the streamed sweeps
   std::vector<void*> allocs;
   // host mirrors
-  void* scalHost = nullptr;  // pinned: residual, toiBits, counters[10]
+  void* scalHost = nullptr;  // pinned: residual, toiBits, counters[12], the tile solves' abort flag
   void* scalDev = nullptr;
   std::vector<double> stage;
   pdipc_counters cnt;
@@ -61,11 +62,17 @@ struct pdipc_handle {
     allocs.push_back(*p);
     return PDIPC_OK;
   }
+  // Copies and waits on the handle's own stream: the legacy stream must not be
+  // used while another thread's handle captures its graphs.
+  hipError_t copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, stream);
+    return e != hipSuccess ? e : hipStreamSynchronize(stream);
+  }
   template <class T>
   int upload(T** p, const std::vector<T>& v) {
     int rc = alloc(p, v.size());
     if (rc) return rc;
-    if (!v.empty()) HIPCHK(hipMemcpy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+    if (!v.empty()) HIPCHK(copy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
     return PDIPC_OK;
   }
   void release(void* p) {
@@ -85,16 +92,18 @@ struct pdipc_handle {
     if (stream) (void)hipStreamDestroy(stream);
   }
   void drop_graphs() {
-    for (auto& row : lgGraph)
-      for (auto& g : row)
-        if (g) {
-          (void)hipGraphExecDestroy(g);
-          g = nullptr;
-        }
+    for (auto& tiles : lgGraph)
+      for (auto& row : tiles)
+        for (auto& g : row)
+          if (g) {
+            (void)hipGraphExecDestroy(g);
+            g = nullptr;
+          }
   }
   double* hResidual() { return (double*)scalHost; }
   unsigned long long* hToi() { return (unsigned long long*)((char*)scalHost + 8); }
   int* hCounters() { return (int*)((char*)scalHost + 16); }
+  int hTileAbort() { return *(int*)((char*)scalHost + 64); }
 };
 
 
@@ -108,6 +117,27 @@ int broad_phase(pdipc_handle* h, const double* x, const double* dx);
 int collision(pdipc_handle* h);
 int require_device(pdipc_handle* h);
 int advance(pdipc_handle* h);
+// The tile solves wait for each other, so only one handle per device launches
+// them at a time: a call that runs solves holds the device's turn for its
+// duration, or, when another thread's handle has it, runs the streamed sweeps
+// (the same results bit for bit).
+class TileTurn {
+ public:
+  explicit TileTurn(pdipc_handle* h);
+  ~TileTurn();
+  TileTurn(const TileTurn&) = delete;
+  TileTurn& operator=(const TileTurn&) = delete;
+
+ private:
+  pdipc_handle* h_;
+  bool held_ = false;
+};
+// returned by read_scalars (and what calls it) when a tile solve gave up
+// waiting; tile_recover clears the flag, switches the handle to the streamed
+// sweeps for the rest of the call and restores X as the outer iteration
+// found it
+constexpr int kTileAborted = 1000;
+int tile_recover(pdipc_handle* h, int outer);
 int adjoint_refresh_values(pdipc_handle* h);  // adjoint.hip: after a stiffness change
 int noalloc_setup(int device);                 // noalloc.hip: with `device` current
 }  // namespace pdipc

@@ -27,9 +27,10 @@ int setup_threads() {
 }
 
 // fn(begin, end, t) over `parts` contiguous ranges of [0, n), one thread each
+// (fewer when a range would hold less than `grain` items)
 template <class F>
-void parallel_ranges(int64_t n, int parts, F fn) {
-  parts = (int)std::max<int64_t>(1, std::min<int64_t>(parts, n / 1024 + 1));
+void parallel_ranges(int64_t n, int parts, F fn, int64_t grain = 1024) {
+  parts = (int)std::max<int64_t>(1, std::min<int64_t>(parts, n / grain + 1));
   std::vector<std::thread> th;
   for (int t = 0; t < parts; t++) {
     int64_t b = n * t / parts, e = n * (t + 1) / parts;
@@ -545,6 +546,8 @@ std::string build_host_setup(const std::vector<ModelInput>& sims, const std::vec
     nPts += nv;
   }
   hs.nSim = nPts;
+  hs.modelBase.assign(base.begin(), base.begin() + sims.size());
+  hs.modelBase.push_back(nPts);
   hs.nTets = (int)hs.tetW.size();
   for (size_t si = 0; si < statics.size(); si++) {
     const ModelInput& m = statics[si];
@@ -966,6 +969,140 @@ void build_sell(const HostSetup& hs, int lanes, SellLayout& L) {
       std::copy(hs.p2Ib.begin() + hs.p2Off[q], hs.p2Ib.begin() + hs.p2Off[q + 1], L.pIb.begin() + L.pOff[e]);
     }
   });
+}
+
+// Points [lo, hi) of `order` (one model) by recursive bisection across the
+// longest side of their bounding box, every cut at a multiple of R, so that
+// each run of R points between multiples is compact; ties by id.
+static void bisect_points(const HostSetup& hs, int R, int lo, int hi, std::vector<int>& order) {
+  while (hi - lo > 1 && lo / R != (hi - 1) / R) {
+    double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+    for (int p = lo; p < hi; p++)
+      for (int k = 0; k < 3; k++) {
+        const double v = hs.X[3 * (size_t)order[p] + k];
+        mn[k] = std::min(mn[k], v);
+        mx[k] = std::max(mx[k], v);
+      }
+    int ax = 0;
+    for (int k = 1; k < 3; k++)
+      if (mx[k] - mn[k] > mx[ax] - mn[ax]) ax = k;
+    const int first = (lo / R + 1) * R, last = (hi - 1) / R * R;  // the multiples inside (lo, hi)
+    const int cut = std::min(last, std::max(first, (int)(((int64_t)lo + hi + R) / 2 / R * R)));
+    std::nth_element(order.begin() + lo, order.begin() + cut, order.begin() + hi, [&](int a, int b) {
+      const double u = hs.X[3 * (size_t)a + ax], v = hs.X[3 * (size_t)b + ax];
+      return u != v ? u < v : a < b;
+    });
+    bisect_points(hs, R, lo, cut, order);
+    lo = cut;
+  }
+}
+
+void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, SolveTiles& T) {
+  T = SolveTiles();
+  const int n = hs.nSim;
+  if (L.lanes != 8 || n < 1 || maxTiles < 1 || L.sliceOff.back() > INT32_MAX) return;
+  // One tile while a workgroup's own LDS reads cost less than an exchange
+  // (FP64 solve of 144 rows 32 us, as five tiles 36; of 576 rows 55 us as three
+  // tiles of 256 rows, 37 as tiles of 32); then small tiles until every compute
+  // unit has one (rows per tile 32 / 64 / 128, FP64 solves: 64^2 cloth 38 / 40 /
+  // 45 us, 13^3-cell tet block 51 / 55 / 58 us), then as many rows as that takes.
+  const int R = n <= 160 ? n : std::max(32, (n + maxTiles - 1) / maxTiles);
+  if (R <= 64) T.threads = 256, T.tpr = 4;
+  else if (R <= 128) T.threads = 512, T.tpr = 4;
+  else if (R <= 256) T.threads = 512, T.tpr = 2;
+  else if (R <= 512) T.threads = 512, T.tpr = 1;
+  else return;  // the entries would not fit a workgroup's registers
+  const int wmax = L.nSlices > 0 ? *std::max_element(L.sliceW.begin(), L.sliceW.end()) : 0;
+  T.width = wmax <= 8 ? 8 : 12;
+  if (wmax > 12) return;
+  T.rowsPerTile = R;
+  T.nTiles = (n + R - 1) / R;
+  std::vector<int> order(n);
+  std::iota(order.begin(), order.end(), 0);
+  for (size_t m = 0; m + 1 < hs.modelBase.size(); m++) bisect_points(hs, R, hs.modelBase[m], hs.modelBase[m + 1], order);
+  T.rows.assign((size_t)T.nTiles * R, -1);
+  std::vector<int> owner(n);
+  for (int t = 0; t < T.nTiles; t++) {
+    const int b = t * R, e = std::min(n, b + R);
+    std::copy(order.begin() + b, order.begin() + e, T.rows.begin() + b);
+    std::sort(T.rows.begin() + b, T.rows.begin() + e);
+    for (int p = b; p < e; p++) owner[T.rows[p]] = t;
+  }
+  const int nt = setup_threads();
+  std::vector<std::vector<int>> halo(T.nTiles);
+  auto each_entry = [&](int row, auto&& fn) {
+    for (int q = hs.m2Off[row]; q < hs.m2Off[row + 1]; q++) fn(hs.m2Col[q]);
+  };
+  parallel_ranges(T.nTiles, nt, [&](int64_t t0, int64_t t1, int) {
+    for (int t = (int)t0; t < (int)t1; t++) {
+      std::vector<int>& H = halo[t];
+      for (int r = 0; r < R; r++)
+        if (const int row = T.rows[(size_t)t * R + r]; row >= 0)
+          each_entry(row, [&](int c) {
+            if (owner[c] != t) H.push_back(c);
+          });
+      std::sort(H.begin(), H.end());
+      H.erase(std::unique(H.begin(), H.end()), H.end());
+    }
+  }, 8);
+  // The exchange needs a symmetric neighbour relation.  M^2's pattern is
+  // symmetric up to entries at the drop threshold: where tile a reads b but b
+  // does not read a, b also reads one row of a.
+  std::vector<std::vector<int>> reads(T.nTiles);
+  for (int t = 0; t < T.nTiles; t++) {
+    for (int r : halo[t]) reads[t].push_back(owner[r]);
+    std::sort(reads[t].begin(), reads[t].end());
+    reads[t].erase(std::unique(reads[t].begin(), reads[t].end()), reads[t].end());
+  }
+  for (int t = 0; t < T.nTiles; t++)
+    for (int o : reads[t])
+      if (!std::binary_search(reads[o].begin(), reads[o].end(), t)) {
+        std::vector<int>& H = halo[o];
+        const int row = T.rows[(size_t)t * R];
+        H.insert(std::upper_bound(H.begin(), H.end(), row), row);
+      }
+  T.haloOff.assign(1, 0);
+  size_t most = 0;
+  for (auto& H : halo) {
+    T.halo.insert(T.halo.end(), H.begin(), H.end());
+    T.haloOff.push_back((int)T.halo.size());
+    most = std::max(most, H.size());
+  }
+  T.uCap = (int)(((size_t)R + most + 7) / 8 * 8);
+  // the staged FP32 rows must fit the 160 KB of LDS (FP64 ones are checked
+  // against the device) and an index 16 bits
+  if ((size_t)T.uCap * 12 > (160u << 10)) return;
+  const int BT = T.threads, rw = 64 / T.tpr, subs = 8 / T.tpr, E = subs * T.width;
+  T.loc.assign((size_t)T.nTiles * E * BT, 0);
+  T.rowEntry.assign(T.rows.size(), 0);
+  T.rowWidth.assign(T.rows.size(), 0);
+  parallel_ranges(T.nTiles, nt, [&](int64_t t0, int64_t t1, int) {
+    std::vector<int> place(n, 0);
+    for (int t = (int)t0; t < (int)t1; t++) {
+      for (int r = 0; r < R; r++)
+        if (const int row = T.rows[(size_t)t * R + r]; row >= 0) place[row] = r;
+      for (size_t u = 0; u < halo[t].size(); u++) place[halo[t][u]] = R + (int)u;
+      uint16_t* loc = T.loc.data() + (size_t)t * E * BT;
+      for (int r = 0; r < R; r++) {
+        const int row = T.rows[(size_t)t * R + r];
+        if (row < 0) continue;
+        const int slot = L.slotOf.empty() ? row : L.slotOf[row], s = slot / 8;
+        T.rowEntry[(size_t)t * R + r] = (int)L.entry(s, (slot % 8) * 8, 0);
+        T.rowWidth[(size_t)t * R + r] = L.sliceW[s];
+        for (int part = 0; part < T.tpr; part++) {
+          const int th = (r / rw) * 64 + part * rw + r % rw;
+          for (int g = 0; g < subs; g++)
+            for (int c = 0; c < T.width; c++) {
+              const int e = g * T.width + c;
+              const int lane = (slot % 8) * 8 + part + g * T.tpr;
+              loc[((size_t)(e / 8) * BT + th) * 8 + e % 8] =
+                  c < L.sliceW[s] ? (uint16_t)place[L.col[L.entry(s, lane, c)]] : (uint16_t)r;
+            }
+        }
+      }
+    }
+  }, 8);
+  T.ok = true;
 }
 
 }  // namespace pdipc

@@ -79,6 +79,7 @@ struct HostSetup {
   std::vector<int> peOff, peList;        // patch -> owned edges
   std::vector<uint8_t> patchStatic;      // 1 if the patch belongs to a static model
   std::vector<double> colMass;           // nTotal
+  std::vector<int> modelBase;            // simulated models: first point of each, then nSim
   // fixture images (boundary.dat / patchInfo.dat) per simulated model
   std::vector<std::vector<int>> boundaryDat, patchDat;
   int64_t nnzR1 = 0, nnzR2 = 0, n2paths = 0;
@@ -159,5 +160,25 @@ constexpr int kStageMaxCols = 1024; // largest staged union (16 KiB of FP32 rows
 constexpr int kNarrowTileSlices = 2;  // slices per narrow tile (a 128-lane workgroup)
 constexpr int kNarrowMaxCols = 256;   // largest narrow union (8-bit indices)
 void build_sell(const HostSetup& hs, int lanes, SellLayout& out);
+
+// Tiles of the single-launch Chebyshev solves (k_tiles.hip) for a SELL layout
+// of 8 lanes per row: the simulated points ordered by recursive bisection of
+// their initial positions, model by model, cut every `rowsPerTile` points; the
+// rows of a tile ascend.  Thread (row rl, part) of a tile holds the SELL lanes
+// part, part + tpr, ... of the row: thread (rl / rw) * 64 + part * rw + rl % rw
+// with rw = 64 / tpr; its entry g * width + c is chunk c of lane part + g * tpr.
+// `loc` is an entry's LDS index: the row's place in the tile, or rowsPerTile +
+// its place in the tile's halo; padding entries point at the thread's own row.
+struct SolveTiles {
+  bool ok = false;
+  int rowsPerTile = 0, nTiles = 0, threads = 0, tpr = 0, width = 0, uCap = 0;
+  std::vector<int> rows;      // nTiles * rowsPerTile, -1 past the last row
+  std::vector<int> rowEntry;  // per row of `rows`: the SELL entry of its lane 0, chunk 0
+  std::vector<int> rowWidth;  // and its slice's entries per lane
+  std::vector<int> haloOff;   // nTiles + 1
+  std::vector<int> halo;      // ascending per tile
+  std::vector<uint16_t> loc;  // [tile][8-entry chunk][thread][8]
+};
+void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, SolveTiles& out);
 
 }  // namespace pdipc

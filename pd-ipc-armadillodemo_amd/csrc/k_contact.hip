@@ -506,11 +506,13 @@ __global__ void k_col_rank(int nSim, int cap, const int* __restrict__ ptOff, con
   }
 }
 
-__global__ void k_col_gather(int nSim, int ld, const int* __restrict__ ptOff,
+// `abort` (when given): a tile solve of this outer iteration gave up and the
+// host repeats the iteration, which reads the terms of the one before
+__global__ void k_col_gather(int nSim, int ld, const int* __restrict__ abort, const int* __restrict__ ptOff,
                              const unsigned long long* __restrict__ entSorted, const double* __restrict__ actW,
                              const double* __restrict__ actT, double* __restrict__ diag, double* __restrict__ rhs) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nSim) return;
+  if (i >= nSim || (abort && *abort)) return;
   int o = ptOff[i], e = ptOff[i + 1];
   double d = 0.0, r[3] = {0.0, 0.0, 0.0};
   for (int p = o; p < e; p++) {
@@ -773,7 +775,7 @@ int launch_collision(DeviceMesh& m, int nRecs, double dhat, double kappa, double
   launch_t(m.timer, TC_BARRIER, k_col_rank, dim3(512), dim3(kBlock), 0, s, m.nSim, 4 * m.actCap, m.ptOff, m.entKey,
            m.entA, m.entPt, m.entSorted);
   launch_t(m.timer, TC_BARRIER, k_col_gather, dim3((m.nSim + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nSim, m.ld,
-           m.ptOff, m.entSorted, m.actW, m.actT, m.colDiag, m.colRhs);
+           m.tile.on ? m.tile.abort : (const int*)nullptr, m.ptOff, m.entSorted, m.actW, m.actT, m.colDiag, m.colRhs);
   return 0;
 }
 

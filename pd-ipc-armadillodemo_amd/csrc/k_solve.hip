@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(kBlock, 8) k_first64(int n, int nSlices, int l
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     int idx = k * ld + row;
-    c[k] = (ft.w * ft.w * cr[k] + (2.0 - ft.w) * ft.w * ft.b[idx]) / di;
+    c[k] = first_term(ft.w, cr[k], ft.b[idx], di);
     y[k] = acc[k] + c[k];
     x0[k] = X[idx];
   }
@@ -685,7 +685,7 @@ __global__ void __launch_bounds__(kBlock, 8) k_first64s(int n, int nSlices, int 
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     const int idx = k * ld + row;
-    c[k] = (ft.w * ft.w * cr[k] + (2.0 - ft.w) * ft.w * ft.b[idx]) / di;
+    c[k] = first_term(ft.w, cr[k], ft.b[idx], di);
     y[k] = acc[k] + c[k];
     x0[k] = X[idx];
   }
@@ -926,7 +926,14 @@ void launch_sweep32(const DeviceMesh& m, int grid, float W, const float4* cur, c
 // forward pass) receives every iterate x_1 .. x_iters in SoA as well; both
 // forms run the same kernels, so their iterates are bit-identical.
 template <int G>
-void solve64(const DeviceMesh& m, double w, double rho, int iters, double* const* outs, hipStream_t s) {
+void solve64(const DeviceMesh& m, double w, double rho, int iters, double* const* outs, int parity, hipStream_t s) {
+  if constexpr (G == 8) {
+    if (m.tile.use(0)) {
+      const int64_t stride = outs && iters > 1 ? outs[2] - outs[1] : 0;  // the recorded iterates are equally spaced
+      launch_tile_solve64(m, w, iters, parity, outs ? outs[1] : nullptr, stride, s);
+      return;
+    }
+  }
   const int grid = (m.nSlices * kWave + kBlock - 1) / kBlock;
   const FirstTermArgs ft{m.r1Off, m.r1Col, m.r1Val, m.sysDiag, m.sysRhs, w};
   double r = rho * rho;
@@ -992,10 +999,10 @@ void solve64(const DeviceMesh& m, double w, double rho, int iters, double* const
 }
 
 template <int G>
-void solve_impl(const DeviceMesh& m, double w, double rho, int iters, int precision, bool residualReady,
+void solve_impl(const DeviceMesh& m, double w, double rho, int iters, int precision, bool residualReady, int parity,
                 hipStream_t s) {
   if (precision == 0) {
-    solve64<G>(m, w, rho, iters, nullptr, s);
+    solve64<G>(m, w, rho, iters, nullptr, parity, s);
     return;
   }
   const int grid = (m.nSlices * kWave + kBlock - 1) / kBlock;
@@ -1010,6 +1017,12 @@ void solve_impl(const DeviceMesh& m, double w, double rho, int iters, int precis
              m.r1Val, m.sysDiag, m.X, m.sysRhs, m.xa0, m.cA);
   launch_t(m.timer, TC_FIRST, k_res_b<GR>, dim3(gridR), dim3(kBlock), 0, s, m.nSim, w, m.r1Off, m.r1Col, m.r1Val,
            m.sysDiag, m.xa0, m.cA, pre, cur, m.r0);
+  if constexpr (G == 8) {
+    if (m.tile.use(1)) {
+      launch_tile_solve32(m, iters, parity, s);
+      return;
+    }
+  }
   if (iters <= 1) {
     hipLaunchKernelGGL(k_apply_delta, dim3((m.nSim + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nSim, m.ld, cur,
                        m.X);
@@ -1406,12 +1419,13 @@ void launch_operators(const DeviceMesh& m, double omega, int precision, hipStrea
            omega, m.m2RowFlag, m.dDirty, m.m2R1, m.p2Off, m.p2K, m.p2A, m.sysDiag, m.m2Val, m.m2ValF);
 }
 
-void launch_solve_taped(const DeviceMesh& m, double omega, double rho, int iters, double* const* outs, hipStream_t s) {
+void launch_solve_taped(const DeviceMesh& m, double omega, double rho, int iters, double* const* outs, hipStream_t s,
+                        int parity) {
   switch (m.sellLanes) {
-    case 1: solve64<1>(m, omega, rho, iters, outs, s); break;
-    case 2: solve64<2>(m, omega, rho, iters, outs, s); break;
-    case 8: solve64<8>(m, omega, rho, iters, outs, s); break;
-    default: solve64<4>(m, omega, rho, iters, outs, s); break;
+    case 1: solve64<1>(m, omega, rho, iters, outs, parity, s); break;
+    case 2: solve64<2>(m, omega, rho, iters, outs, parity, s); break;
+    case 8: solve64<8>(m, omega, rho, iters, outs, parity, s); break;
+    default: solve64<4>(m, omega, rho, iters, outs, parity, s); break;
   }
 }
 
@@ -1455,12 +1469,12 @@ void launch_adj_ops_gather(const DeviceMesh& m, const AdjMesh& a, double omega, 
 }
 
 void launch_solve(const DeviceMesh& m, double omega, double rho, int iters, int precision, hipStream_t s,
-                  bool residualReady) {
+                  bool residualReady, int parity) {
   switch (m.sellLanes) {
-    case 1: solve_impl<1>(m, omega, rho, iters, precision, residualReady, s); break;
-    case 2: solve_impl<2>(m, omega, rho, iters, precision, residualReady, s); break;
-    case 8: solve_impl<8>(m, omega, rho, iters, precision, residualReady, s); break;
-    default: solve_impl<4>(m, omega, rho, iters, precision, residualReady, s); break;
+    case 1: solve_impl<1>(m, omega, rho, iters, precision, residualReady, parity, s); break;
+    case 2: solve_impl<2>(m, omega, rho, iters, precision, residualReady, parity, s); break;
+    case 8: solve_impl<8>(m, omega, rho, iters, precision, residualReady, parity, s); break;
+    default: solve_impl<4>(m, omega, rho, iters, precision, residualReady, parity, s); break;
   }
 }
 

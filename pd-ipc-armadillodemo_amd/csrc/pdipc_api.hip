@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -66,9 +67,79 @@ int check_launch(pdipc_handle* h) {
   return PDIPC_OK;
 }
 
+constexpr size_t kScalarBytes = 128;
+
 int read_scalars(pdipc_handle* h) {
-  HIPCHK(hipMemcpyAsync(h->scalHost, h->scalDev, 64, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(hipMemcpyAsync(h->scalHost, h->scalDev, kScalarBytes, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
+  return h->m.tile.on && h->hTileAbort() ? kTileAborted : PDIPC_OK;
+}
+
+// ---- tile solves
+namespace {
+std::atomic<int> g_tileTurn[64];  // per device: 1 while a handle may launch tile solves
+constexpr int kTileMaxAborts = 2;  // a handle that gave up this often keeps to the streamed sweeps
+}  // namespace
+
+TileTurn::TileTurn(pdipc_handle* h) : h_(h) {
+  TileMesh& t = h->m.tile;
+  t.on = false;
+  if (!t.built || h->tileAborts >= kTileMaxAborts || h->device < 0 || h->device >= 64) return;
+  int free = 0;
+  held_ = g_tileTurn[h->device].compare_exchange_strong(free, 1);
+  t.on = held_;
+}
+TileTurn::~TileTurn() {
+  h_->m.tile.on = false;
+  if (!held_) return;
+  (void)hipStreamSynchronize(h_->stream);  // no solve of this handle is left on the device
+  g_tileTurn[h_->device].store(0);
+}
+
+int tile_recover(pdipc_handle* h, int outer) {
+  DeviceMesh& m = h->m;
+  h->tileAborts++;
+  m.tile.on = false;
+  HIPCHK(hipMemsetAsync(m.tile.abort, 0, sizeof(int), h->stream));
+  launch_copy(m.X, outer == 0 ? m.X0 : m.Xold, 3 * (int64_t)m.ld, h->stream);
+  if (outer == 0) launch_predict(m, h->prm.dt, h->stream);
+  return check_launch(h);
+}
+
+// builds and uploads the tiles; without them (rows too many or too wide, or
+// sell_stage other than 1) the streamed sweeps run
+int upload_tiles(pdipc_handle* h) {
+  DeviceMesh& m = h->m;
+  if (h->prm.sell_stage != 1) return PDIPC_OK;
+  int cus = 0;
+  HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
+  SolveTiles T;
+  build_solve_tiles(h->hs, h->sell, cus, T);
+  if (!T.ok) return PDIPC_OK;
+  TileMesh& t = m.tile;
+  t.cfg.threads = T.threads;
+  t.cfg.tpr = T.tpr;
+  t.cfg.width = T.width;
+  t.cfg.laneMajor = h->sell.laneMajor();
+  t.nTiles = T.nTiles;
+  t.rowsPerTile = T.rowsPerTile;
+  t.uCap = T.uCap;
+  tile_check(m, cus, h->prm.cheb_iters);
+  if (!t.ok32 && !t.ok64) return PDIPC_OK;
+  // the sweeps' weights, as the streamed solves compute them
+  std::vector<double> W(std::max(1, h->prm.cheb_iters));
+  const double r = h->prm.rho * h->prm.rho;
+  W[0] = 2.0 / (2.0 - r);
+  for (size_t k = 1; k < W.size(); k++) W[k] = 4.0 / (4.0 - r * W[k - 1]);
+  std::vector<int4> rows(T.rows.size());
+  for (size_t i = 0; i < rows.size(); i++) rows[i] = make_int4(T.rows[i], T.rowEntry[i], T.rowWidth[i], 0);
+  int rc;
+  if ((rc = h->upload(&t.rows, rows)) || (rc = h->upload(&t.haloOff, T.haloOff)) ||
+      (rc = h->upload(&t.halo, T.halo)) || (rc = h->upload(&t.loc, T.loc)) || (rc = h->upload(&t.cheb, W)) ||
+      (rc = h->alloc(&t.slots, 2 * 12 * (size_t)m.ld)))
+    return rc;
+  t.abort = (int*)((char*)h->scalDev + 64);
+  t.built = true;
   return PDIPC_OK;
 }
 
@@ -91,19 +162,19 @@ int upload_all(pdipc_handle* h) {
   AL(initRhs, V3); AL(sysRhs, V3); AL(firstTerm, V3); AL(colRhs, V3); AL(clothA, V3); AL(Xrest, V3);
   AL(dPre, m.ld); AL(dCur, m.ld); AL(dNext, m.ld); AL(r0, m.ld);
   AL(xa0, m.ld); AL(xa1, m.ld); AL(xa2, m.ld); AL(cA, m.ld);
-  for (Row64* p : {m.xa0, m.xa1, m.xa2, m.cA}) HIPCHK(hipMemset(p, 0, m.ld * sizeof(Row64)));
+  for (Row64* p : {m.xa0, m.xa1, m.xa2, m.cA}) HIPCHK(hipMemsetAsync(p, 0, m.ld * sizeof(Row64), h->stream));
   for (double* p : {m.X, m.Xold, m.X0, m.Dir, m.Pre, m.Next, m.V, m.initRhs, m.sysRhs, m.firstTerm, m.colRhs, m.clothA,
                     m.Xrest})
-    HIPCHK(hipMemset(p, 0, V3 * sizeof(double)));
-  for (float4* p : {m.dPre, m.dCur, m.dNext, m.r0}) HIPCHK(hipMemset(p, 0, m.ld * sizeof(float4)));
+    HIPCHK(hipMemsetAsync(p, 0, V3 * sizeof(double), h->stream));
+  for (float4* p : {m.dPre, m.dCur, m.dNext, m.r0}) HIPCHK(hipMemsetAsync(p, 0, m.ld * sizeof(float4), h->stream));
   UP(mass, hs.mass); UP(invMass, hs.invMass); UP(gravY, hs.gravY); UP(fixK, hs.fixK); UP(fixFlag, hs.fixFlag);
   UP(colMass, hs.colMass); UP(elasticDiag, hs.elasticDiag);
   AL(inertialDiag, hs.nSim); AL(sysDiag, hs.nSim); AL(colDiag, hs.nTotal);
   AL(dStale, hs.nSim); AL(dChanged, hs.nSim); AL(dDirty, hs.nSim);
-  HIPCHK(hipMemset(m.dStale, 1, std::max(1, hs.nSim)));  // first update recomputes every row
-  HIPCHK(hipMemset(m.sysDiag, 0, std::max(1, hs.nSim) * sizeof(double)));
-  HIPCHK(hipMemset(m.inertialDiag, 0, std::max(1, hs.nSim) * sizeof(double)));
-  HIPCHK(hipMemset(m.colDiag, 0, std::max(1, hs.nTotal) * sizeof(double)));
+  HIPCHK(hipMemsetAsync(m.dStale, 1, std::max(1, hs.nSim), h->stream));  // first update recomputes every row
+  HIPCHK(hipMemsetAsync(m.sysDiag, 0, std::max(1, hs.nSim) * sizeof(double), h->stream));
+  HIPCHK(hipMemsetAsync(m.inertialDiag, 0, std::max(1, hs.nSim) * sizeof(double), h->stream));
+  HIPCHK(hipMemsetAsync(m.colDiag, 0, std::max(1, hs.nTotal) * sizeof(double), h->stream));
   UP(cCenter, hs.cCenter); UP(cOff, hs.cOff.empty() ? std::vector<int>{0} : hs.cOff); UP(cNbr, hs.cNbr);
   UP(clothOfPoint, hs.clothOfPoint); UP(cRest, hs.cRest); UP(cLbo, hs.cLbo); UP(cBendIn, hs.cBendIn);
   {
@@ -225,22 +296,22 @@ int upload_all(pdipc_handle* h) {
   AL(checkCount, 1);
   // scalars: residual (8), toiBits (8), counters (10 ints)
   void* sd = nullptr;
-  HIPCHK(hipMalloc(&sd, 64));
+  HIPCHK(hipMalloc(&sd, kScalarBytes));
   h->allocs.push_back(sd);
-  HIPCHK(hipMemset(sd, 0, 64));
+  HIPCHK(hipMemsetAsync(sd, 0, kScalarBytes, h->stream));
   h->scalDev = sd;
   m.residual = (double*)sd;
   m.toiBits = (unsigned long long*)((char*)sd + 8);
   m.counters = (int*)((char*)sd + 16);
-  HIPCHK(hipHostMalloc(&h->scalHost, 64, hipHostMallocDefault));
-  memset(h->scalHost, 0, 64);
+  HIPCHK(hipHostMalloc(&h->scalHost, kScalarBytes, hipHostMallocDefault));
+  memset(h->scalHost, 0, kScalarBytes);
   // initial positions
   {
     std::vector<double> soa(V3, 0.0);
     for (int i = 0; i < hs.nTotal; i++)
       for (int k = 0; k < 3; k++) soa[(size_t)k * m.ld + i] = hs.X[3 * (size_t)i + k];
     for (double* p : {m.X, m.Xold, m.X0, m.Pre, m.Next, m.Xrest})
-      HIPCHK(hipMemcpy(p, soa.data(), V3 * sizeof(double), hipMemcpyHostToDevice));
+      HIPCHK(h->copy(p, soa.data(), V3 * sizeof(double), hipMemcpyHostToDevice));
   }
 #undef UP
 #undef AL
@@ -369,10 +440,11 @@ void enqueue_local_global(pdipc_handle* h, int withCol) {
   hipStream_t s = h->stream;
   launch_diag(m, withCol, s);
   launch_operators(m, p.omega, p.precision, s);
+  if (m.tile.use(p.precision)) launch_tile_reset(m, s);
   for (int it = 0; it < p.lg_iters; it++) {
     bool fused = p.precision == PDIPC_FP32_SPLIT;  // k_rhs also runs the residual's first pass
     launch_local(m, p.precision, p.sigma_lo, p.sigma_hi, withCol, s, fused ? p.omega : -1.0);
-    launch_solve(m, p.omega, p.rho, p.cheb_iters, p.precision, s, fused);
+    launch_solve(m, p.omega, p.rho, p.cheb_iters, p.precision, s, fused, it & 1);
   }
 }
 
@@ -384,7 +456,8 @@ int local_global(pdipc_handle* h, int withCol) {
     enqueue_local_global(h, withCol);
     return check_launch(h);
   }
-  hipGraphExec_t& g = h->lgGraph[withCol ? 1 : 0][h->prm.precision == 1 ? 1 : 0];
+  hipGraphExec_t& g =
+      h->lgGraph[h->m.tile.use(h->prm.precision) ? 1 : 0][withCol ? 1 : 0][h->prm.precision == 1 ? 1 : 0];
   if (!g) {
     hipGraph_t graph = nullptr;
     HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
@@ -399,6 +472,45 @@ int local_global(pdipc_handle* h, int withCol) {
   }
   HIPCHK(hipGraphLaunch(g, h->stream));
   return check_launch(h);
+}
+
+// One outer iteration: the local/global loop, the search direction, the broad
+// phase (first iteration only), the time of impact, the clamp and the barrier
+// terms; ends with the scalars on the host.
+int outer_iteration(pdipc_handle* h, int outer, bool activeCol, bool* tracked) {
+  DeviceMesh& m = h->m;
+  const pdipc_params& p = h->prm;
+  hipStream_t s = h->stream;
+  int rc;
+  if ((rc = local_global(h, activeCol ? 1 : 0))) return rc;
+  launch_direction(m, s);
+  if (outer == 0) {
+    hipEvent_t b0 = nullptr, b1 = nullptr;
+    if (m.timer && m.timer->take(TC_BROAD, &b0, &b1)) HIPCHK(hipEventRecord(b0, s));
+    rc = broad_phase(h, m.Xold, m.Dir);
+    if (b1) HIPCHK(hipEventRecord(b1, s));
+    if (rc) return rc;
+  }
+  const bool track = p.track_toi_argmin && h->lastRecs > 0;  // (launch_direction reset the TOI minimum)
+  *tracked = track;
+  if (track) {  // per-record TOIs, then the first record attaining the minimum
+    if (h->trackCap < h->lastRecs) {
+      h->release(h->trackToi);
+      h->trackToi = nullptr;
+      h->trackCap = 0;
+      if ((rc = h->alloc(&h->trackToi, (size_t)h->lastRecs))) return rc;
+      h->trackCap = h->lastRecs;
+    }
+    HIPCHK(hipMemsetAsync(m.counters + 4, 0x7f, sizeof(int), s));
+    launch_ccd_records(m, m.recs, h->lastRecs, m.Xold, m.X, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
+                       p.touch_policy, h->trackToi, m.counters + 4, s);
+    launch_argmin_path(m, h->lastRecs, m.Xold, m.X, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap, p.touch_policy,
+                       m.counters + 4, s);
+  } else {
+    launch_ccd(m, h->lastRecs, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap, p.touch_policy, s);
+  }
+  launch_clamp_residual(m, p.toi_scale, s);
+  return collision(h);  // also reads the scalars back
 }
 
 int advance(pdipc_handle* h) {
@@ -416,34 +528,11 @@ int advance(pdipc_handle* h) {
   uint64_t argminHash = 0, activeHash = 0;  // diagnostics (track_toi_argmin), wrapping arithmetic
   h->cnt.lg_iters = 0;
   for (; outer < p.max_outer; outer++) {
-    if ((rc = local_global(h, activeCol ? 1 : 0))) return rc;
+    bool track = false;
+    rc = outer_iteration(h, outer, activeCol, &track);
+    if (rc == kTileAborted && !(rc = tile_recover(h, outer))) rc = outer_iteration(h, outer, activeCol, &track);
+    if (rc) return rc;
     h->cnt.lg_iters += p.lg_iters;
-    launch_direction(m, s);
-    if (outer == 0) {
-      hipEvent_t b0 = nullptr, b1 = nullptr;
-      if (m.timer && m.timer->take(TC_BROAD, &b0, &b1)) HIPCHK(hipEventRecord(b0, s));
-      if ((rc = broad_phase(h, m.Xold, m.Dir))) return rc;
-      if (b1) HIPCHK(hipEventRecord(b1, s));
-    }
-    const bool track = p.track_toi_argmin && h->lastRecs > 0;  // (launch_direction reset the TOI minimum)
-    if (track) {  // per-record TOIs, then the first record attaining the minimum
-      if (h->trackCap < h->lastRecs) {
-        h->release(h->trackToi);
-        h->trackToi = nullptr;
-        h->trackCap = 0;
-        if ((rc = h->alloc(&h->trackToi, (size_t)h->lastRecs))) return rc;
-        h->trackCap = h->lastRecs;
-      }
-      HIPCHK(hipMemsetAsync(m.counters + 4, 0x7f, sizeof(int), s));
-      launch_ccd_records(m, m.recs, h->lastRecs, m.Xold, m.X, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
-                         p.touch_policy, h->trackToi, m.counters + 4, s);
-      launch_argmin_path(m, h->lastRecs, m.Xold, m.X, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
-                         p.touch_policy, m.counters + 4, s);
-    } else {
-      launch_ccd(m, h->lastRecs, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap, p.touch_policy, s);
-    }
-    launch_clamp_residual(m, p.toi_scale, s);
-    if ((rc = collision(h))) return rc;  // also reads the scalars back
     if (p.track_toi_argmin) {  // the record attaining the minimum TOI, its ACCD exit path, the active set
       const int am = track ? h->hCounters()[4] : 0x7f7f7f7f;
       const bool hit = am >= 0 && am < h->lastRecs;
@@ -619,13 +708,12 @@ int pdipc_set_cloth_stiffness(pdipc_handle* h, int model, const double* k, int n
   build_sell(h->hs, h->sell.lanes, h->sell);
   DeviceMesh& m = h->m;
   const HostSetup& hs = h->hs;
-  HIPCHK(hipStreamSynchronize(h->stream));  // the uploads below go through the null stream
-  HIPCHK(hipMemcpy(m.elasticDiag, hs.elasticDiag.data(), hs.elasticDiag.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(m.r1Val, hs.r1Val.data(), hs.r1Val.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(m.cStrain, hs.cStrain.data(), hs.cStrain.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(m.m2R1, h->sell.r1.data(), h->sell.r1.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(m.p2A, h->sell.pA.data(), h->sell.pA.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemset(m.dStale, 1, std::max(1, hs.nSim)));  // every M^2 row is recomputed next
+  HIPCHK(h->copy(m.elasticDiag, hs.elasticDiag.data(), hs.elasticDiag.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(h->copy(m.r1Val, hs.r1Val.data(), hs.r1Val.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(h->copy(m.cStrain, hs.cStrain.data(), hs.cStrain.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(h->copy(m.m2R1, h->sell.r1.data(), h->sell.r1.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(h->copy(m.p2A, h->sell.pA.data(), h->sell.pA.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemsetAsync(m.dStale, 1, std::max(1, hs.nSim), h->stream));  // every M^2 row is recomputed next
   return pdipc::adjoint_refresh_values(h);
 }
 
@@ -669,7 +757,7 @@ int pdipc_init(pdipc_handle* h) {
   HIPCHK(hipGetDevice(&h->device));
   if ((rc = pdipc::noalloc_setup(h->device))) return rc;
   HIPCHK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-  if ((rc = upload_all(h))) return rc;
+  if ((rc = upload_all(h)) || (rc = upload_tiles(h))) return rc;
   h->cnt.sell_entries = h->m.sellEntries;
   h->deviceReady = true;
   return PDIPC_OK;
@@ -684,7 +772,7 @@ static int fold_timer(pdipc_handle* h) {
     float ms = 0.0f;
     HIPCHK(hipEventElapsedTime(&ms, t->pool[2 * i], t->pool[2 * i + 1]));
     t->us[t->cls[i]] += 1000.0 * ms;
-    t->count[t->cls[i]]++;
+    t->count[t->cls[i]] += t->weight[i];
   }
   t->used = 0;
   return PDIPC_OK;
@@ -693,6 +781,7 @@ static int fold_timer(pdipc_handle* h) {
 int pdipc_step(pdipc_handle* h, int nsteps) {
   int rc = require_device(h);
   if (rc) return rc;
+  pdipc::TileTurn turn(h);
   for (int i = 0; i < nsteps; i++) {
     if ((rc = advance(h))) return rc;
     if ((rc = fold_timer(h))) return rc;
@@ -955,6 +1044,48 @@ int pdipc_sweep_staging(pdipc_handle* h, int* path) {
   return PDIPC_OK;
 }
 
+int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort) {
+  int rc = require_device(h);
+  if (rc) return rc;
+  const TileMesh& t = h->m.tile;
+  if (info) {
+    const bool may = t.built && h->tileAborts < kTileMaxAborts;
+    info[0] = t.built ? 1 : 0;
+    info[1] = may && t.ok32 ? 1 : 0;
+    info[2] = may && t.ok64 ? 1 : 0;
+    info[3] = t.nTiles;
+    info[4] = t.rowsPerTile;
+    info[5] = h->tileAborts;
+  }
+  if (request_abort && t.built) {
+    const int one = 1;
+    HIPCHK(hipMemcpyAsync(t.abort, &one, sizeof(int), hipMemcpyHostToDevice, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
+  }
+  return PDIPC_OK;
+}
+
+int pdipc_debug_tile_layout(pdipc_handle* h, int max_tiles, long long* sizes, int* rows, int* halo_off, int* halo,
+                            unsigned short* loc) {
+  if (!h) return fail(PDIPC_E_ARG, "null handle");
+  if (!h->hostReady) return fail(PDIPC_E_ARG, "pdipc_host_setup has not run");
+  if (max_tiles < 1) return fail(PDIPC_E_ARG, "max_tiles must be positive");
+  if (!sizes) return fail(PDIPC_E_ARG, "null sizes");
+  SellLayout L;
+  build_sell(h->hs, 8, L);
+  SolveTiles T;
+  build_solve_tiles(h->hs, L, max_tiles, T);
+  const long long sz[8] = {T.ok ? 1 : 0, T.nTiles, T.rowsPerTile, (long long)T.halo.size(),
+                           T.threads,    T.tpr,    T.width,       T.uCap};
+  std::copy(sz, sz + 8, sizes);
+  if (!T.ok) return PDIPC_OK;
+  if (rows) std::copy(T.rows.begin(), T.rows.end(), rows);
+  if (halo_off) std::copy(T.haloOff.begin(), T.haloOff.end(), halo_off);
+  if (halo) std::copy(T.halo.begin(), T.halo.end(), halo);
+  if (loc) std::copy(T.loc.begin(), T.loc.end(), loc);
+  return PDIPC_OK;
+}
+
 int pdipc_debug_broad_phase(pdipc_handle* h, const double* xold, const double* dx, int* count) {
   int rc = require_device(h);
   if (rc) return rc;
@@ -1018,8 +1149,17 @@ int pdipc_debug_solve(pdipc_handle* h, const double* diag, const double* rhs, co
   if ((rc = put_soa(h, m.sysRhs, rhs, m.nSim))) return rc;
   if ((rc = put_soa(h, m.X, x0, m.nTotal))) return rc;
   launch_operators(m, h->prm.omega, h->prm.precision, h->stream);
+  pdipc::TileTurn turn(h);
+  if (m.tile.use(h->prm.precision)) launch_tile_reset(m, h->stream);
   launch_solve(m, h->prm.omega, h->prm.rho, h->prm.cheb_iters, h->prm.precision, h->stream);
   if ((rc = check_launch(h))) return rc;
+  rc = read_scalars(h);
+  if (rc == kTileAborted) {  // once more with the streamed sweeps
+    if ((rc = tile_recover(h, 1)) || (rc = put_soa(h, m.X, x0, m.nTotal))) return rc;
+    launch_solve(m, h->prm.omega, h->prm.rho, h->prm.cheb_iters, h->prm.precision, h->stream);
+    rc = check_launch(h);
+  }
+  if (rc) return rc;
   return get_soa(h, m.X, xout, m.nSim);
 }
 

@@ -90,6 +90,9 @@ SIGNATURES = {
                                                        ctypes.POINTER(ctypes.c_ushort),
                                                        ctypes.POINTER(ctypes.c_ubyte)]),
     "pdipc_sweep_staging": (ctypes.c_int, [_H, _I]),
+    "pdipc_tile_solves": (ctypes.c_int, [_H, _I, ctypes.c_int]),
+    "pdipc_debug_tile_layout": (ctypes.c_int, [_H, ctypes.c_int, ctypes.POINTER(ctypes.c_longlong), _I, _I, _I,
+                                               ctypes.POINTER(ctypes.c_ushort)]),
     "pdipc_debug_sell_layout": (ctypes.c_int, [_H, ctypes.c_int, ctypes.POINTER(ctypes.c_longlong),
                                                ctypes.POINTER(ctypes.c_longlong), _I, _I, _I,
                                                ctypes.POINTER(ctypes.c_short), _I]),
@@ -371,6 +374,29 @@ class Simulator:
         v = ctypes.c_int()
         _check(lib().pdipc_sweep_staging(self.h, ctypes.byref(v)))
         return v.value
+
+    def tile_solves(self, request_abort=False):
+        """Whether this handle's Chebyshev solves run as tiles (one launch per
+        solve), the tiling, and how often a tile gave up waiting."""
+        info = np.zeros(6, np.int32)
+        _check(lib().pdipc_tile_solves(self.h, _ip(info), 1 if request_abort else 0))
+        return dict(zip(("built", "fp32", "fp64", "tiles", "rows_per_tile", "aborts"), (int(v) for v in info)))
+
+    def tile_layout(self, max_tiles=256):
+        """The tile solves' tables for at most max_tiles tiles (host precompute
+        only), or None when the scene does not tile."""
+        sz = np.zeros(8, np.int64)
+        szp = sz.ctypes.data_as(ctypes.POINTER(ctypes.c_longlong))
+        _check(lib().pdipc_debug_tile_layout(self.h, max_tiles, szp, None, None, None, None))
+        ok, nt, R, nh, threads, tpr, width, cap = (int(v) for v in sz)
+        if not ok:
+            return None
+        rows, off, halo = np.zeros(nt * R, np.int32), np.zeros(nt + 1, np.int32), np.zeros(max(nh, 1), np.int32)
+        loc = np.zeros(nt * threads * (8 // tpr) * width, np.uint16)
+        _check(lib().pdipc_debug_tile_layout(self.h, max_tiles, szp, _ip(rows), _ip(off), _ip(halo),
+                                             loc.ctypes.data_as(ctypes.POINTER(ctypes.c_ushort))))
+        return dict(rows=rows.reshape(nt, R), halo_off=off, halo=halo[:nh], loc=loc, threads=threads, tpr=tpr,
+                    width=width, cap=cap)
 
     def model_dat(self, model, which):
         n = ctypes.c_int()

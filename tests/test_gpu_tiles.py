@@ -1,0 +1,113 @@
+"""The tile solves (a whole Chebyshev solve in one launch) against the streamed
+sweeps: the same bits, over the tilings' edges, both precisions, few and many
+sweeps; when a tile gives up waiting; and with several handles stepping at
+once from different threads."""
+
+import threading
+
+import numpy as np
+import pytest
+
+import pdipc
+import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _cloth(n, **kw):
+    return scenes.cloth_over_sphere(n, 2, ground=True, seed=2, patch_dim=n, sphere_patch_dim=12, height=0.166, **kw)
+
+
+# (scene, rows per tile): one tile (4 and 144 rows), tiles of 32 rows with a
+# remainder, and every thread mapping above (88, 157, 352 rows per tile); rows
+# of 12 entries per lane, three models
+SCENES = [("2", 4), ("12", 144), ("13", 32), ("91", 33), ("150", 88), ("200", 157), ("300", 352), ("tets6", 32),
+          ("tets20", 38), ("layers", 32)]
+
+
+@pytest.mark.parametrize("which,rows", SCENES)
+def test_tile_solves_match_streamed_sweeps(which, rows):
+    if which.startswith("tets"):
+        sc = scenes.config2(cells=int(which[4:]), cloth_n=20)
+    elif which == "layers":
+        sc = scenes.config4(n=40, side=80.0 / 1024)
+    else:
+        sc = _cloth(int(which))
+    for iters in (15, 1, 2, 3, 6):
+        sc["params"]["cheb_iters"] = iters
+        for prec in (pdipc.FP64, pdipc.FP32_SPLIT):
+            print(f"case: {which}, {iters} sweeps, precision {prec}", flush=True)
+            a = pdipc.Simulator.from_scene(sc, precision=prec)
+            b = pdipc.Simulator.from_scene(sc, precision=prec, sell_stage=2)
+            info = a.tile_solves()
+            assert info["rows_per_tile"] == rows and info["fp32"] == 1 and info["fp64"] == 1
+            assert b.tile_solves()["built"] == 0
+            rng = np.random.default_rng(iters)
+            x = a.x()
+            x[: a.sim] += rng.normal(0, 1e-3, (a.sim, 3))
+            diag, rhs = rng.uniform(2e5, 4e5, a.sim), rng.normal(0, 1e3, (a.sim, 3))
+            for rep in range(3):  # a second launch finds the first one's publications
+                assert np.array_equal(a.debug_solve(diag, rhs + rep, x), b.debug_solve(diag, rhs + rep, x)), rep
+        if iters == 15:
+            for prec in (pdipc.FP64, pdipc.FP32_SPLIT):
+                for graphs in (0, 1):
+                    sims = [pdipc.Simulator.from_scene(sc, precision=prec, use_graphs=graphs, sell_stage=st)
+                            for st in (1, 2)]
+                    for s in sims:
+                        s.step(3)
+                    assert np.array_equal(sims[0].x(), sims[1].x()) and np.array_equal(sims[0].v(), sims[1].v())
+                    assert sims[0].tile_solves()["aborts"] == 0
+
+
+@pytest.mark.parametrize("prec", [pdipc.FP64, pdipc.FP32_SPLIT])
+def test_given_up_solve_repeats_with_streamed_sweeps(prec):
+    sc = _cloth(40)
+    print(f"case: tile abort, precision {prec}", flush=True)
+    a = pdipc.Simulator.from_scene(sc, precision=prec, use_graphs=1)
+    b = pdipc.Simulator.from_scene(sc, precision=prec, use_graphs=1)
+    for k in range(6):
+        if k in (1, 4):
+            a.tile_solves(request_abort=True)
+        a.step(1)
+        b.step(1)
+        assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v()), k
+        assert a.counters() == b.counters()
+    assert a.tile_solves()["aborts"] == 2 and b.tile_solves()["aborts"] == 0
+    # twice is enough: the handle keeps to the streamed sweeps
+    assert a.tile_solves()["fp64"] == 0 and b.tile_solves()["fp64"] == 1
+    if prec == pdipc.FP64:
+        c = pdipc.Simulator.from_scene(sc, precision=prec)
+        d = pdipc.Simulator.from_scene(sc, precision=prec)
+        g = np.random.default_rng(0).normal(size=(c.sim, 3))
+        c.tile_solves(request_abort=True)
+        c.rollout(3, 0)
+        d.rollout(3, 0)
+        assert np.array_equal(c.x(), d.x())
+        for u, w in zip(c.backward(dx=g), d.backward(dx=g)):
+            assert np.allclose(u, w, rtol=1e-9, atol=1e-12 * max(np.abs(w).max(initial=0.0), 1e-300))
+        assert c.tile_solves()["aborts"] == 1
+
+
+def test_handles_stepping_from_several_threads():
+    """One handle at a time has the device's turn for tile solves; the others
+    stream meanwhile, and every one gets the bits it gets alone."""
+    scs = [_cloth(48), _cloth(33, kappa=2e3), scenes.config2(cells=5, cloth_n=12)]
+    print("case: three handles in three threads", flush=True)
+
+    def go(sc, out, i):
+        s = pdipc.Simulator.from_scene(sc, use_graphs=i % 2)
+        for _ in range(4):
+            s.step(2)
+        out[i] = (s.x(), s.v(), s.tile_solves()["aborts"])
+
+    alone, together = [None] * 3, [None] * 3
+    for i, sc in enumerate(scs):
+        go(sc, alone, i)
+    ts = [threading.Thread(target=go, args=(sc, together, i)) for i, sc in enumerate(scs)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for p, q in zip(alone, together):
+        assert np.array_equal(p[0], q[0]) and np.array_equal(p[1], q[1])
+        assert p[2] == 0 and q[2] == 0
