@@ -19,12 +19,6 @@ struct __align__(32) Row64 {
   double x, y, z, w;
 };
 
-// c = (w^2 sum_j R1_ij b_j / D_j + (2 - w) w b_i) / D_i of one component, given
-// the sum: one rounding sequence for every kernel that forms it
-__device__ __forceinline__ double first_term(double w, double sum, double b, double d) {
-  return __builtin_fma(w * w, sum, (2.0 - w) * w * b) / d;
-}
-
 // LBVH node for the stackless traversal: box rounded outward to float (a
 // superset of the exact box, used only to prune), the left child (internal
 // nodes) or the patch id (leaves), and the next node in depth-first preorder
@@ -118,6 +112,12 @@ struct TileMesh {
   unsigned long long* slots = nullptr;  // two sets of four publication slots
   double* cheb = nullptr;               // W_1 .. of the Chebyshev recurrence
   int* abort = nullptr;                 // set by a tile that gave up waiting
+  // the local/global loop in one launch (scenes of cloths only, curvCap > 0)
+  bool loop32 = false, loop64 = false;
+  int curvCap = 0;
+  int4* curvItems = nullptr;
+  uint16_t *curvLoc = nullptr, *ringLoc = nullptr, *ringItem = nullptr, *r1Loc = nullptr;
+  bool loop(int precision) const { return on && (precision == 0 ? loop64 : loop32); }
   bool use(int precision) const { return on && (precision == 0 ? ok64 : ok32); }
 };
 
@@ -264,6 +264,10 @@ void launch_tile_reset(const DeviceMesh& m, hipStream_t s);
 void launch_tile_solve32(const DeviceMesh& m, int iters, int parity, hipStream_t s);
 void launch_tile_solve64(const DeviceMesh& m, double w, int iters, int parity, double* out, int64_t outStride,
                          hipStream_t s);
+// all local/global passes of an outer iteration in one launch (m.tile.loop());
+// with rhsOut / itOut (FP64) every pass's rhs and iterates are recorded
+void launch_tile_loop(const DeviceMesh& m, int precision, double w, int passes, int iters, int withCol,
+                      double* rhsOut, int64_t rhsStride, double* itOut, int64_t itStride, hipStream_t s);
 // k_solve.hip
 void launch_operators(const DeviceMesh& m, double omega, int precision, hipStream_t s);
 void launch_solve(const DeviceMesh& m, double omega, double rho, int chebIters, int precision, hipStream_t s,

@@ -1002,11 +1002,11 @@ void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, S
   const int n = hs.nSim;
   if (L.lanes != 8 || n < 1 || maxTiles < 1 || L.sliceOff.back() > INT32_MAX) return;
   // One tile while a workgroup's own LDS reads cost less than an exchange
-  // (FP64 solve of 144 rows 32 us, as five tiles 36; of 576 rows 55 us as three
-  // tiles of 256 rows, 37 as tiles of 32); then small tiles until every compute
-  // unit has one (rows per tile 32 / 64 / 128, FP64 solves: 64^2 cloth 38 / 40 /
-  // 45 us, 13^3-cell tet block 51 / 55 / 58 us), then as many rows as that takes.
-  const int R = n <= 160 ? n : std::max(32, (n + maxTiles - 1) / maxTiles);
+  // (per pass, FP32 / FP64: 144 rows 23 / 39 us, as five tiles 28 / 31); then
+  // small tiles until every compute unit has one (rows per tile 32 / 64 / 128,
+  // FP64 solves: 64^2 cloth 38 / 40 / 45 us, 13^3-cell tet block 51 / 55 / 58 us),
+  // then as many rows as that takes.
+  const int R = n <= 128 ? n : std::max(32, (n + maxTiles - 1) / maxTiles);
   if (R <= 64) T.threads = 256, T.tpr = 4;
   else if (R <= 128) T.threads = 512, T.tpr = 4;
   else if (R <= 256) T.threads = 512, T.tpr = 2;
@@ -1029,18 +1029,33 @@ void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, S
     for (int p = b; p < e; p++) owner[T.rows[p]] = t;
   }
   const int nt = setup_threads();
-  std::vector<std::vector<int>> halo(T.nTiles);
-  auto each_entry = [&](int row, auto&& fn) {
-    for (int q = hs.m2Off[row]; q < hs.m2Off[row + 1]; q++) fn(hs.m2Col[q]);
+  const bool cloths = hs.nCloth == n && hs.nTets == 0;
+  std::vector<std::vector<int>> halo(T.nTiles), ringHalo(T.nTiles);
+  auto ring_of = [&](int row, auto&& fn) {  // fn(slot, point)
+    const int c = hs.clothOfPoint[row];
+    for (int s = hs.cOff[c]; s < hs.cOff[c + 1]; s++) fn(s, hs.cNbr[s]);
   };
   parallel_ranges(T.nTiles, nt, [&](int64_t t0, int64_t t1, int) {
     for (int t = (int)t0; t < (int)t1; t++) {
-      std::vector<int>& H = halo[t];
+      std::vector<int>&H = halo[t], &G = ringHalo[t];
+      auto read = [&](int c) {
+        if (owner[c] != t) H.push_back(c);
+      };
       for (int r = 0; r < R; r++)
-        if (const int row = T.rows[(size_t)t * R + r]; row >= 0)
-          each_entry(row, [&](int c) {
-            if (owner[c] != t) H.push_back(c);
+        if (const int row = T.rows[(size_t)t * R + r]; row >= 0) {
+          for (int q = hs.m2Off[row]; q < hs.m2Off[row + 1]; q++) read(hs.m2Col[q]);
+          if (!cloths) continue;
+          for (int q = hs.r1Off[row]; q < hs.r1Off[row + 1]; q++) read(hs.r1Col[q]);
+          ring_of(row, [&](int, int c) {
+            if (owner[c] != t) G.push_back(c);
           });
+        }
+      std::sort(G.begin(), G.end());
+      G.erase(std::unique(G.begin(), G.end()), G.end());
+      for (int c : G) {
+        read(c);
+        ring_of(c, [&](int, int b) { read(b); });
+      }
       std::sort(H.begin(), H.end());
       H.erase(std::unique(H.begin(), H.end()), H.end());
     }
@@ -1102,6 +1117,58 @@ void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, S
       }
     }
   }, 8);
+  if (cloths) {
+    size_t mostRing = 0;
+    for (auto& G : ringHalo) mostRing = std::max(mostRing, G.size());
+    T.curvCap = (int)(((size_t)R + mostRing + 1) / 2 * 2);
+    T.curvItems.assign(4 * (size_t)T.nTiles * T.curvCap, 0);
+    T.ringLoc.assign(hs.cNbr.size(), 0);
+    T.ringItem.assign(hs.cNbr.size(), 0);
+    T.r1Loc.assign(hs.r1Col.size(), 0);
+    std::vector<int> first(T.nTiles + 1, 0);  // each tile's start in curvLoc
+    for (int t = 0; t < T.nTiles; t++) {
+      int slots = 0;
+      auto count = [&](int row) {
+        const int k = hs.clothOfPoint[row];
+        slots += hs.cOff[k + 1] - hs.cOff[k];
+      };
+      for (int r = 0; r < R; r++)
+        if (const int row = T.rows[(size_t)t * R + r]; row >= 0) count(row);
+      for (int row : ringHalo[t]) count(row);
+      first[t + 1] = first[t] + slots;
+    }
+    T.curvLoc.assign(first[T.nTiles], 0);
+    parallel_ranges(T.nTiles, nt, [&](int64_t t0, int64_t t1, int) {
+      std::vector<int> place(n, 0), item(n, 0);
+      for (int t = (int)t0; t < (int)t1; t++) {
+        for (int r = 0; r < R; r++)
+          if (const int row = T.rows[(size_t)t * R + r]; row >= 0) place[row] = item[row] = r;
+        for (size_t u = 0; u < halo[t].size(); u++) place[halo[t][u]] = R + (int)u;
+        for (size_t u = 0; u < ringHalo[t].size(); u++) item[ringHalo[t][u]] = R + (int)u;
+        int at = first[t];
+        auto put = [&](int i, int row) {
+          const int k = hs.clothOfPoint[row];
+          int* it = T.curvItems.data() + 4 * ((size_t)t * T.curvCap + i);
+          it[0] = hs.cOff[k];
+          it[1] = hs.cOff[k + 1] - hs.cOff[k];
+          it[2] = at;
+          it[3] = k;
+          ring_of(row, [&](int, int c) { T.curvLoc[at++] = (uint16_t)place[c]; });
+        };
+        for (int r = 0; r < R; r++) {
+          const int row = T.rows[(size_t)t * R + r];
+          if (row < 0) continue;
+          put(r, row);
+          ring_of(row, [&](int s, int c) {
+            T.ringLoc[s] = (uint16_t)place[c];
+            T.ringItem[s] = (uint16_t)item[c];
+          });
+          for (int q = hs.r1Off[row]; q < hs.r1Off[row + 1]; q++) T.r1Loc[q] = (uint16_t)place[hs.r1Col[q]];
+        }
+        for (size_t u = 0; u < ringHalo[t].size(); u++) put(R + (int)u, ringHalo[t][u]);
+      }
+    }, 8);
+  }
   T.ok = true;
 }
 

@@ -178,6 +178,18 @@ struct SolveTiles {
   std::vector<int> haloOff;   // nTiles + 1
   std::vector<int> halo;      // ascending per tile
   std::vector<uint16_t> loc;  // [tile][8-entry chunk][thread][8]
+  // For the single-launch local/global loop, when every simulated point is a
+  // cloth point (curvCap > 0; the halos then also hold the columns of R1 and
+  // the rings the curvature items read).  Curvature items of a tile: its rows
+  // in order, then the ring neighbours other tiles own; each its first ring
+  // slot, slot count, first index into curvLoc (the LDS places of its ring)
+  // and cloth vertex.
+  int curvCap = 0;
+  std::vector<int> curvItems;       // 4 per item, [tile][curvCap], zero slots where unused
+  std::vector<uint16_t> curvLoc;
+  std::vector<uint16_t> ringLoc;    // per ring slot: LDS place of its point in its centre's tile
+  std::vector<uint16_t> ringItem;   // per ring slot: its point's curvature item there
+  std::vector<uint16_t> r1Loc;      // per R1 entry: LDS place of its column in its row's tile
 };
 void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, SolveTiles& out);
 

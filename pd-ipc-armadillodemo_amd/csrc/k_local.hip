@@ -11,6 +11,7 @@
 // (double, or float in the FP32-split mode); edge vectors are formed in double
 // and rounded once, so FP32 never sees absolute coordinates.
 #include "device.hpp"
+#include "local_ops.hpp"
 
 namespace pdipc {
 namespace {
@@ -140,14 +141,7 @@ __global__ void k_cloth_curvature(int nCloth, int ld, const int* __restrict__ cC
     for (int k = 0; k < 3; k++) a[k] += l * (T)(X[k * ld + j] - xi[k]);
   }
   double ad[3];
-#pragma unroll
-  for (int k = 0; k < 3; k++) ad[k] = (double)a[k] + lsum * xi[k];
-  double n = sqrt(ad[0] * ad[0] + ad[1] * ad[1] + ad[2] * ad[2]);
-  if (n >= 1e-10) {
-    double sc = cH0[c] / n;
-#pragma unroll
-    for (int k = 0; k < 3; k++) ad[k] *= sc;
-  }
+  curvature_rescale(a, lsum, xi, cH0[c], ad);
 #pragma unroll
   for (int k = 0; k < 3; k++) A[k * ld + i] = ad[k];
 }
@@ -322,10 +316,7 @@ __global__ void k_rhs(int nSim, int ld, int nT, int withCol, ResidualArgs ra, co
         T d[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) d[k] = (T)(xi[k] - xj[b][k]);
-        T len = dsqrt<T>(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-        T rc = (T)stiff[b] * ((T)rest[b] / len);
-#pragma unroll
-        for (int k = 0; k < 3; k++) sp[k] += rc * d[k];
+        add_spring(d, stiff[b], rest[b], sp);
       }
 #pragma unroll
       for (int k = 0; k < 3; k++) bd[k] += bw[b] * aj[b][k];
@@ -378,12 +369,7 @@ __global__ void k_rhs(int nSim, int ld, int nT, int withCol, ResidualArgs ra, co
     const double w = ra.w;
     double vv[3], pp[3];
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      double y = (1.0 - w) * xi[k] + w * sx[k] / di;
-      double u = r[k] / di;
-      vv[k] = y + w * u;
-      pp[k] = (1.0 - w) * y + (2.0 - w) * w * u - xi[k];
-    }
+    for (int k = 0; k < 3; k++) residual_first(w, xi[k], sx[k], r[k], di, &vv[k], &pp[k]);
     ra.v[i] = Row64{vv[0], vv[1], vv[2], 0.0};
     ra.pt[i] = Row64{pp[0], pp[1], pp[2], 0.0};
   }

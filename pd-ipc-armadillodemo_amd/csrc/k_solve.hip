@@ -30,6 +30,7 @@
 
 #include "device.hpp"
 #include "host_setup.hpp"  // kTileSlices
+#include "local_ops.hpp"
 
 namespace pdipc {
 namespace {

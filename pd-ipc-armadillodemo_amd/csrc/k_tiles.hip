@@ -41,13 +41,14 @@
 // the abort flag, every tile leaves, X keeps a finite value, and the host
 // repeats the outer iteration with the streamed kernels.
 #include "device.hpp"
+#include "local_ops.hpp"
 
 namespace pdipc {
 namespace {
 
 constexpr unsigned long long kTileEmpty = 0xfff5a5a5fff5a5a5ull;
 constexpr unsigned long long kTileWaitTicks = 1000000ull;  // 10 ms of the 100 MHz wall clock
-constexpr int kPollBatch = 6;  // words per thread polled together
+constexpr int kRowWords = 3;   // words per row in a publication slot (FP32 vectors use two)
 
 __device__ __forceinline__ void publish(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -113,10 +114,12 @@ struct TileShape {  // what one launch works on (device pointers of DeviceMesh)
   int iters;
 };
 
-template <class T, int BT, int TPR, int W, bool LM>
+// PB: words per thread polled together; LEAN: keep the LDS indices packed
+template <class T, int BT, int TPR, int W, bool LM, int PB, bool LEAN>
 struct TileState {
   static constexpr int SUBS = 8 / TPR, E = SUBS * W, RW = kWave / TPR, NW = TileWords<T>::N;
   using V2 = typename TileWords<T>::V2;
+  using Words = TileWords<T>;
   T v[E];
   unsigned li[E / 2];
   int rl, part, row;  // row < 0: this thread holds no row
@@ -125,8 +128,9 @@ struct TileState {
   V2* xy;  // LDS: the staged iterate, (x, y) pairs and z values, own rows first, then the halo
   T* z;
   double* cheb;        // LDS: the sweeps' weights
-  int hw[kPollBatch];  // word offset of the thread's first polled words (-1: none)
+  int hw[PB];  // word offset of the thread's first polled words (-1: none)
 
+  template <bool EMPTY_OTHER>
   __device__ __forceinline__ void init(const TileShape& a, const T* __restrict__ val, char* lds) {
     const int t = threadIdx.x, tile = blockIdx.x;
     xy = (V2*)lds;
@@ -178,25 +182,20 @@ struct TileState {
 #pragma unroll
       for (int e = 0; e < E; e++) v[e] = T(0);
 #pragma unroll
-    for (int q = 0; q < kPollBatch; q++) {
+    for (int q = 0; q < PB; q++) {
       const int i = t + q * BT;
-      hw[q] = i < nHalo * NW ? halo[i / NW] * NW + i % NW : -1;
+      hw[q] = i < nHalo * NW ? halo[i / NW] * kRowWords + i % NW : -1;
     }
     // empty the other set's slots for the next launch
-    if (row >= 0 && nHalo > 0)
-      for (int w = part; w < NW; w += TPR)
+    if (EMPTY_OTHER && row >= 0 && nHalo > 0)
+      for (int w = part; w < kRowWords; w += TPR)
 #pragma unroll
-        for (int s = 0; s < 4; s++) publish(a.other + s * a.slotStride + (size_t)row * NW + w, kTileEmpty);
+        for (int s = 0; s < 4; s++) publish(a.other + s * a.slotStride + (size_t)row * kRowWords + w, kTileEmpty);
   }
-
-  // Keeps the compiler from unpacking the LDS indices once for all sweeps where
-  // the unpacked ones would not fit the registers beside the entries.
-  // (unpacked: an address for the pair and one for z per entry)
-  static constexpr bool kLean = E * (2 + (int)sizeof(T) / 4) > 100;
 
   // M^2 times the staged iterate, at the thread's row (in all its parts)
   __device__ __forceinline__ void apply(T (&acc)[3]) {
-    if constexpr (kLean)
+    if constexpr (LEAN)  // (opaque per sweep: the compiler would unpack them once for all sweeps)
 #pragma unroll
       for (int e = 0; e < E / 2; e++) asm volatile("" : "+v"(li[e]));
     T s[3][SUBS];
@@ -227,71 +226,85 @@ struct TileState {
     for (int k = 0; k < 3; k++) acc[k] = lane_tree<TPR, T>(s[k]);
   }
 
-  // publication j of the row
-  __device__ __forceinline__ void send(const TileShape& a, int j, const T (&d)[3]) const {
+  // publication j of the row (values of type U), emptying `old` words of
+  // publication j - 2
+  template <class U>
+  __device__ __forceinline__ void send(const TileShape& a, int j, const U (&d)[3], int old) const {
     if (row < 0 || nHalo == 0) return;  // without a halo nobody reads this tile's rows
-    unsigned long long* s = a.slots + (size_t)row * NW;
+    unsigned long long* s = a.slots + (size_t)row * kRowWords;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the words emptied a sweep ago have reached memory
-    for (int w = part; w < NW; w += TPR) publish(s + (size_t)(j & 3) * a.slotStride + w, TileWords<T>::word(d, w));
+    for (int w = part; w < TileWords<U>::N; w += TPR)
+      publish(s + (size_t)(j & 3) * a.slotStride + w, TileWords<U>::word(d, w));
     if (j >= 2)
-      for (int w = part; w < NW; w += TPR) publish(s + (size_t)((j + 2) & 3) * a.slotStride + w, kTileEmpty);
+      for (int w = part; w < old; w += TPR) publish(s + (size_t)((j + 2) & 3) * a.slotStride + w, kTileEmpty);
   }
-  __device__ __forceinline__ void stage_own(T x, T y, T w) const {
+  template <class U, class U2>
+  __device__ __forceinline__ void stage_own(U2* pxy, U* pz, U x, U y, U w) const {
     if (row < 0 || part != 0) return;
-    xy[rl] = V2{x, y};
-    z[rl] = w;
+    pxy[rl] = U2{x, y};
+    pz[rl] = w;
   }
   // polls the words at off[] (-1: none) until all have arrived, then stages them
-  __device__ __forceinline__ bool poll(const TileShape& a, const unsigned long long* s, const int (&off)[kPollBatch],
-                                       int i0, unsigned long long t0) const {
-    unsigned long long w[kPollBatch];
+  template <class U, class U2>
+  __device__ __forceinline__ bool poll(const TileShape& a, const unsigned long long* s, const int (&off)[PB],
+                                       int i0, unsigned long long t0, U2* pxy, U* pz) const {
+    constexpr int N = TileWords<U>::N;
+    unsigned long long w[PB];
     for (int spin = 1;; spin++) {
       bool ready = true;
 #pragma unroll
-      for (int q = 0; q < kPollBatch; q++) w[q] = off[q] >= 0 ? peek(s + off[q]) : 0ull;
+      for (int q = 0; q < PB; q++) w[q] = off[q] >= 0 ? peek(s + off[q]) : 0ull;
 #pragma unroll
-      for (int q = 0; q < kPollBatch; q++) ready = ready && w[q] != kTileEmpty;
+      for (int q = 0; q < PB; q++) ready = ready && w[q] != kTileEmpty;
       if (ready) break;
       if ((spin & 63) == 0 && (wall_clock64() - t0 > kTileWaitTicks ||
                                __hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
         return false;
     }
 #pragma unroll
-    for (int q = 0; q < kPollBatch; q++) {
+    for (int q = 0; q < PB; q++) {
       const int i = i0 + q * BT;
-      if (off[q] >= 0) TileWords<T>::unpack(w[q], i % NW, xy, z, a.R + i / NW);
+      if (off[q] >= 0) TileWords<U>::unpack(w[q], i % N, pxy, pz, a.R + i / N);
     }
     return true;
   }
   // stages publication j of the neighbours' rows; false: gave up waiting
-  __device__ __forceinline__ bool receive(const TileShape& a, int j, unsigned long long t0) const {
-    const int items = nHalo * NW;
+  template <class U, class U2>
+  __device__ __forceinline__ bool receive(const TileShape& a, int j, unsigned long long t0, U2* pxy, U* pz) const {
+    constexpr int N = TileWords<U>::N;
+    const int items = nHalo * N;
     if (items == 0) return true;
     const unsigned long long* s = a.slots + (size_t)(j & 3) * a.slotStride;
     // the neighbours finish at about the same time and a store takes about 0.4 us
     // to arrive: polling at once only delays it (256^2 cloth, per sweep: 2.7 us
     // without this pause, 2.3 us with it)
     __builtin_amdgcn_s_sleep(6);
-    bool ok = poll(a, s, hw, threadIdx.x, t0);
-    for (int i0 = threadIdx.x + kPollBatch * BT; i0 < items; i0 += kPollBatch * BT) {
-      int off[kPollBatch];
+    bool ok = true;
+    int i0 = threadIdx.x;
+    if constexpr (N == NW) {  // the words of the solve's own type are listed at the start
+      ok = poll(a, s, hw, i0, t0, pxy, pz);
+      i0 += PB * BT;
+    }
+    for (; i0 < items; i0 += PB * BT) {
+      int off[PB];
 #pragma unroll
-      for (int q = 0; q < kPollBatch; q++) {
+      for (int q = 0; q < PB; q++) {
         const int i = i0 + q * BT;
-        off[q] = i < items ? halo[i / NW] * NW + i % NW : -1;
+        off[q] = i < items ? halo[i / N] * kRowWords + i % N : -1;
       }
-      ok = poll(a, s, off, i0, t0) && ok;
+      ok = poll(a, s, off, i0, t0, pxy, pz) && ok;
     }
     return ok;
   }
-  // ends sweep j: the row's new iterate to the neighbours and into LDS, theirs
+  // publication j: the row's new vector to the neighbours and into LDS, theirs
   // into LDS; false (for the whole workgroup): some wait was given up
-  __device__ __forceinline__ bool exchange(const TileShape& a, int j, const T (&d)[3], int* flag,
-                                           unsigned long long t0) const {
-    send(a, j, d);
-    __syncthreads();  // every row of the tile has read the old iterate
-    stage_own(d[0], d[1], d[2]);
-    if (!receive(a, j, t0)) {
+  template <class U, class U2>
+  __device__ __forceinline__ bool exchange(const TileShape& a, int j, const U (&d)[3], int old, int* flag,
+                                           unsigned long long t0, U2* pxy, U* pz) const {
+    send(a, j, d, old);
+    __syncthreads();  // every row of the tile has read the old vector
+    stage_own(pxy, pz, d[0], d[1], d[2]);
+    if (!receive(a, j, t0, pxy, pz)) {
       *flag = 1;
       __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -306,6 +319,11 @@ template <class T>
 constexpr size_t tile_lds_bytes(int uCap, int iters) {
   return (size_t)uCap * 3 * sizeof(T) + (size_t)iters * sizeof(double);
 }
+
+// The unpacked LDS indices (an address for the pair and one for z per entry)
+// are kept where they fit the registers beside the entries.
+template <class T, int TPR, int W>
+constexpr bool tile_lean() { return 8 / TPR * W * (2 + (int)sizeof(T) / 4) > 100; }
 
 // leaves the kernel at its start when an earlier launch gave up (the same
 // answer for the whole workgroup)
@@ -323,8 +341,8 @@ __global__ void __launch_bounds__(BT) k_tile_solve32(TileShape a, const float* _
   extern __shared__ __attribute__((aligned(16))) char tileLds[];
   __shared__ int flag;
   if (tile_aborted(a.abort, &flag)) return;
-  TileState<float, BT, TPR, W, LM> st;
-  st.init(a, val, tileLds);
+  TileState<float, BT, TPR, W, LM, 6, tile_lean<float, TPR, W>()> st;
+  st.template init<true>(a, val, tileLds);
   for (int u = threadIdx.x; u < st.nHalo; u += BT) {
     const float4 q = r0[st.halo[u]];
     st.xy[a.R + u] = make_float2(q.x, q.y);
@@ -336,7 +354,7 @@ __global__ void __launch_bounds__(BT) k_tile_solve32(TileShape a, const float* _
     r[0] = cur[0] = q.x;
     r[1] = cur[1] = q.y;
     r[2] = cur[2] = q.z;
-    st.stage_own(q.x, q.y, q.z);
+    st.stage_own(st.xy, st.z, q.x, q.y, q.z);
   }
   __syncthreads();
   const unsigned long long t0 = wall_clock64();
@@ -351,7 +369,7 @@ __global__ void __launch_bounds__(BT) k_tile_solve32(TileShape a, const float* _
       pre[k] = cur[k];
       cur[k] = d[k];
     }
-    if (it < a.iters - 1 && !st.exchange(a, it - 1, d, &flag, t0)) return;
+    if (it < a.iters - 1 && !st.exchange(a, it - 1, d, 2, &flag, t0, st.xy, st.z)) return;
   }
   if (st.row >= 0 && st.part == 0)
 #pragma unroll
@@ -375,10 +393,10 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
   extern __shared__ __attribute__((aligned(16))) char tileLds[];
   __shared__ int flag;
   if (tile_aborted(a.abort, &flag)) return;
-  using State = TileState<double, BT, TPR, W, LM>;
+  using State = TileState<double, BT, TPR, W, LM, 6, tile_lean<double, TPR, W>()>;
   constexpr int SUBS = State::SUBS;
   State st;
-  st.init(a, val, tileLds);
+  st.template init<true>(a, val, tileLds);
   for (int u = threadIdx.x; u < st.nHalo; u += BT) {
     const int h = st.halo[u];
     st.xy[a.R + u] = make_double2(X[h], X[a.ld + h]);
@@ -394,7 +412,7 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
       bi[k] = ft.b[k * a.ld + rr];
       cur[k] = X[k * a.ld + rr];
     }
-    st.stage_own(cur[0], cur[1], cur[2]);
+    st.stage_own(st.xy, st.z, cur[0], cur[1], cur[2]);
     // lane s of the row sums the R1 entries s, s + 8, ...
     double s[3][SUBS];
 #pragma unroll
@@ -442,7 +460,7 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
       pre[k] = cur[k];
       cur[k] = d[k];
     }
-    if (it < a.iters - 1 && !st.exchange(a, it, d, &flag, t0)) return;
+    if (it < a.iters - 1 && !st.exchange(a, it, d, 3, &flag, t0, st.xy, st.z)) return;
     if (out && st.row >= 0 && st.part == 0)
 #pragma unroll
       for (int k = 0; k < 3; k++) out[it * outStride + k * a.ld + st.row] = d[k];
@@ -450,6 +468,310 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
   if (st.row >= 0 && st.part == 0)
 #pragma unroll
     for (int k = 0; k < 3; k++) X[k * a.ld + st.row] = cur[k];
+}
+
+// ---- the whole local/global loop of an outer iteration
+//
+// For scenes of cloths only, one launch runs every local/global pass: the
+// matrix stays in the registers through all of them, positions and the
+// intermediate vectors stay in LDS, and the curvature, right-hand-side and
+// residual kernels with their boundaries (26 us per pass of a 256^2 cloth,
+// 10 us of a 64^2 one, beside solves of 38 and 26) become phases between
+// exchanges.  A pass:
+//   curvature   a_i of the tile's rows and, again, of the neighbouring rows
+//               their bending sums read (no exchange)
+//   rhs         springs, bending, collision and position terms of each row; in
+//               FP32-split also the first residual pass (v and its pointwise part)
+//   exchange    v (FP32-split) or the rhs (FP64)
+//   residual    delta_1 = r0 (FP32-split), or the first term c (FP64)
+//   sweeps      as in the solves above, every iterate exchanged; the last one
+//               moves the staged positions, own and neighbours'
+// The sums over a point's ring and R1 entries are dealt to 4 lanes (first
+// term: 8) and combined as k_rhs, k_res_b and k_first64 do, with the same
+// rounding sequences (local_ops.hpp): the results are theirs bit for bit.
+// Measured per pass, separate kernels -> one launch: FP32 256^2 cloth 66 -> 49
+// us (sweeps 36, the rest 13), 64^2 38 -> 29; FP64 64^2 50 -> 32.
+struct TileLoop {
+  const int4* curvItems;     // [tile][curvCap]: first ring slot, slots, index of the first LDS place, cloth vertex
+  int curvCap;               // per tile: its rows' items (R of them), then the neighbours'
+  const uint16_t* curvLoc;   // LDS places of the items' ring slots
+  const uint16_t* ringLoc;   // per ring slot: LDS place of its point in the owner's tile
+  const uint16_t* ringItem;  // per ring slot: its point's curvature item there
+  const uint16_t* r1Loc;     // per R1 entry: LDS place of its column in the row's tile
+  const int2* ringRange;
+  const double *cRest, *cStrain, *cBendIn, *cLbo, *cH0;
+  const int* r1Off;
+  const double *r1Val, *D;
+  const double *initRhs, *colRhs, *fixK, *Xrest;
+  int withCol, passes;
+  double w;
+  double* X;
+  double* rhsOut;  // recorded steps: every pass's rhs and iterates (SoA, at these strides)
+  int64_t rhsStride;
+  double* itOut;
+  int64_t itStride;
+};
+
+// lanes l, l + TPR, ... of 4 held by a thread, combined as xor 2, 1
+template <int TPR, class T>
+__device__ __forceinline__ T quad_tree(const T (&s)[4 / TPR]) {
+  if constexpr (TPR == 1) return (s[0] + s[2]) + (s[1] + s[3]);
+  if constexpr (TPR == 2) {
+    const T a = s[0] + s[1];
+    return a + __shfl_xor(a, 32, kWave);
+  }
+  if constexpr (TPR == 4) {
+    T a = s[0];
+    a += __shfl_xor(a, 32, kWave);
+    return a + __shfl_xor(a, 16, kWave);
+  }
+}
+
+template <class T>
+constexpr size_t tile_loop_lds(int uCap, int aCap, int iters) {
+  // the iterate and the weights; the positions (FP32-split: the iterate is a
+  // correction); v or the rhs; D (FP64, for the first term); the curvature vectors
+  return ((tile_lds_bytes<T>(uCap, iters) + 15) & ~(size_t)15) + (size_t)uCap * (sizeof(T) == 4 ? 48 : 32) +
+         (size_t)aCap * 24;
+}
+
+template <class T, int BT, int TPR, int W, bool LM>
+__global__ void __launch_bounds__(BT) k_tile_loop(TileShape a, TileLoop g, const T* __restrict__ val) {
+  extern __shared__ __attribute__((aligned(16))) char tileLds[];
+  __shared__ int flag;
+  if (tile_aborted(a.abort, &flag)) return;
+  constexpr bool F32 = sizeof(T) == 4;
+  using State = TileState<T, BT, TPR, W, LM, 3, tile_lean<T, TPR, W>()>;
+  constexpr int SUBS = State::SUBS, QL = 4 / TPR;
+  State st;
+  st.template init<false>(a, val, tileLds);
+  const int t = threadIdx.x, U = a.uCap, ld = a.ld;
+  // LDS arrays after the iterate and the weights
+  char* p = tileLds + ((tile_lds_bytes<T>(U, a.iters) + 15) & ~(size_t)15);
+  double2* Vxy = (double2*)p;  // v (FP32-split) or the rhs (FP64)
+  double2* Pxy = Vxy + U;      // positions (FP32-split)
+  double2* Axy = F32 ? Pxy + U : Vxy + U;
+  double* Vz = (double*)(Axy + g.curvCap);
+  double* Pz = Vz + U;  // positions' z (FP32-split) or D (FP64)
+  double* Az = Pz + U;
+  if constexpr (!F32) {  // FP64: the iterate is the position
+    Pxy = (double2*)st.xy;
+    Pz = (double*)st.z;
+  }
+  double* Dl = Vz + U;  // FP64
+  for (int u = t; u < st.nHalo; u += BT) {
+    const int h = st.halo[u];
+    Pxy[a.R + u] = make_double2(g.X[h], g.X[ld + h]);
+    Pz[a.R + u] = g.X[2 * ld + h];
+    if constexpr (!F32) Dl[a.R + u] = g.D[h];
+  }
+  // the row's own constants
+  const int rr = st.row >= 0 ? st.row : 0;
+  const bool live = st.row >= 0;
+  const int2 ring = live ? g.ringRange[rr] : make_int2(0, 0);
+  const int q0 = live ? g.r1Off[rr] : 0, q1 = live ? g.r1Off[rr + 1] : 0;
+  const double di = g.D[rr], kf = g.fixK[rr];
+  double xi[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) xi[k] = g.X[k * ld + rr];
+  st.stage_own(Pxy, Pz, xi[0], xi[1], xi[2]);
+  if constexpr (!F32)
+    if (live && st.part == 0) Dl[st.rl] = di;
+  __syncthreads();
+  int j = 0;  // publications so far
+  for (int pass = 0; pass < g.passes; pass++) {
+    const bool last = pass == g.passes - 1;
+    const unsigned long long t0 = wall_clock64();
+    // curvature
+    for (int i = t; i < g.curvCap; i += BT) {
+      const int4 it = g.curvItems[(size_t)blockIdx.x * g.curvCap + i];
+      if (it.y == 0) continue;
+      const uint16_t* loc = g.curvLoc + it.z;
+      const int me = loc[0];
+      const double x[3] = {Pxy[me].x, Pxy[me].y, Pz[me]};
+      double lsum = g.cLbo[it.x];
+      T s[3] = {T(0), T(0), T(0)};
+      for (int q = 1; q < it.y; q++) {
+        const int u = loc[q];
+        const double lq = g.cLbo[it.x + q];
+        const T l = (T)lq;
+        lsum += lq;
+        const double2 pu = Pxy[u];
+        s[0] = fmad(l, (T)(pu.x - x[0]), s[0]);
+        s[1] = fmad(l, (T)(pu.y - x[1]), s[1]);
+        s[2] = fmad(l, (T)(Pz[u] - x[2]), s[2]);
+      }
+      double ad[3];
+      curvature_rescale(s, lsum, x, g.cH0[it.w], ad);
+      Axy[i] = make_double2(ad[0], ad[1]);
+      Az[i] = ad[2];
+    }
+    __syncthreads();
+    // rhs
+    double r[3];
+    {
+      T sp[3][QL];
+      double bd[3][QL], sx[3][QL];
+#pragma unroll
+      for (int q = 0; q < QL; q++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          sp[k][q] = T(0);
+          bd[k][q] = sx[k][q] = 0.0;
+        }
+      for (int s0 = ring.x; s0 < ring.y; s0 += 4)
+#pragma unroll
+        for (int q = 0; q < QL; q++) {
+          const int s = s0 + st.part + TPR * q;
+          if (s >= ring.y) continue;
+          const double2 pu = Pxy[g.ringLoc[s]];
+          const double pz = Pz[g.ringLoc[s]];
+          const int ai = g.ringItem[s];
+          const double bw = g.cBendIn[s];
+          if (s > ring.x) {
+            const T d[3] = {(T)(xi[0] - pu.x), (T)(xi[1] - pu.y), (T)(xi[2] - pz)};
+            T f[3] = {sp[0][q], sp[1][q], sp[2][q]};
+            add_spring(d, g.cStrain[s], g.cRest[s], f);
+#pragma unroll
+            for (int k = 0; k < 3; k++) sp[k][q] = f[k];
+          }
+          const double2 au = Axy[ai];
+          bd[0][q] = fmad(bw, au.x, bd[0][q]);
+          bd[1][q] = fmad(bw, au.y, bd[1][q]);
+          bd[2][q] = fmad(bw, Az[ai], bd[2][q]);
+        }
+      if constexpr (F32)
+        for (int e0 = q0; e0 < q1; e0 += 4)
+#pragma unroll
+          for (int q = 0; q < QL; q++) {
+            const int e = e0 + st.part + TPR * q;
+            if (e >= q1) continue;
+            const int u = g.r1Loc[e];
+            const double av = g.r1Val[e];
+            const double2 pu = Pxy[u];
+            sx[0][q] = fmad(av, pu.x, sx[0][q]);
+            sx[1][q] = fmad(av, pu.y, sx[1][q]);
+            sx[2][q] = fmad(av, Pz[u], sx[2][q]);
+          }
+      double vv[3], pt[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const T spk = quad_tree<TPR, T>(sp[k]);
+        const double bdk = quad_tree<TPR, double>(bd[k]);
+        r[k] = g.initRhs[k * ld + rr];
+        if (ring.y > ring.x) r[k] += (double)spk + bdk;
+        if (g.withCol) r[k] += g.colRhs[k * ld + rr];
+        if (kf != 0.0) r[k] = fmad(kf, g.Xrest[k * ld + rr], r[k]);
+        if constexpr (F32) {
+          const double sxk = quad_tree<TPR, double>(sx[k]);
+          residual_first(g.w, xi[k], sxk, r[k], di, &vv[k], &pt[k]);
+        }
+      }
+      if constexpr (F32) {
+        if (!st.exchange(a, j, vv, 2, &flag, t0, Vxy, Vz)) return;
+        j++;
+#pragma unroll
+        for (int k = 0; k < 3; k++) r[k] = pt[k];
+      } else {
+        if (!st.exchange(a, j, r, 3, &flag, t0, Vxy, Vz)) return;
+        j++;
+        if (g.rhsOut && live && st.part == 0)
+#pragma unroll
+          for (int k = 0; k < 3; k++) g.rhsOut[pass * g.rhsStride + k * ld + st.row] = r[k];
+      }
+    }
+    if constexpr (F32) {
+      // second residual pass: delta_1 = r0 = pt + (w / D) R1 v
+      double sv[3][QL];
+#pragma unroll
+      for (int q = 0; q < QL; q++) sv[0][q] = sv[1][q] = sv[2][q] = 0.0;
+      for (int e0 = q0; e0 < q1; e0 += 4)
+#pragma unroll
+        for (int q = 0; q < QL; q++) {
+          const int e = e0 + st.part + TPR * q;
+          if (e >= q1) continue;
+          const int u = g.r1Loc[e];
+          const double av = g.r1Val[e];
+          const double2 vu = Vxy[u];
+          sv[0][q] = fmad(av, vu.x, sv[0][q]);
+          sv[1][q] = fmad(av, vu.y, sv[1][q]);
+          sv[2][q] = fmad(av, Vz[u], sv[2][q]);
+        }
+      const double f = g.w / di;
+      float r0[3], pre[3] = {0.f, 0.f, 0.f}, cur[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) r0[k] = cur[k] = (float)fmad(f, quad_tree<TPR, double>(sv[k]), r[k]);
+      for (int it = 0;; it++) {  // cur = delta_{it + 1}
+        const bool done = it == a.iters - 1;
+        if (done && last) break;
+        // (publication j - 2 was v, of three words, at it = 1)
+        if (!st.exchange(a, j, cur, it == 1 ? 3 : 2, &flag, t0, (float2*)st.xy, (float*)st.z)) return;
+        j++;
+        if (done) break;
+        const float Wc = (float)st.cheb[it];
+        float acc[3];
+        st.apply(acc);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          const float d = fmad(Wc, acc[k] + r0[k] - pre[k], pre[k]);
+          pre[k] = cur[k];
+          cur[k] = d;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 3; k++) xi[k] += (double)cur[k];
+      if (!last) {  // the staged positions move with the last correction
+        for (int u = t; u < a.R + st.nHalo; u += BT) {
+          const float2 d = ((float2*)st.xy)[u];
+          Pxy[u].x += (double)d.x;
+          Pxy[u].y += (double)d.y;
+          Pz[u] += (double)((float*)st.z)[u];
+        }
+        __syncthreads();
+      }
+    } else {
+      // the first term c from the staged rhs (8 lanes, as k_first64)
+      double s[3][SUBS], c[3];
+#pragma unroll
+      for (int q = 0; q < SUBS; q++) s[0][q] = s[1][q] = s[2][q] = 0.0;
+      for (int e0 = q0; e0 < q1; e0 += 8)
+#pragma unroll
+        for (int q = 0; q < SUBS; q++) {
+          const int e = e0 + st.part + TPR * q;
+          if (e >= q1) continue;
+          const int u = g.r1Loc[e];
+          const double f = g.r1Val[e] / Dl[u];
+          const double2 bu = Vxy[u];
+          s[0][q] = fmad(f, bu.x, s[0][q]);
+          s[1][q] = fmad(f, bu.y, s[1][q]);
+          s[2][q] = fmad(f, Vz[u], s[2][q]);
+        }
+#pragma unroll
+      for (int k = 0; k < 3; k++) c[k] = first_term(g.w, lane_tree<TPR, double>(s[k]), r[k], di);
+      double pre[3] = {0.0, 0.0, 0.0};
+      for (int it = 0; it < a.iters; it++) {
+        const double Wc = it > 0 ? st.cheb[it - 1] : 0.0;
+        double acc[3], d[3];
+        st.apply((T(&)[3])acc);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          d[k] = it == 0 ? acc[k] + c[k] : fmad(Wc, acc[k] + c[k] - pre[k], pre[k]);
+          pre[k] = xi[k];
+          xi[k] = d[k];
+        }
+        if (!(last && it == a.iters - 1)) {
+          if (!st.exchange(a, j, d, 3, &flag, t0, (double2*)st.xy, (double*)st.z)) return;
+          j++;
+        }
+        if (g.itOut && live && st.part == 0)
+#pragma unroll
+          for (int k = 0; k < 3; k++) g.itOut[(pass * (int64_t)a.iters + it) * g.itStride + k * ld + st.row] = d[k];
+      }
+    }
+  }
+  if (live && st.part == 0)
+#pragma unroll
+    for (int k = 0; k < 3; k++) g.X[k * ld + st.row] = xi[k];
 }
 
 __global__ void k_tile_reset(size_t n, unsigned long long* __restrict__ slots) {
@@ -491,7 +813,26 @@ Solve64 solve64_kernel(const TileConfig& c) {
   return nullptr;
 }
 
-TileShape shape_of(const DeviceMesh& m, int parity, int words, int iters) {
+// Not with one thread per row, nor in FP64 with two: the entries and the passes'
+// other phases would need more registers than a thread has (FP64, 256 rows per
+// tile: 124 us per pass with 100 registers spilled, 92 as separate kernels).
+template <class T>
+auto loop_kernel(const TileConfig& c) -> void (*)(TileShape, TileLoop, const T*) {
+#define PICK(BT, TPR)                                              \
+  if (c.threads == BT && c.tpr == TPR) {                           \
+    if (c.laneMajor) return k_tile_loop<T, BT, TPR, 8, true>;      \
+    if (c.width == 8) return k_tile_loop<T, BT, TPR, 8, false>;    \
+  }
+  PICK(256, 4)
+  PICK(512, 4)
+  if constexpr (sizeof(T) == 4) {
+    PICK(512, 2)
+  }
+#undef PICK
+  return nullptr;
+}
+
+TileShape shape_of(const DeviceMesh& m, int parity, int iters) {
   TileShape a;
   a.n = m.nSim;
   a.ld = m.ld;
@@ -501,8 +842,8 @@ TileShape shape_of(const DeviceMesh& m, int parity, int words, int iters) {
   a.haloOff = m.tile.haloOff;
   a.halo = m.tile.halo;
   a.loc = m.tile.loc;
-  a.slotStride = (size_t)m.ld * words;
-  const size_t set = 4 * (size_t)m.ld * 3;  // words per set, sized for FP64
+  a.slotStride = (size_t)m.ld * kRowWords;
+  const size_t set = 4 * a.slotStride;  // words per set
   a.slots = m.tile.slots + (parity ? set : 0);
   a.other = m.tile.slots + (parity ? 0 : set);
   a.abort = m.tile.abort;
@@ -533,16 +874,21 @@ void tile_check(DeviceMesh& m, int cus, int iters) {
   TileConfig& c = m.tile.cfg;
   m.tile.ok32 = fits(solve32_kernel(c), c.threads, tile_lds_bytes<float>(m.tile.uCap, iters), m.tile.nTiles, cus);
   m.tile.ok64 = fits(solve64_kernel(c), c.threads, tile_lds_bytes<double>(m.tile.uCap, iters), m.tile.nTiles, cus);
+  if (m.tile.curvCap == 0) return;
+  m.tile.loop32 = m.tile.ok32 && fits(loop_kernel<float>(c), c.threads,
+                                      tile_loop_lds<float>(m.tile.uCap, m.tile.curvCap, iters), m.tile.nTiles, cus);
+  m.tile.loop64 = m.tile.ok64 && fits(loop_kernel<double>(c), c.threads,
+                                      tile_loop_lds<double>(m.tile.uCap, m.tile.curvCap, iters), m.tile.nTiles, cus);
 }
 
 void launch_tile_reset(const DeviceMesh& m, hipStream_t s) {
-  const size_t n = 4 * (size_t)m.ld * 3;
+  const size_t n = 4 * (size_t)m.ld * kRowWords;
   hipLaunchKernelGGL(k_tile_reset, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, m.tile.slots);
 }
 
 void launch_tile_solve32(const DeviceMesh& m, int iters, int parity, hipStream_t s) {
   launch_t(m.timer, TC_SWEEP32, solve32_kernel(m.tile.cfg), dim3(m.tile.nTiles), dim3(m.tile.cfg.threads),
-           (uint32_t)tile_lds_bytes<float>(m.tile.uCap, iters), s, shape_of(m, parity, 2, iters), (const float*)m.m2ValF,
+           (uint32_t)tile_lds_bytes<float>(m.tile.uCap, iters), s, shape_of(m, parity, iters), (const float*)m.m2ValF,
            (const float4*)m.r0, m.X);
   if (m.timer) m.timer->weigh(iters - 1);
 }
@@ -551,9 +897,49 @@ void launch_tile_solve64(const DeviceMesh& m, double w, int iters, int parity, d
                          hipStream_t s) {
   const TileFirst ft{m.r1Off, m.r1Col, m.r1Val, m.sysDiag, m.sysRhs, w};
   launch_t(m.timer, TC_SWEEP64, solve64_kernel(m.tile.cfg), dim3(m.tile.nTiles), dim3(m.tile.cfg.threads),
-           (uint32_t)tile_lds_bytes<double>(m.tile.uCap, iters), s, shape_of(m, parity, 3, iters), (const double*)m.m2Val, ft,
+           (uint32_t)tile_lds_bytes<double>(m.tile.uCap, iters), s, shape_of(m, parity, iters), (const double*)m.m2Val, ft,
            m.X, out, outStride);
   if (m.timer) m.timer->weigh(iters - 1);
+}
+
+void launch_tile_loop(const DeviceMesh& m, int precision, double w, int passes, int iters, int withCol,
+                      double* rhsOut, int64_t rhsStride, double* itOut, int64_t itStride, hipStream_t s) {
+  const TileMesh& t = m.tile;
+  TileLoop g;
+  g.curvItems = t.curvItems;
+  g.curvCap = t.curvCap;
+  g.curvLoc = t.curvLoc;
+  g.ringLoc = t.ringLoc;
+  g.ringItem = t.ringItem;
+  g.r1Loc = t.r1Loc;
+  g.ringRange = m.ringRange;
+  g.cRest = m.cRest;
+  g.cStrain = m.cStrain;
+  g.cBendIn = m.cBendIn;
+  g.cLbo = m.cLbo;
+  g.cH0 = m.cH0;
+  g.r1Off = m.r1Off;
+  g.r1Val = m.r1Val;
+  g.D = m.sysDiag;
+  g.initRhs = m.initRhs;
+  g.colRhs = m.colRhs;
+  g.fixK = m.fixK;
+  g.Xrest = m.Xrest;
+  g.withCol = withCol;
+  g.passes = passes;
+  g.w = w;
+  g.X = m.X;
+  g.rhsOut = rhsOut;
+  g.rhsStride = rhsStride;
+  g.itOut = itOut;
+  g.itStride = itStride;
+  const TileShape a = shape_of(m, 0, iters);
+  if (precision == 0)
+    hipLaunchKernelGGL(loop_kernel<double>(t.cfg), dim3(t.nTiles), dim3(t.cfg.threads),
+                       tile_loop_lds<double>(t.uCap, t.curvCap, iters), s, a, g, (const double*)m.m2Val);
+  else
+    hipLaunchKernelGGL(loop_kernel<float>(t.cfg), dim3(t.nTiles), dim3(t.cfg.threads),
+                       tile_loop_lds<float>(t.uCap, t.curvCap, iters), s, a, g, (const float*)m.m2ValF);
 }
 
 }  // namespace pdipc

@@ -124,6 +124,7 @@ int upload_tiles(pdipc_handle* h) {
   t.nTiles = T.nTiles;
   t.rowsPerTile = T.rowsPerTile;
   t.uCap = T.uCap;
+  t.curvCap = T.curvCap;
   tile_check(m, cus, h->prm.cheb_iters);
   if (!t.ok32 && !t.ok64) return PDIPC_OK;
   // the sweeps' weights, as the streamed solves compute them
@@ -138,6 +139,15 @@ int upload_tiles(pdipc_handle* h) {
       (rc = h->upload(&t.halo, T.halo)) || (rc = h->upload(&t.loc, T.loc)) || (rc = h->upload(&t.cheb, W)) ||
       (rc = h->alloc(&t.slots, 2 * 12 * (size_t)m.ld)))
     return rc;
+  if (t.loop32 || t.loop64) {
+    std::vector<int4> items(T.curvItems.size() / 4);
+    for (size_t i = 0; i < items.size(); i++)
+      items[i] = make_int4(T.curvItems[4 * i], T.curvItems[4 * i + 1], T.curvItems[4 * i + 2], T.curvItems[4 * i + 3]);
+    if ((rc = h->upload(&t.curvItems, items)) || (rc = h->upload(&t.curvLoc, T.curvLoc)) ||
+        (rc = h->upload(&t.ringLoc, T.ringLoc)) || (rc = h->upload(&t.ringItem, T.ringItem)) ||
+        (rc = h->upload(&t.r1Loc, T.r1Loc)))
+      return rc;
+  }
   t.abort = (int*)((char*)h->scalDev + 64);
   t.built = true;
   return PDIPC_OK;
@@ -441,6 +451,10 @@ void enqueue_local_global(pdipc_handle* h, int withCol) {
   launch_diag(m, withCol, s);
   launch_operators(m, p.omega, p.precision, s);
   if (m.tile.use(p.precision)) launch_tile_reset(m, s);
+  if (m.tile.loop(p.precision) && !m.timer) {  // kernel timing times the passes' kernels one by one
+    launch_tile_loop(m, p.precision, p.omega, p.lg_iters, p.cheb_iters, withCol, nullptr, 0, nullptr, 0, s);
+    return;
+  }
   for (int it = 0; it < p.lg_iters; it++) {
     bool fused = p.precision == PDIPC_FP32_SPLIT;  // k_rhs also runs the residual's first pass
     launch_local(m, p.precision, p.sigma_lo, p.sigma_hi, withCol, s, fused ? p.omega : -1.0);
