@@ -1011,10 +1011,11 @@ void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, S
   else if (R <= 128) T.threads = 512, T.tpr = 4;
   else if (R <= 256) T.threads = 512, T.tpr = 2;
   else if (R <= 512) T.threads = 512, T.tpr = 1;
+  else if (R <= 1024) T.threads = 1024, T.tpr = 1;  // FP32 only, two rows per launched thread
   else return;  // the entries would not fit a workgroup's registers
   const int wmax = L.nSlices > 0 ? *std::max_element(L.sliceW.begin(), L.sliceW.end()) : 0;
   T.width = wmax <= 8 ? 8 : 12;
-  if (wmax > 12) return;
+  if (wmax > (R <= 512 ? 12 : 8)) return;
   T.rowsPerTile = R;
   T.nTiles = (n + R - 1) / R;
   std::vector<int> order(n);
@@ -1084,6 +1085,10 @@ void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, S
     most = std::max(most, H.size());
   }
   T.uCap = (int)(((size_t)R + most + 7) / 8 * 8);
+  std::vector<char> wanted(n, 0);
+  for (int c : T.halo) wanted[c] = 1;
+  T.rowRead.assign(T.rows.size(), 0);
+  for (size_t i = 0; i < T.rows.size(); i++) T.rowRead[i] = T.rows[i] >= 0 && wanted[T.rows[i]];
   // the staged FP32 rows must fit the 160 KB of LDS (FP64 ones are checked
   // against the device) and an index 16 bits
   if ((size_t)T.uCap * 12 > (160u << 10)) return;

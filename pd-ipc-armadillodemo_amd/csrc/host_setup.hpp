@@ -175,6 +175,7 @@ struct SolveTiles {
   std::vector<int> rows;      // nTiles * rowsPerTile, -1 past the last row
   std::vector<int> rowEntry;  // per row of `rows`: the SELL entry of its lane 0, chunk 0
   std::vector<int> rowWidth;  // and its slice's entries per lane
+  std::vector<int> rowRead;   // and whether another tile's halo holds it
   std::vector<int> haloOff;   // nTiles + 1
   std::vector<int> halo;      // ascending per tile
   std::vector<uint16_t> loc;  // [tile][8-entry chunk][thread][8]

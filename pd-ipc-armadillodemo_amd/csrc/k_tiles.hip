@@ -24,8 +24,9 @@
 // Exchange: an iterate's row is published as 8-byte words (FP32: (x, y) and
 // (z, 0); FP64: x, y, z) by relaxed agent-scope atomic stores, and read by the
 // neighbours with relaxed agent-scope atomic loads that repeat until the word
-// is no longer kTileEmpty, a NaN no iterate can hold.  The data are their own
-// flag: no fence and no barrier between workgroups.  Publication j of a launch
+// is no longer kTileEmpty, a NaN no iterate can hold.  Only rows that other
+// tiles read are published (512^2 cloth, all rows: 8.6 us per sweep, 6.5 with
+// the 44 % that are read).  The data are their own flag: no fence and no barrier between workgroups.  Publication j of a launch
 // goes to slot j % 4.  After publishing j a thread empties its words of
 // publication j - 2: it has staged publication j - 1 of all neighbours, who had
 // staged j - 2 before publishing it (the neighbour relation is symmetric).  It
@@ -40,6 +41,8 @@
 // arrive -- another process's kernels hold compute units for good -- raises
 // the abort flag, every tile leaves, X keeps a finite value, and the host
 // repeats the outer iteration with the streamed kernels.
+#include <algorithm>
+
 #include "device.hpp"
 #include "local_ops.hpp"
 
@@ -102,7 +105,7 @@ __device__ __forceinline__ T lane_tree(const T (&s)[8 / TPR]) {
 
 struct TileShape {  // what one launch works on (device pointers of DeviceMesh)
   int n, ld, R, uCap;
-  const int4* rows;     // [tile][R]: row (-1 past the last), its first SELL entry, entries per lane
+  const int4* rows;     // [tile][R]: row (-1 past the last), its first SELL entry, entries per lane, read by other tiles
   const int* haloOff;   // [tile + 1]
   const int* halo;      // rows of other tiles that the tile's entries read
   const uint16_t* loc;  // [tile][chunk of 8 entries][thread][8]: LDS index per entry
@@ -123,6 +126,7 @@ struct TileState {
   T v[E];
   unsigned li[E / 2];
   int rl, part, row;  // row < 0: this thread holds no row
+  bool pub;           // other tiles read the row
   int nHalo;
   const int* halo;
   V2* xy;  // LDS: the staged iterate, (x, y) pairs and z values, own rows first, then the halo
@@ -130,29 +134,20 @@ struct TileState {
   double* cheb;        // LDS: the sweeps' weights
   int hw[PB];  // word offset of the thread's first polled words (-1: none)
 
-  template <bool EMPTY_OTHER>
-  __device__ __forceinline__ void init(const TileShape& a, const T* __restrict__ val, char* lds) {
-    const int t = threadIdx.x, tile = blockIdx.x;
-    xy = (V2*)lds;
-    z = (T*)(lds + (size_t)a.uCap * sizeof(V2));
-    cheb = (double*)(lds + (size_t)a.uCap * 3 * sizeof(T));
-    for (int k = t; k < a.iters - 1; k += BT) cheb[k] = a.cheb[k];
-    const int ln = t % kWave;
-    rl = (t / kWave) * RW + ln % RW;
-    part = ln / RW;
-    const int4 ri = rl < a.R ? a.rows[(size_t)tile * a.R + rl] : make_int4(-1, 0, 0, 0);
-    row = ri.x;
-    halo = a.halo + a.haloOff[tile];
-    nHalo = a.haloOff[tile + 1] - a.haloOff[tile];
-    const uint4* lp = (const uint4*)a.loc + (size_t)tile * (E / 8) * BT + t;
+  // a row's LDS indices (tables of `threads` threads per tile, here thread t's)
+  static __device__ __forceinline__ void load_loc(const TileShape& a, int threads, int t, unsigned (&li)[E / 2]) {
+    const uint4* lp = (const uint4*)a.loc + (size_t)blockIdx.x * (E / 8) * threads + t;
 #pragma unroll
     for (int c = 0; c < E / 8; c++) {
-      const uint4 q = lp[(size_t)c * BT];
+      const uint4 q = lp[(size_t)c * threads];
       li[4 * c] = q.x;
       li[4 * c + 1] = q.y;
       li[4 * c + 2] = q.z;
       li[4 * c + 3] = q.w;
     }
+  }
+  // the entries of a row in lanes part, part + TPR, ... (threads without a row: some row's)
+  static __device__ __forceinline__ void load_val(const int4& ri, int part, const T* __restrict__ val, T (&v)[E]) {
     if constexpr (LM) {  // lane-major, width 8: a lane's entries are one aligned run
       const T* p = val + ri.y + part * 8;
 #pragma unroll
@@ -178,59 +173,106 @@ struct TileState {
 #pragma unroll
         for (int c = 0; c < W; c++) v[g * W + c] = c < ri.z ? p[(int64_t)c * kWave + g * TPR] : T(0);
     }
-    if (row < 0)
-#pragma unroll
-      for (int e = 0; e < E; e++) v[e] = T(0);
+  }
+  // LDS pointers, weights, halo and the first polled words
+  __device__ __forceinline__ void setup(const TileShape& a, char* lds) {
+    const int t = threadIdx.x, tile = blockIdx.x;
+    xy = (V2*)lds;
+    z = (T*)(lds + (size_t)a.uCap * sizeof(V2));
+    cheb = (double*)(lds + (size_t)a.uCap * 3 * sizeof(T));
+    for (int k = t; k < a.iters - 1; k += BT) cheb[k] = a.cheb[k];
+    halo = a.halo + a.haloOff[tile];
+    nHalo = a.haloOff[tile + 1] - a.haloOff[tile];
 #pragma unroll
     for (int q = 0; q < PB; q++) {
       const int i = t + q * BT;
       hw[q] = i < nHalo * NW ? halo[i / NW] * kRowWords + i % NW : -1;
     }
-    // empty the other set's slots for the next launch
-    if (EMPTY_OTHER && row >= 0 && nHalo > 0)
-      for (int w = part; w < kRowWords; w += TPR)
+  }
+  // empties the other set's words of a published row, for the next launch
+  __device__ __forceinline__ void empty_other(const TileShape& a, int r) const {
+    for (int w = part; w < NW; w += TPR)
 #pragma unroll
-        for (int s = 0; s < 4; s++) publish(a.other + s * a.slotStride + (size_t)row * kRowWords + w, kTileEmpty);
+      for (int s = 0; s < 4; s++) publish(a.other + s * a.slotStride + (size_t)r * kRowWords + w, kTileEmpty);
   }
 
-  // M^2 times the staged iterate, at the thread's row (in all its parts)
-  __device__ __forceinline__ void apply(T (&acc)[3]) {
-    if constexpr (LEAN)  // (opaque per sweep: the compiler would unpack them once for all sweeps)
+  __device__ __forceinline__ void load(const TileShape& a, const int4& ri, const T* __restrict__ val) {
+    load_loc(a, BT, threadIdx.x, li);
+    load_val(ri, part, val, v);
+  }
+  template <bool EMPTY_OTHER, bool LOAD = true>
+  __device__ __forceinline__ int4 init(const TileShape& a, const T* __restrict__ val, char* lds) {
+    setup(a, lds);
+    const int t = threadIdx.x, ln = t % kWave;
+    rl = (t / kWave) * RW + ln % RW;
+    part = ln / RW;
+    const int4 ri = rl < a.R ? a.rows[(size_t)blockIdx.x * a.R + rl] : make_int4(-1, 0, 0, 0);
+    row = ri.x;
+    pub = ri.w != 0;
+    if constexpr (LOAD) load(a, ri, val);
+    if (EMPTY_OTHER && pub) empty_other(a, row);
+    return ri;
+  }
+
+  // M^2 times the staged iterate at one row, lanes G0, G0 + STEP, ... of the
+  // thread's: the lanes' sums advance together, one entry of each per step, so
+  // their additions are independent and the steps' LDS reads overlap them
+  template <int G0, int STEP, int N>
+  __device__ __forceinline__ void lanes(const T (&v)[E], const unsigned (&li)[E / 2], T (&s)[3][N]) const {
 #pragma unroll
-      for (int e = 0; e < E / 2; e++) asm volatile("" : "+v"(li[e]));
-    T s[3][SUBS];
-#pragma unroll
-    for (int g = 0; g < SUBS; g++) s[0][g] = s[1][g] = s[2][g] = T(0);
-    // the lanes' sums advance together, one entry of each per step: their
-    // additions are independent, and the steps' LDS reads overlap them
+    for (int g = 0; g < N; g++) s[0][g] = s[1][g] = s[2][g] = T(0);
 #pragma unroll
     for (int c = 0; c < W; c++) {
-      V2 p[SUBS];
-      T zz[SUBS];
+      V2 p[N];
+      T zz[N];
 #pragma unroll
-      for (int g = 0; g < SUBS; g++) {
-        const int e = g * W + c;
+      for (int g = 0; g < N; g++) {
+        const int e = (G0 + g * STEP) * W + c;
         const unsigned l = (e & 1) ? li[e / 2] >> 16 : li[e / 2] & 0xffffu;
         p[g] = xy[l];
         zz[g] = z[l];
       }
 #pragma unroll
-      for (int g = 0; g < SUBS; g++) {
-        const int e = g * W + c;
+      for (int g = 0; g < N; g++) {
+        const int e = (G0 + g * STEP) * W + c;
         s[0][g] += v[e] * p[g].x;
         s[1][g] += v[e] * p[g].y;
         s[2][g] += v[e] * zz[g];
       }
+      if constexpr (STEP > 1) __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  // the thread's row (in all its parts)
+  __device__ __forceinline__ void apply(T (&acc)[3]) {
+    if constexpr (LEAN)  // (opaque per sweep: the compiler would unpack them once for all sweeps)
 #pragma unroll
-    for (int k = 0; k < 3; k++) acc[k] = lane_tree<TPR, T>(s[k]);
+      for (int e = 0; e < E / 2; e++) asm volatile("" : "+v"(li[e]));
+    if constexpr (TPR == 1 && LEAN) {
+      apply_halves(v, li, acc);
+    } else {
+      T s[3][SUBS];
+      lanes<0, 1, SUBS>(v, li, s);
+#pragma unroll
+      for (int k = 0; k < 3; k++) acc[k] = lane_tree<TPR, T>(s[k]);
+    }
+  }
+  // one thread per row with few registers left: the even lanes, then the odd
+  // ones (the two sides of the lane tree's last addition)
+  __device__ __forceinline__ void apply_halves(const T (&v)[E], const unsigned (&li)[E / 2], T (&acc)[3]) const {
+    T s[3][4], even[3];
+    lanes<0, 2, 4>(v, li, s);
+#pragma unroll
+    for (int k = 0; k < 3; k++) even[k] = (s[k][0] + s[k][2]) + (s[k][1] + s[k][3]);
+    lanes<1, 2, 4>(v, li, s);
+#pragma unroll
+    for (int k = 0; k < 3; k++) acc[k] = even[k] + ((s[k][0] + s[k][2]) + (s[k][1] + s[k][3]));
   }
 
   // publication j of the row (values of type U), emptying `old` words of
   // publication j - 2
   template <class U>
   __device__ __forceinline__ void send(const TileShape& a, int j, const U (&d)[3], int old) const {
-    if (row < 0 || nHalo == 0) return;  // without a halo nobody reads this tile's rows
+    if (!pub) return;
     unsigned long long* s = a.slots + (size_t)row * kRowWords;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the words emptied a sweep ago have reached memory
     for (int w = part; w < TileWords<U>::N; w += TPR)
@@ -376,6 +418,126 @@ __global__ void __launch_bounds__(BT) k_tile_solve32(TileShape a, const float* _
     for (int k = 0; k < 3; k++) X[k * a.ld + st.row] += (double)cur[k];
 }
 
+// The same with two rows per thread (t and t + BT of tables laid out for 2 BT
+// threads), for tiles of 513 to 1024 rows of width 8: entries and LDS indices
+// take 192 of a thread's 256 registers, so r0 and delta_{k-1} are kept in LDS
+// and a row's lanes advance in two halves (even lanes, then odd ones: the two
+// sides of the lane tree's last addition).  512^2 cloth: 117 us per solve (24
+// to load 100 MB of entries and indices, then 6.5 per sweep: 3.4 LDS reads and
+// FMAs, 3.1 exchange) against 270 us streamed (18 per sweep at 5.6 TB/s).
+constexpr int kTwoThreads = 512;
+constexpr size_t tile_two_lds_bytes(int uCap, int iters) {
+  return tile_lds_bytes<float>(uCap, iters) + 2 * (size_t)(2 * kTwoThreads) * 3 * sizeof(float);
+}
+template <bool LM>
+__global__ void __launch_bounds__(kTwoThreads) k_tile_solve32_two(TileShape a, const float* __restrict__ val,
+                                                                  const float4* __restrict__ r0,
+                                                                  double* __restrict__ X) {
+  constexpr int BT = kTwoThreads;
+  using St = TileState<float, BT, 1, 8, LM, 4, true>;
+  extern __shared__ __attribute__((aligned(16))) char tileLds[];
+  __shared__ int flag;
+  if (tile_aborted(a.abort, &flag)) return;
+  St st;
+  st.setup(a, tileLds);
+  st.part = 0;
+  float* rs = (float*)(tileLds + tile_lds_bytes<float>(a.uCap, a.iters));  // r0, then delta_{k-1}, of the own rows
+  float* ps = rs + 3 * 2 * BT;
+  float v[2][St::E];
+  unsigned li[2][St::E / 2];
+  int row[2], rl[2];
+  bool pub[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    rl[q] = threadIdx.x + q * BT;
+    const int4 ri = rl[q] < a.R ? a.rows[(size_t)blockIdx.x * a.R + rl[q]] : make_int4(-1, 0, 0, 0);
+    row[q] = ri.x;
+    St::load_loc(a, 2 * BT, rl[q], li[q]);
+    St::load_val(ri, 0, val, v[q]);
+    pub[q] = ri.w != 0;
+    if (pub[q]) st.empty_other(a, row[q]);
+    const float4 r = row[q] >= 0 ? r0[row[q]] : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row[q] >= 0) {
+      st.xy[rl[q]] = make_float2(r.x, r.y);
+      st.z[rl[q]] = r.z;
+    }
+    rs[3 * rl[q]] = r.x;
+    rs[3 * rl[q] + 1] = r.y;
+    rs[3 * rl[q] + 2] = r.z;
+    ps[3 * rl[q]] = ps[3 * rl[q] + 1] = ps[3 * rl[q] + 2] = 0.f;
+  }
+  for (int u = threadIdx.x; u < st.nHalo; u += BT) {
+    const float4 q = r0[st.halo[u]];
+    st.xy[a.R + u] = make_float2(q.x, q.y);
+    st.z[a.R + u] = q.z;
+  }
+  __syncthreads();
+  const unsigned long long t0 = wall_clock64();
+  for (int it = 1; it < a.iters; it++) {
+    const float Wc = (float)st.cheb[it - 1];
+    float d[2][3];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+#pragma unroll
+      for (int e = 0; e < St::E / 2; e++) asm volatile("" : "+v"(li[q][e]));  // (not unpacked for all sweeps)
+      float acc[3];
+      st.apply_halves(v[q], li[q], acc);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const float pre = ps[3 * rl[q] + k];
+        d[q][k] = Wc * (acc[k] + rs[3 * rl[q] + k] - pre) + pre;
+      }
+    }
+    if (it == a.iters - 1) {
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        if (row[q] >= 0)
+#pragma unroll
+          for (int k = 0; k < 3; k++) X[k * a.ld + row[q]] += (double)d[q][k];
+      return;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the words emptied a sweep ago have reached memory
+    const int j = it - 1;
+    const size_t now = (size_t)(j & 3) * a.slotStride, old = (size_t)((j + 2) & 3) * a.slotStride;
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+      if (pub[q])
+#pragma unroll
+        for (int w = 0; w < 2; w++)
+          publish(a.slots + now + (size_t)row[q] * kRowWords + w, TileWords<float>::word(d[q], w));
+    if (j >= 2)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        if (pub[q])
+#pragma unroll
+          for (int w = 0; w < 2; w++) publish(a.slots + old + (size_t)row[q] * kRowWords + w, kTileEmpty);
+    __syncthreads();  // every row of the tile has read the old iterate
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+      if (row[q] >= 0) {
+        const int r = rl[q];
+        const float2 c = st.xy[r];
+        ps[3 * r] = c.x;
+        ps[3 * r + 1] = c.y;
+        ps[3 * r + 2] = st.z[r];
+        st.xy[r] = make_float2(d[q][0], d[q][1]);
+        st.z[r] = d[q][2];
+      }
+    if (!st.receive(a, j, t0, st.xy, st.z)) {
+      flag = 1;
+      __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (flag != 0) return;
+  }
+  // one sweep only: delta_1 = r0
+#pragma unroll
+  for (int q = 0; q < 2; q++)
+    if (row[q] >= 0)
+#pragma unroll
+      for (int k = 0; k < 3; k++) X[k * a.ld + row[q]] += (double)rs[3 * rl[q] + k];
+}
+
 // FP64: x_0 = X, c computed here from R1, D and b (as k_first64), x_1 = M^2 x_0 + c,
 // x_{k+1} = W_k (M^2 x_k + c - x_{k-1}) + x_{k-1}; the last to X.  With `out`
 // every iterate x_k also goes to out + (k - 1) outStride (SoA).
@@ -396,7 +558,8 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
   using State = TileState<double, BT, TPR, W, LM, 6, tile_lean<double, TPR, W>()>;
   constexpr int SUBS = State::SUBS;
   State st;
-  st.template init<true>(a, val, tileLds);
+  // (one thread per row: the entries' registers are not free before c is formed)
+  const int4 ri = st.template init<true, (TPR > 1)>(a, val, tileLds);
   for (int u = threadIdx.x; u < st.nHalo; u += BT) {
     const int h = st.halo[u];
     st.xy[a.R + u] = make_double2(X[h], X[a.ld + h]);
@@ -442,6 +605,7 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
       c[k] = first_term(ft.w, lane_tree<TPR, double>(s[k]), bi[k], di);
     }
   }
+  if constexpr (TPR == 1) st.load(a, ri, val);
   __syncthreads();
   const unsigned long long t0 = wall_clock64();
   for (int it = 0; it < a.iters; it++) {
@@ -796,7 +960,15 @@ Solve32 solve32_kernel(const TileConfig& c) {
   PICK(512, 2)
   PICK(512, 1)
 #undef PICK
+  if (c.threads == 2 * kTwoThreads && c.width == 8)
+    return c.laneMajor ? k_tile_solve32_two<true> : k_tile_solve32_two<false>;
   return nullptr;
+}
+// launched threads and LDS of an FP32 solve
+int solve32_threads(const TileConfig& c) { return std::min(c.threads, 512); }
+size_t solve32_lds(const TileMesh& t, int iters) {
+  return t.cfg.threads == 2 * kTwoThreads ? tile_two_lds_bytes(t.uCap, iters)
+                                          : tile_lds_bytes<float>(t.uCap, iters);
 }
 Solve64 solve64_kernel(const TileConfig& c) {
 #define PICK(BT, TPR)                                            \
@@ -872,7 +1044,7 @@ bool fits(K kernel, int threads, size_t lds, int tiles, int cus) {
 
 void tile_check(DeviceMesh& m, int cus, int iters) {
   TileConfig& c = m.tile.cfg;
-  m.tile.ok32 = fits(solve32_kernel(c), c.threads, tile_lds_bytes<float>(m.tile.uCap, iters), m.tile.nTiles, cus);
+  m.tile.ok32 = fits(solve32_kernel(c), solve32_threads(c), solve32_lds(m.tile, iters), m.tile.nTiles, cus);
   m.tile.ok64 = fits(solve64_kernel(c), c.threads, tile_lds_bytes<double>(m.tile.uCap, iters), m.tile.nTiles, cus);
   if (m.tile.curvCap == 0) return;
   m.tile.loop32 = m.tile.ok32 && fits(loop_kernel<float>(c), c.threads,
@@ -887,8 +1059,8 @@ void launch_tile_reset(const DeviceMesh& m, hipStream_t s) {
 }
 
 void launch_tile_solve32(const DeviceMesh& m, int iters, int parity, hipStream_t s) {
-  launch_t(m.timer, TC_SWEEP32, solve32_kernel(m.tile.cfg), dim3(m.tile.nTiles), dim3(m.tile.cfg.threads),
-           (uint32_t)tile_lds_bytes<float>(m.tile.uCap, iters), s, shape_of(m, parity, iters), (const float*)m.m2ValF,
+  launch_t(m.timer, TC_SWEEP32, solve32_kernel(m.tile.cfg), dim3(m.tile.nTiles),
+           dim3(solve32_threads(m.tile.cfg)), (uint32_t)solve32_lds(m.tile, iters), s, shape_of(m, parity, iters), (const float*)m.m2ValF,
            (const float4*)m.r0, m.X);
   if (m.timer) m.timer->weigh(iters - 1);
 }

@@ -133,7 +133,7 @@ int upload_tiles(pdipc_handle* h) {
   W[0] = 2.0 / (2.0 - r);
   for (size_t k = 1; k < W.size(); k++) W[k] = 4.0 / (4.0 - r * W[k - 1]);
   std::vector<int4> rows(T.rows.size());
-  for (size_t i = 0; i < rows.size(); i++) rows[i] = make_int4(T.rows[i], T.rowEntry[i], T.rowWidth[i], 0);
+  for (size_t i = 0; i < rows.size(); i++) rows[i] = make_int4(T.rows[i], T.rowEntry[i], T.rowWidth[i], T.rowRead[i]);
   int rc;
   if ((rc = h->upload(&t.rows, rows)) || (rc = h->upload(&t.haloOff, T.haloOff)) ||
       (rc = h->upload(&t.halo, T.halo)) || (rc = h->upload(&t.loc, T.loc)) || (rc = h->upload(&t.cheb, W)) ||

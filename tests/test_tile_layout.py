@@ -23,10 +23,10 @@ def _scene(which):
 
 
 # rows 4 to 9,216 over 1 to 256 tiles: one tile, tiles of 32 rows, and 2, 4
-# and 8 lanes per thread; cloths of varying and of the common width 8, tets
+# and 8 lanes per thread, two rows per thread; cloths of varying and of the common width 8, tets
 # (12 entries per lane), several models
 @pytest.mark.parametrize("which,max_tiles", [("2", 256), ("11", 256), ("12", 256), ("96", 256), ("96", 100),
-                                             ("96", 40), ("96", 20), ("tets", 256), ("tets", 3), ("layers", 256)])
+                                             ("96", 40), ("96", 20), ("96", 10), ("tets", 256), ("tets", 3), ("layers", 256)])
 def test_tiles_cover_the_rows_and_entries(which, max_tiles):
     sim = pdipc.Simulator.from_scene(_scene(which), init=False)
     sim.host_setup()
@@ -91,4 +91,4 @@ def test_tiles_cover_the_rows_and_entries(which, max_tiles):
 def test_scenes_that_do_not_tile():
     sim = pdipc.Simulator.from_scene(_scene("96"), init=False)
     sim.host_setup()
-    assert sim.tile_layout(17) is None  # 543 rows per tile: over a workgroup's registers
+    assert sim.tile_layout(8) is None  # 1,152 rows per tile: over a workgroup's registers
