@@ -135,6 +135,7 @@ struct DeviceMesh {
   float4 *dPre = nullptr, *dCur = nullptr, *dNext = nullptr, *r0 = nullptr;
   // per point
   double *mass = nullptr, *invMass = nullptr, *gravY = nullptr, *fixK = nullptr, *colMass = nullptr;
+  float4* packed = nullptr;  // nTotal 32-byte rows for the record kernels (k_contact.hip)
   int* fixFlag = nullptr;
   double *inertialDiag = nullptr, *elasticDiag = nullptr, *sysDiag = nullptr, *colDiag = nullptr;
   // rows whose diagonal changed since the last M^2 update; dStale forces rows
@@ -347,8 +348,8 @@ void launch_toi_init(const DeviceMesh& m, hipStream_t s);
 void launch_ccd(const DeviceMesh& m, int nRecs, double filter, int iters, double step, double gap, int touchPolicy,
                 hipStream_t s);
 // CCD over m.recs on AoS positions; the minimum of workgroup b into blockMin[b]
-// for b < ceil(nRecs / kBlock) (every such entry written, no atomics)
-void launch_ccd_blockmin(const DeviceMesh& m, int nRecs, const double* x0Aos, const double* x1Aos, double filter,
+// (every entry below the returned count, at most ceil(nRecs / kBlock), is written)
+int launch_ccd_blockmin(const DeviceMesh& m, int nRecs, const double* x0Aos, const double* x1Aos, double filter,
                          int iters, double step, double gap, int touchPolicy, double* blockMin, hipStream_t s);
 // writes colDiag / colRhs of every simulated point (deterministic order)
 int launch_collision(DeviceMesh& m, int nRecs, double dhat, double kappa, double dt, hipStream_t s);

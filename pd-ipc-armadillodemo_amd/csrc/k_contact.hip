@@ -8,6 +8,9 @@
 //                :2756-2892): weight = barrier(d^2) + min(m_p, m_q)/dt^2 on the
 //                four diagonal entries, weight * target on the four rhs rows.
 // Records are int4: point-triangle (p, t0, t1, t2); edge-edge (~a0, a1, b0, b1).
+#include <algorithm>
+#include <cstdint>
+
 #include "device.hpp"
 #include "dual.hpp"
 
@@ -15,6 +18,14 @@ namespace pdipc {
 namespace {
 
 constexpr int kBlock = 256;
+// From here on a pass packs its points and filters the records by certificate;
+// below, packing (4 to 10 us per pass) costs more than it saves.  k_ccd and
+// k_col_terms with every record in full / with certificates: 733 K records 20
+// and 10 us / 17 and 11, 5.2 M 103 and 60 / 49 and 39, 21 M 387 and 213 / 163
+// and 128.
+constexpr int kManyRecs = 1 << 21;
+// the same where nothing is packed (k_ccd_blockmin, 3 M records: 54 -> 41 us)
+constexpr int kManyRecsAos = 1 << 18;
 
 template <class T>
 struct P3T { T v[3]; };
@@ -252,28 +263,161 @@ __host__ __device__ inline P3 load3(const double* X, int ld, int i) { return {{X
 
 __global__ void k_toi_init(unsigned long long* bits) { *bits = (unsigned long long)__double_as_longlong(1.0); }
 
-// One record's ACCD time of impact between positions X0 and X1 (1 when the
-// record shares a vertex or fails the swept-box filter).  Component c of point
-// i is X[c * cs + i * ps]: cs = ld, ps = 1 for the SoA state vectors, cs = 1,
-// ps = 3 for AoS arrays.
-__device__ __forceinline__ double record_toi(int4 r, int cs, int ps, const double* __restrict__ X0,
-                                             const double* __restrict__ X1, double filter, int iters, double step,
-                                             double gapf, int touchPolicy) {
+// ---- certificates: most records are far apart for their motion, or for dHat
+//
+// Per record, k_ccd takes 24 gathered coordinates and about 500 instructions,
+// mostly FP64 (they bound it: 76 % of the vector issue slots), to find that
+// nothing touches within the move, and k_col_terms 12 and 230 to find that the
+// barrier is not active.  For 99 % of a cloth's records a lower bound of the
+// distance says so as well.  It is formed in FP32 from rows packed once per
+// pass (two 16-byte loads per point, or one), where the gathers bound it, and
+// the other records take the full path: the results are the same.
+
+using P3f = P3T<float>;
+// 32-byte rows x, y, z, 0, dx, dy, dz, 0 of a pass's moves (k_pack_moves)
+struct PackedMoves {
+  const float4* rows;
+  __device__ __forceinline__ void get(int i, P3f& x, P3f& dx) const {
+    const float4 a = rows[2 * (int64_t)i], b = rows[2 * (int64_t)i + 1];
+    x = {{a.x, a.y, a.z}};
+    dx = {{b.x, b.y, b.z}};
+  }
+};
+// Moves in FP64: the state vectors, or a caller's arrays of points
+struct SoaMoves {
+  const double *X0, *X1;
+  int64_t ld;
+  __device__ __forceinline__ void get(int i, P3& x, P3& dx) const {
+    x = {{X0[i], X0[ld + i], X0[2 * ld + i]}};
+    const P3 y = {{X1[i], X1[ld + i], X1[2 * ld + i]}};
+    dx = sub(y, x);
+  }
+};
+struct AosMoves {
+  const double *X0, *X1;
+  __device__ __forceinline__ void get(int i, P3& x, P3& dx) const {
+    const int64_t b = 3 * (int64_t)i;
+    x = {{X0[b], X0[b + 1], X0[b + 2]}};
+    const P3 y = {{X1[b], X1[b + 1], X1[b + 2]}};
+    dx = sub(y, x);
+  }
+  __device__ __forceinline__ void get(int i, P3f& x, P3f& dx) const {
+    P3 a, b;
+    get(i, a, b);
+    x = {{(float)a.v[0], (float)a.v[1], (float)a.v[2]}};
+    dx = {{(float)b.v[0], (float)b.v[1], (float)b.v[2]}};
+  }
+};
+
+__global__ void __launch_bounds__(kBlock) k_pack_moves(int n, SoaMoves mv, float4* __restrict__ rows) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  P3 x, dx;
+  mv.get(i, x, dx);
+  rows[2 * (int64_t)i] = make_float4((float)x.v[0], (float)x.v[1], (float)x.v[2], 0.f);
+  rows[2 * (int64_t)i + 1] = make_float4((float)dx.v[0], (float)dx.v[1], (float)dx.v[2], 0.f);
+}
+__global__ void __launch_bounds__(kBlock) k_pack_points(int n, int ld, const double* __restrict__ X,
+                                                        float4* __restrict__ rows) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) rows[i] = make_float4((float)X[i], (float)X[ld + i], (float)X[2 * ld + i], 0.f);
+}
+
+__host__ __device__ inline bool record_ids(int4 r, int id[4]) {  // false for shared-vertex pairs (skipped)
   int type = r.x < 0 ? 1 : 0;
-  int id[4] = {type ? ~r.x : r.x, r.y, r.z, r.w};
+  id[0] = type ? ~r.x : r.x; id[1] = r.y; id[2] = r.z; id[3] = r.w;
   bool skip = type == 0 ? (id[0] == id[1] || id[0] == id[2] || id[0] == id[3])
                         : (id[0] == id[2] || id[0] == id[3] || id[1] == id[2] || id[1] == id[3]);
-  if (skip) return 1.0;
-  P3 x[4], dx[4];
+  return !skip;
+}
+
+// The two primitives' separation along the line n between their centres: their
+// distance is at least gap / |n|, less the rounding of FP32 coordinates,
+// differences, products and roots: under 16 * 2^-24 of the largest coordinate,
+// and so of `size`, their sum (both sides have twice that).
+struct Separation {
+  float gap, len, size;
+};
+__device__ __forceinline__ float sum_abs(const P3f& p) { return fabsf(p.v[0]) + fabsf(p.v[1]) + fabsf(p.v[2]); }
+__device__ __forceinline__ Separation separation(int type, const P3f (&x)[4]) {
+  const P3f a = sub(x[1], x[0]), b = sub(x[2], x[0]), c = sub(x[3], x[0]);
+  const float sa = type == 0 ? 1.f : -1.f;  // point / triangle, or edge (0, 1) / edge (2, 3)
+  P3f n;
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int64_t b = (int64_t)id[q] * ps;
-    x[q] = {{X0[b], X0[b + cs], X0[b + 2 * (int64_t)cs]}};
-    P3 y = {{X1[b], X1[b + cs], X1[b + 2 * (int64_t)cs]}};
-    dx[q] = sub(y, x[q]);
+  for (int k = 0; k < 3; k++) n.v[k] = b.v[k] + c.v[k] + sa * a.v[k];
+  const float pa = dot(n, a), lo = fminf(dot(n, b), dot(n, c));
+  return {type == 0 ? fminf(pa, lo) : lo - fmaxf(pa, 0.f), __builtin_amdgcn_sqrtf(dot(n, n)),
+          (sum_abs(x[0]) + sum_abs(x[1])) + (sum_abs(x[2]) + sum_abs(x[3]))};
+}
+constexpr float kRound = 2e-6f;    // 32 * 2^-24
+constexpr float kMargin = 1.0001f;
+
+// ACCD of the record returns 1 at its first step: it moves less than
+// step * distance.  With all |dx_i - dx_0| <= E (here: the root of their squares'
+// sum, so that a NaN in any of them certifies nothing) no point moves more than
+// 1.75 E against the mean, and the two displacements' sum is at most 3.5 E.  The
+// distance ACCD computes is one between points of the two primitives.  (1e-8:
+// its own test is d > 1e-9.)
+__device__ __forceinline__ bool surely_no_impact(int type, const P3f (&x)[4], const P3f (&dx)[4], float step) {
+  const Separation s = separation(type, x);
+  const P3f a = sub(dx[1], dx[0]), b = sub(dx[2], dx[0]), c = sub(dx[3], dx[0]);
+  const float e = __builtin_amdgcn_sqrtf(dot(a, a) + dot(b, b) + dot(c, c));
+  const float need = kMargin * 3.5f * e + kRound * (sum_abs(dx[0]) + e);
+  const float gap = s.gap - s.len * (kRound * s.size + 1e-8f);
+  return (step * gap > s.len * need) & (gap > 0.f) & (s.gap < 1e30f);
+}
+// the record's distance is at least dHat, so its barrier is not active
+__device__ __forceinline__ bool surely_inactive(int type, const P3f (&x)[4], float dHat) {
+  const Separation s = separation(type, x);
+  return (s.gap > s.len * (kMargin * dHat + kRound * s.size + 1e-8f)) & (s.gap < 1e30f);
+}
+
+// Runs `cheap(r)` over the records, a wavefront of them at a time (branch-free:
+// it takes any record, and the lanes past the last one an empty one), and
+// `full(t)` over those it keeps: they wait in the wavefront's LDS queue until
+// every lane has one (or the records end), so the costly part runs with full
+// wavefronts.  Two wavefronts of records at a time, whose loads overlap, and
+// 1,024 or 4,096 workgroups measured the same: the gathers bound it.
+constexpr int kShareBlocks = 2048;
+struct WaveQueue {
+  int rec[kBlock / kWave][2 * kWave];
+};
+template <class Cheap, class Full>
+__device__ __forceinline__ void for_kept_records(int nRecs, const int4* __restrict__ recs, WaveQueue& queue, Cheap cheap,
+                                                 Full full) {
+  const int lane = threadIdx.x % kWave, stride = gridDim.x * kBlock;
+  int* q = queue.rec[threadIdx.x / kWave];
+  int n = 0;  // queued (the same in every lane)
+  int base = (int)min((int64_t)blockIdx.x * kBlock + (int)threadIdx.x - lane, (int64_t)nRecs);
+  int4 r = lane < nRecs - base ? recs[base + lane] : make_int4(0, 0, 0, 0);
+  for (bool more = true; more;) {
+    const int next = nRecs - base > stride ? base + stride : nRecs;
+    const int4 cur = r;
+    r = lane < nRecs - next ? recs[next + lane] : make_int4(0, 0, 0, 0);
+    const bool keep = cheap(cur) & (lane < nRecs - base);
+    const unsigned long long b = __ballot(keep);
+    if (keep) q[n + (int)__popcll(b & ((1ull << lane) - 1ull))] = base + lane;
+    n += (int)__popcll(b);
+    base = next;
+    more = base < nRecs;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    while (n >= kWave || (!more && n > 0)) {
+      const int m = min(n, kWave);
+      n -= m;
+      if (lane < m) full(q[n + lane]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
   }
-  bool pass = type == 0 ? pt_ccd_filter(x, dx, filter) : ee_ccd_filter(x, dx, filter);
-  return pass ? accd(type, x, dx, iters, step, gapf, touchPolicy) : 1.0;
+}
+
+// a record's points and moves (false: it shares a vertex)
+template <class Moves, class T>
+__device__ __forceinline__ bool record_moves(int4 r, const Moves& mv, P3T<T> (&x)[4], P3T<T> (&dx)[4]) {
+  int id[4];
+  const bool distinct = record_ids(r, id);
+#pragma unroll
+  for (int q = 0; q < 4; q++) mv.get(id[q], x[q], dx[q]);
+  return distinct;
 }
 
 __device__ __forceinline__ double wave_min(double toi) {
@@ -284,34 +428,76 @@ __device__ __forceinline__ double wave_min(double toi) {
   return toi;
 }
 
-__global__ void __launch_bounds__(kBlock) k_ccd(int nRecs, int ld, const int4* __restrict__ recs,
-                                                const double* __restrict__ X0, const double* __restrict__ X1,
-                                                double filter, int iters, double step, double gapf, int touchPolicy,
-                                                unsigned long long* __restrict__ toiBits) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
+struct AccdParams {
+  double filter;
+  int iters;
+  double step, gapf;
+  int touchPolicy;
+};
+// One record's ACCD time of impact (1 when it shares a vertex or fails the
+// swept-box filter)
+template <class Moves>
+__device__ __forceinline__ double record_toi(int4 r, const Moves& mv, const AccdParams& p) {
+  const int type = r.x < 0 ? 1 : 0;
+  P3 x[4], dx[4];
+  if (!record_moves(r, mv, x, dx)) return 1.0;
+  const bool pass = type == 0 ? pt_ccd_filter(x, dx, p.filter) : ee_ccd_filter(x, dx, p.filter);
+  return pass ? accd(type, x, dx, p.iters, p.step, p.gapf, p.touchPolicy) : 1.0;
+}
+// The smallest time of impact over the wavefront's records
+template <class Quick, class Moves>
+__device__ __forceinline__ double share_toi(int nRecs, const int4* __restrict__ recs, const Quick& quick, const Moves& mv,
+                                            const AccdParams& p) {
+  __shared__ WaveQueue queue;
+  const float step = 0.9999f * (float)p.step;
+  double toi = 1.0;
+  for_kept_records(
+      nRecs, recs, queue,
+      [&](int4 r) {
+        P3f x[4], dx[4];
+        const bool distinct = record_moves(r, quick, x, dx);
+        return distinct & !surely_no_impact(r.x < 0 ? 1 : 0, x, dx, step);
+      },
+      [&](int t) {
+        const double v = record_toi(recs[t], mv, p);
+        if (v < toi) toi = v;  // NaN (reference rule) never wins
+      });
+  return wave_min(toi);
+}
+
+// the same, one record per thread
+template <class Moves>
+__device__ __forceinline__ double thread_toi(int nRecs, const int4* __restrict__ recs, const Moves& mv,
+                                             const AccdParams& p) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
   double toi = 1.0;
   if (t < nRecs) {
-    double v = record_toi(recs[t], ld, 1, X0, X1, filter, iters, step, gapf, touchPolicy);
-    if (v < toi) toi = v;  // NaN (reference rule) never wins
+    const double v = record_toi(recs[t], mv, p);
+    if (v < toi) toi = v;
   }
-  toi = wave_min(toi);
+  return wave_min(toi);
+}
+
+__device__ __forceinline__ void lower_toi(double toi, unsigned long long* toiBits) {
   if ((threadIdx.x % kWave) == 0 && toi < 1.0) atomicMin(toiBits, (unsigned long long)__double_as_longlong(toi));
+}
+__global__ void __launch_bounds__(kBlock) k_ccd(int nRecs, const int4* __restrict__ recs, PackedMoves quick, SoaMoves mv,
+                                                AccdParams p, unsigned long long* __restrict__ toiBits) {
+  lower_toi(share_toi(nRecs, recs, quick, mv, p), toiBits);
+}
+// (one record per thread, for few of them)
+__global__ void __launch_bounds__(kBlock) k_ccd_few(int nRecs, const int4* __restrict__ recs, SoaMoves mv, AccdParams p,
+                                                    unsigned long long* __restrict__ toiBits) {
+  lower_toi(thread_toi(nRecs, recs, mv, p), toiBits);
 }
 
 // The same minimum without atomics on AoS positions: each workgroup writes its
 // own minimum to blockMin[blockIdx.x] (every entry of the grid is written).
-__global__ void __launch_bounds__(kBlock) k_ccd_blockmin(int nRecs, const int4* __restrict__ recs,
-                                                         const double* __restrict__ X0, const double* __restrict__ X1,
-                                                         double filter, int iters, double step, double gapf,
-                                                         int touchPolicy, double* __restrict__ blockMin) {
+template <bool MANY>
+__global__ void __launch_bounds__(kBlock) k_ccd_blockmin(int nRecs, const int4* __restrict__ recs, AosMoves mv,
+                                                         AccdParams p, double* __restrict__ blockMin) {
   __shared__ double waveMin[kBlock / kWave];
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  double toi = 1.0;
-  if (t < nRecs) {
-    double v = record_toi(recs[t], 1, 3, X0, X1, filter, iters, step, gapf, touchPolicy);
-    if (v < toi) toi = v;
-  }
-  toi = wave_min(toi);
+  const double toi = MANY ? share_toi(nRecs, recs, mv, mv, p) : thread_toi(nRecs, recs, mv, p);
   if ((threadIdx.x % kWave) == 0) waveMin[threadIdx.x / kWave] = toi;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -394,14 +580,6 @@ __host__ __device__ inline bool pair_terms(int type, const P3T<T>* x, const doub
   return true;
 }
 
-__host__ __device__ inline bool record_ids(int4 r, int id[4]) {  // false for shared-vertex pairs (skipped)
-  int type = r.x < 0 ? 1 : 0;
-  id[0] = type ? ~r.x : r.x; id[1] = r.y; id[2] = r.z; id[3] = r.w;
-  bool skip = type == 0 ? (id[0] == id[1] || id[0] == id[2] || id[0] == id[3])
-                        : (id[0] == id[2] || id[0] == id[3] || id[1] == id[2] || id[1] == id[3]);
-  return !skip;
-}
-
 // The collision terms are summed per point in a fixed order (ascending record,
 // then corner), so the step is bit-reproducible: no floating-point atomics.
 //   1. k_col_terms: each active record appends (wave-aggregated) its weight and
@@ -410,52 +588,75 @@ __host__ __device__ inline bool record_ids(int4 r, int id[4]) {  // false for sh
 //   3. k_col_fill: every (point, record, corner) entry goes to its point's range;
 //   4. k_col_rank: each entry moves to its rank by (record, corner) in the range;
 //   5. k_col_gather: per point, the ordered range is summed.
-__global__ void __launch_bounds__(kBlock) k_col_terms(int nRecs, int ld, int nSim, const int4* __restrict__ recs,
-                                                      const double* __restrict__ X, const double* __restrict__ cm,
-                                                      double dHat, double kappa, double dt, int actCap,
-                                                      int* __restrict__ actRec, double* __restrict__ actW,
-                                                      double* __restrict__ actT, int* __restrict__ ptCount,
-                                                      int* __restrict__ counters) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  int lane = threadIdx.x % kWave;
+struct ColTerms {
+  int ld, nSim, actCap;
+  const int4* recs;
+  const double *X, *cm;
+  double dHat, kappa, dt;
+  int* actRec;
+  double *actW, *actT;
+  int *ptCount, *counters;
+};
+// record t (any subset of a wavefront's lanes)
+__device__ __forceinline__ void record_terms(const ColTerms& c, int t) {
   bool active = false;
   double w = 0.0;
   P3 tgt[4];
   int id[4] = {0, 0, 0, 0};
-  if (t < nRecs) {
-    int4 r = recs[t];
-    int type = r.x < 0 ? 1 : 0;
-    if (record_ids(r, id)) {
-      P3 x[4];
+  const int4 r = c.recs[t];
+  const int type = r.x < 0 ? 1 : 0;
+  if (record_ids(r, id)) {
+    P3 x[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++) x[q] = load3(X, ld, id[q]);
-      if (cd_filter(type, x, dHat)) {
-        double cmq[4] = {cm[id[0]], cm[id[1]], cm[id[2]], cm[id[3]]};
-        active = pair_terms(type, x, cmq, dHat, kappa, dt, &w, tgt);
-      }
+    for (int q = 0; q < 4; q++) x[q] = load3(c.X, c.ld, id[q]);
+    if (cd_filter(type, x, c.dHat)) {
+      const double cmq[4] = {c.cm[id[0]], c.cm[id[1]], c.cm[id[2]], c.cm[id[3]]};
+      active = pair_terms(type, x, cmq, c.dHat, c.kappa, c.dt, &w, tgt);
     }
   }
-  unsigned long long b = __ballot(active);
+  const unsigned long long b = __ballot(active);
   if (!b) return;
-  int leader = __ffsll((long long)b) - 1;
+  const int lane = threadIdx.x % kWave, leader = __ffsll((long long)b) - 1;
   int base = 0;
-  if (lane == leader) base = atomicAdd(counters + 2, (int)__popcll(b));
+  if (lane == leader) base = atomicAdd(c.counters + 2, (int)__popcll(b));
   base = __shfl(base, leader, kWave);
   if (!active) return;
-  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  int a = base + (int)__popcll(b & lt);
-  if (a >= actCap) {
-    atomicOr(counters + 5, 1);  // the host grows the list and repeats the pass
+  const int a = base + (int)__popcll(b & ((1ull << lane) - 1ull));
+  if (a >= c.actCap) {
+    atomicOr(c.counters + 5, 1);  // the host grows the list and repeats the pass
     return;
   }
-  actRec[a] = t;
-  actW[a] = w;
+  c.actRec[a] = t;
+  c.actW[a] = w;
 #pragma unroll
   for (int q = 0; q < 4; q++) {
 #pragma unroll
-    for (int k = 0; k < 3; k++) actT[(int64_t)a * 12 + 3 * q + k] = tgt[q].v[k];
-    if (id[q] < nSim) atomicAdd(ptCount + id[q], 1);
+    for (int k = 0; k < 3; k++) c.actT[(int64_t)a * 12 + 3 * q + k] = tgt[q].v[k];
+    if (id[q] < c.nSim) atomicAdd(c.ptCount + id[q], 1);
   }
+}
+__global__ void __launch_bounds__(kBlock) k_col_terms(int nRecs, const float4* __restrict__ points, ColTerms c) {
+  __shared__ WaveQueue queue;
+  const float dHat = 1.0001f * fabsf((float)c.dHat);
+  for_kept_records(
+      nRecs, c.recs, queue,
+      [&](int4 r) {
+        int id[4];
+        const bool distinct = record_ids(r, id);
+        P3f x[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const float4 p = points[id[q]];
+          x[q] = {{p.x, p.y, p.z}};
+        }
+        return distinct & !surely_inactive(r.x < 0 ? 1 : 0, x, dHat);
+      },
+      [&](int t) { record_terms(c, t); });
+}
+// one record per thread, for few of them
+__global__ void __launch_bounds__(kBlock) k_col_terms_few(int nRecs, ColTerms c) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < nRecs) record_terms(c, t);
 }
 
 // zeroes the pass's counters (counters[2]: active records, counters[5]: list
@@ -709,6 +910,9 @@ __global__ void k_adj_ccd(int ld, int nSim, const int4* __restrict__ recs, int a
 
 }  // namespace
 
+// workgroups of the kernels that share out the records
+static int share_blocks(int nRecs) { return std::min((nRecs + kBlock - 1) / kBlock, kShareBlocks); }
+
 void launch_toi_init(const DeviceMesh& m, hipStream_t s) {
   hipLaunchKernelGGL(k_toi_init, dim3(1), dim3(1), 0, s, m.toiBits);
 }
@@ -716,15 +920,26 @@ void launch_toi_init(const DeviceMesh& m, hipStream_t s) {
 void launch_ccd(const DeviceMesh& m, int nRecs, double filter, int iters, double step, double gap, int touchPolicy,
                 hipStream_t s) {
   if (nRecs <= 0) return;
-  launch_t(m.timer, TC_CCD, k_ccd, dim3((nRecs + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nRecs, m.ld, m.recs,
-           m.Xold, m.X, filter, iters, step, gap, touchPolicy, m.toiBits);
+  const SoaMoves mv{m.Xold, m.X, m.ld};
+  const AccdParams p{filter, iters, step, gap, touchPolicy};
+  if (nRecs < kManyRecs) {
+    launch_t(m.timer, TC_CCD, k_ccd_few, dim3((nRecs + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nRecs, m.recs, mv, p,
+             m.toiBits);
+    return;
+  }
+  hipLaunchKernelGGL(k_pack_moves, dim3((m.nTotal + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nTotal, mv, m.packed);
+  launch_t(m.timer, TC_CCD, k_ccd, dim3(share_blocks(nRecs)), dim3(kBlock), 0, s, nRecs, m.recs, PackedMoves{m.packed},
+           mv, p, m.toiBits);
 }
 
-void launch_ccd_blockmin(const DeviceMesh& m, int nRecs, const double* x0Aos, const double* x1Aos, double filter,
+int launch_ccd_blockmin(const DeviceMesh& m, int nRecs, const double* x0Aos, const double* x1Aos, double filter,
                          int iters, double step, double gap, int touchPolicy, double* blockMin, hipStream_t s) {
-  if (nRecs <= 0) return;
-  hipLaunchKernelGGL(k_ccd_blockmin, dim3((nRecs + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nRecs, m.recs, x0Aos,
-                     x1Aos, filter, iters, step, gap, touchPolicy, blockMin);
+  if (nRecs <= 0) return 0;
+  const bool many = nRecs >= kManyRecsAos;
+  const int blocks = many ? share_blocks(nRecs) : (nRecs + kBlock - 1) / kBlock;
+  hipLaunchKernelGGL(many ? k_ccd_blockmin<true> : k_ccd_blockmin<false>, dim3(blocks), dim3(kBlock), 0, s, nRecs,
+                     m.recs, AosMoves{x0Aos, x1Aos}, AccdParams{filter, iters, step, gap, touchPolicy}, blockMin);
+  return blocks;
 }
 
 void launch_ccd_records(const DeviceMesh& m, const int4* recs, int nRecs, const double* x0, const double* x1,
@@ -765,10 +980,15 @@ void launch_adj_ccd(const DeviceMesh& m, const int4* recs, int argmin, const dou
 int launch_collision(DeviceMesh& m, int nRecs, double dhat, double kappa, double dt, hipStream_t s) {
   hipLaunchKernelGGL(k_col_clear, dim3((m.nSim + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nSim, m.counters,
                      m.ptCount, m.ptCursor);
-  if (nRecs > 0)
-    launch_t(m.timer, TC_BARRIER, k_col_terms, dim3((nRecs + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nRecs, m.ld,
-             m.nSim, m.recs, m.X, m.colMass, dhat, kappa, dt, m.actCap, m.actRec, m.actW, m.actT, m.ptCount,
-             m.counters);
+  const ColTerms c{m.ld,    m.nSim, m.actCap, m.recs, m.X,       m.colMass, dhat,
+                   kappa, dt,     m.actRec, m.actW, m.actT, m.ptCount, m.counters};
+  if (nRecs >= kManyRecs) {
+    hipLaunchKernelGGL(k_pack_points, dim3((m.nTotal + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nTotal, m.ld, m.X,
+                       m.packed);
+    launch_t(m.timer, TC_BARRIER, k_col_terms, dim3(share_blocks(nRecs)), dim3(kBlock), 0, s, nRecs, m.packed, c);
+  } else if (nRecs > 0) {
+    launch_t(m.timer, TC_BARRIER, k_col_terms_few, dim3((nRecs + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nRecs, c);
+  }
   launch_exclusive_scan(m.ptCount, m.ptOff, m.nSim + 1, nullptr, m.ptScan, s);
   launch_t(m.timer, TC_BARRIER, k_col_fill, dim3(512), dim3(kBlock), 0, s, m.ld, m.nSim, m.actCap, m.recs, m.counters,
            m.actRec, m.ptOff, m.ptCursor, m.entKey, m.entA, m.entPt);

@@ -26,8 +26,9 @@
 // neighbours with relaxed agent-scope atomic loads that repeat until the word
 // is no longer kTileEmpty, a NaN no iterate can hold.  Only rows that other
 // tiles read are published (512^2 cloth, all rows: 8.6 us per sweep, 6.5 with
-// the 44 % that are read).  The data are their own flag: no fence and no barrier between workgroups.  Publication j of a launch
-// goes to slot j % 4.  After publishing j a thread empties its words of
+// the 44 % that are read).  The data are their own flag: no fence and no
+// barrier between workgroups.  Publication j of a launch goes to slot j % 4.
+// After publishing j a thread empties its words of
 // publication j - 2: it has staged publication j - 1 of all neighbours, who had
 // staged j - 2 before publishing it (the neighbour relation is symmetric).  It
 // waits for that store before it publishes j + 1 (a whole sweep later, so the

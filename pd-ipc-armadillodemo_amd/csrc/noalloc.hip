@@ -85,7 +85,8 @@ int pdipc_toi_noalloc(pdipc_handle* h, const double* x0, const double* x1, doubl
   if (!scr) return fail(PDIPC_E_ARG, "pdipc_toi_noalloc: no scratch address for the handle's device");
   hipStream_t s = stream ? (hipStream_t)stream : h->stream;
   const pdipc_params& p = h->prm;
-  launch_ccd_blockmin(h->m, nRecs, x0, x1, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap, p.touch_policy, scr, s);
-  hipLaunchKernelGGL(k_toi_reduce, dim3(1), dim3(kReduceThreads), 0, s, scr, nBlocks, p.toi_scale, toi);
+  const int minima = launch_ccd_blockmin(h->m, nRecs, x0, x1, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
+                                         p.touch_policy, scr, s);
+  hipLaunchKernelGGL(k_toi_reduce, dim3(1), dim3(kReduceThreads), 0, s, scr, minima, p.toi_scale, toi);
   return check_launch(h);
 }

@@ -179,6 +179,7 @@ int upload_all(pdipc_handle* h) {
   for (float4* p : {m.dPre, m.dCur, m.dNext, m.r0}) HIPCHK(hipMemsetAsync(p, 0, m.ld * sizeof(float4), h->stream));
   UP(mass, hs.mass); UP(invMass, hs.invMass); UP(gravY, hs.gravY); UP(fixK, hs.fixK); UP(fixFlag, hs.fixFlag);
   UP(colMass, hs.colMass); UP(elasticDiag, hs.elasticDiag);
+  AL(packed, 2 * (size_t)hs.nTotal);
   AL(inertialDiag, hs.nSim); AL(sysDiag, hs.nSim); AL(colDiag, hs.nTotal);
   AL(dStale, hs.nSim); AL(dChanged, hs.nSim); AL(dDirty, hs.nSim);
   HIPCHK(hipMemsetAsync(m.dStale, 1, std::max(1, hs.nSim), h->stream));  // first update recomputes every row

@@ -1,0 +1,46 @@
+"""The record kernels from 2^21 candidate records on, where most records are
+settled by an FP32 certificate: the time of impact and the barrier terms against
+the oracle, which takes every record through the full FP64 path -- for moves
+that keep apart, approach and collide, near the origin and far from it (where
+the certificate's rounding allowance settles fewer records)."""
+
+import numpy as np
+import pytest
+
+import oracle
+import pdipc
+import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pair():
+    sc = scenes.cloth_over_sphere(184, 4, ground=False, seed=3, patch_dim=184, sphere_patch_dim=32, height=0.1505)
+    return sc, oracle.Oracle(sc), pdipc.Simulator.from_scene(sc)
+
+
+# FP64 ACCD and barrier sums differ from the oracle's by the compilers' fused
+# multiply-adds: a few hundred roundings of relative size 1e-16, amplified by
+# distance / coordinate (1e-3 near the origin, 1e-5 at 50 m)
+@pytest.mark.parametrize("offset,tol", [(0.0, 1e-10), (50.0, 1e-8)])
+@pytest.mark.parametrize("noise", [0.0, 1e-5, 4e-4, 2e-3])
+def test_many_records_match_the_oracle(pair, noise, offset, tol):
+    sc, ref, sim = pair
+    rng = np.random.default_rng(int(noise * 1e6))
+    x0 = ref.x() + offset * np.array([1.0, -0.5, 0.25])
+    x0[: ref.sim] += rng.normal(0, 0.3 * noise, (ref.sim, 3))
+    x1 = x0.copy()
+    x1[: ref.sim, 1] -= 0.5 * noise
+    x1[: ref.sim] += rng.normal(0, noise, (ref.sim, 3))
+    print(f"case: moves of {noise:g}, offset {offset:g}", flush=True)
+    recs = sim.debug_broad_phase(x0, x1 - x0)
+    assert len(recs) == len(ref.debug_broad_phase(x0, x1 - x0)) and len(recs) >= 1 << 21
+    got, want = sim.debug_toi(x0, x1), ref.debug_toi(x0, x1)
+    print(f"  {len(recs)} records, time of impact {got!r}", flush=True)
+    assert (got < 1.0) == (want < 1.0) and abs(got - want) <= tol * want
+    dg, rg, ng = sim.debug_collision(x0)
+    do, ro, no = ref.debug_collision(x0)
+    assert ng == no
+    assert np.abs(dg - do).max() <= tol * np.abs(do).max()
+    assert np.abs(rg - ro).max() <= tol * np.abs(ro).max()
