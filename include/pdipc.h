@@ -224,8 +224,9 @@ int pdipc_sweep_staging(pdipc_handle* h, int* path);
  * the streamed sweeps bit for bit.  info: [0] 1 if this handle has the tables,
  * [1] / [2] 1 if its FP32 / FP64 solves run as tiles, [3] tiles, [4] rows per
  * tile, [5] outer iterations repeated with the streamed sweeps because a tile
- * gave up waiting for its neighbours.  request_abort != 0 makes the next tile
- * solve give up (tests). */
+ * gave up waiting for its neighbours (a backward pass repeated so counts as
+ * one).  request_abort makes the next tile solve of a step (1) or of a backward
+ * pass (2) give up (tests). */
 int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort);
 /* The tile tables for at most max_tiles tiles from the host precompute alone
  * (after pdipc_host_setup; no device).  sizes: [0] 1 if the scene tiles, [1]

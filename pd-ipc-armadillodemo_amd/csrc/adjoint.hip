@@ -136,17 +136,15 @@ struct AdjointState {
   // local/global loops of the recorded forward and of the reverse pass,
   // captured once per collision flag
   hipGraphExec_t fwdGraph[2][2] = {};  // [tile solves][collision flag]
-  hipGraphExec_t revGraph[2] = {nullptr, nullptr};
+  hipGraphExec_t revGraph[2][2] = {};  // the same
   double stats[4] = {0, 0, 0, 0};  // recorded outer iterations, tape bytes, segments, steps
 };
 
 void adjoint_free(AdjointState* a) {
   if (!a) return;
-  for (auto& tiles : a->fwdGraph)
-    for (auto& g : tiles)
-      if (g) (void)hipGraphExecDestroy(g);
-  for (auto& g : a->revGraph)
-    if (g) (void)hipGraphExecDestroy(g);
+  for (auto& graphs : {a->fwdGraph, a->revGraph})
+    for (int t = 0; t < 4; t++)
+      if (graphs[t / 2][t % 2]) (void)hipGraphExecDestroy(graphs[t / 2][t % 2]);
   for (void* p : a->allocs) (void)hipFree(p);
   for (double* p : a->ckX) (void)hipFree(p);
   for (double* p : a->ckV) (void)hipFree(p);
@@ -497,12 +495,14 @@ int reverse_step(pdipc_handle* h, StepTape& st, const double* xbarIn, const doub
     HIPCHK(hipMemsetAsync(m.dChanged, 1, m.nSim, s));
     HIPCHK(hipMemsetAsync(m.dStale, 1, m.nSim, s));  // the next plain step recomputes every row
     launch_operators(m, p.omega, PDIPC_FP64, s);
-    int rc = run_captured(h, A->revGraph[ot.withCol], [&]() {
+    const bool tiles = m.tile.on && m.tile.adj;
+    int rc = run_captured(h, A->revGraph[tiles ? 1 : 0][ot.withCol], [&]() {
+      if (tiles) launch_tile_reset(m, s);
       for (int l = LG - 1; l >= 0; l--) {
         launch_div_rows(m, A->asol, m.sysDiag, A->uS[K], s);  // u_K
         launch_zero(A->uc, (int64_t)V3, s);
         launch_adj_pass(m, A->am, W.data(), K, A->uS.data(), L.it(sg, l, 0), L.it(sg, l, 1), (int64_t)V3,
-                        A->Gbar, A->uc, s);
+                        A->Gbar, A->uc, s, tiles ? (LG - 1 - l) & 1 : -1);
         launch_adj_first(m, p.omega, L.rhs(sg, l), A->uc, A->bbar, A->Dbar, A->R1bar, s);
         launch_adj_local(m, A->am, p.sigma_lo, p.sigma_hi, L.it(sg, l, 0), A->bbar, A->uS[0], A->aA, A->tetAdj,
                          A->asol, A->sbar, A->rhs0bar, ot.withCol ? A->colRacc : nullptr, s);
@@ -523,6 +523,66 @@ int reverse_step(pdipc_handle* h, StepTape& st, const double* xbarIn, const doub
     if ((rc = check_launch(h))) return rc;
   }
   return PDIPC_OK;
+}
+
+// The adjoints of the rolled-out final state (dx, dv) through every step to the
+// initial one (*xOut, *vOut); the stiffness adjoints in sbar, R1bar, DbarEl.
+int reverse_rollout(pdipc_handle* h, const double* dx, const double* dv, double** xOut, double** vOut) {
+  int rc;
+  AdjointState* A = h->adj;
+  DeviceMesh& m = h->m;
+  const HostSetup& hs = h->hs;
+  hipStream_t s = h->stream;
+  const size_t V3 = 3 * (size_t)m.ld;
+  // seeds (AoS over the simulated points; null = zero)
+  std::vector<double> zero(3 * (size_t)m.nSim, 0.0);
+  if ((rc = put_soa(h, A->xbarA, dx ? dx : zero.data(), m.nSim))) return rc;
+  if ((rc = put_soa(h, A->vbarA, dv ? dv : zero.data(), m.nSim))) return rc;
+  launch_zero(A->sbar, (int64_t)hs.cNbr.size(), s);
+  launch_zero(A->R1bar, (int64_t)hs.r1Col.size(), s);
+  launch_zero(A->DbarEl, m.nSim, s);
+  double *xin = A->xbarA, *vin = A->vbarA, *xout = A->xbarB, *vout = A->vbarB;
+  A->stats[2] = 0;
+  if (A->recorded) {  // the rollout's own tape, every step
+    for (int n = A->nSteps - 1; n >= 0; n--) {
+      if ((rc = reverse_step(h, A->seg[n], xin, vin, xout, vout))) return rc;
+      std::swap(xin, xout);
+      std::swap(vin, vout);
+    }
+  }
+  A->stats[0] = A->recorded ? A->stats[0] : 0;
+  double tapeBytes = A->recorded ? A->stats[1] : 0;
+  int nseg = A->recorded ? 0 : (A->nSteps + A->every - 1) / A->every;
+  for (int sg = nseg - 1; sg >= 0; sg--) {
+    int first = sg * A->every, last = std::min(A->nSteps, first + A->every);
+    if (A->lastKept && sg == nseg - 1) {
+      for (const StepTape& st : A->seg) A->stats[0] += (double)st.outers.size();
+    } else {
+      launch_copy(m.X, A->ckX[sg], (int64_t)V3, s);
+      launch_copy(m.V, A->ckV[sg], (int64_t)V3, s);
+      A->lastKept = false;  // the tape now holds this segment
+      A->tape.reset();
+      A->seg.assign(last - first, StepTape());
+      for (int n = first; n < last; n++)
+        if ((rc = taped_step(h, A->seg[n - first]))) return rc;
+    }
+    double used = 0;
+    for (size_t c = 0; c < A->tape.ci && c < A->tape.chunks.size(); c++) used += (double)A->tape.chunks[c].size;
+    used += (double)A->tape.off;
+    tapeBytes = std::max(tapeBytes, used);
+    for (int n = last - 1; n >= first; n--) {
+      if ((rc = reverse_step(h, A->seg[n - first], xin, vin, xout, vout))) return rc;
+      std::swap(xin, xout);
+      std::swap(vin, vout);
+    }
+    A->stats[2] += 1;
+  }
+  A->stats[1] = tapeBytes;
+  A->stats[3] = A->nSteps;
+  HIPCHK(hipStreamSynchronize(s));
+  *xOut = xin;
+  *vOut = vin;
+  return check_launch(h);
 }
 
 }  // namespace
@@ -610,53 +670,18 @@ int pdipc_backward(pdipc_handle* h, const double* dx, const double* dv, double* 
   const HostSetup& hs = h->hs;
   hipStream_t s = h->stream;
   size_t V3 = 3 * (size_t)m.ld;
-  // seeds (AoS over the simulated points; null = zero)
-  std::vector<double> zero(3 * (size_t)m.nSim, 0.0);
-  if ((rc = put_soa(h, A->xbarA, dx ? dx : zero.data(), m.nSim))) return rc;
-  if ((rc = put_soa(h, A->vbarA, dv ? dv : zero.data(), m.nSim))) return rc;
-  launch_zero(A->sbar, (int64_t)hs.cNbr.size(), s);
-  launch_zero(A->R1bar, (int64_t)hs.r1Col.size(), s);
-  launch_zero(A->DbarEl, m.nSim, s);
-  double *xin = A->xbarA, *vin = A->vbarA, *xout = A->xbarB, *vout = A->vbarB;
-  A->stats[2] = 0;
-  if (A->recorded) {  // the rollout's own tape, every step
-    for (int n = A->nSteps - 1; n >= 0; n--) {
-      if ((rc = reverse_step(h, A->seg[n], xin, vin, xout, vout))) return rc;
-      std::swap(xin, xout);
-      std::swap(vin, vout);
+  double *xin = nullptr, *vin = nullptr;
+  if ((rc = reverse_rollout(h, dx, dv, &xin, &vin))) return rc;
+  if (m.tile.built && m.tile.adj) {
+    int gaveUp = 0;  // a tile of some reverse pass gave up waiting: once more, with the streamed sweeps
+    HIPCHK(h->copy(&gaveUp, m.tile.abort + 1, sizeof gaveUp, hipMemcpyDeviceToHost));
+    if (gaveUp) {
+      h->tileAborts++;
+      m.tile.on = false;
+      HIPCHK(hipMemsetAsync(m.tile.abort + 1, 0, sizeof gaveUp, s));
+      if ((rc = reverse_rollout(h, dx, dv, &xin, &vin))) return rc;
     }
   }
-  A->stats[0] = A->recorded ? A->stats[0] : 0;
-  double tapeBytes = A->recorded ? A->stats[1] : 0;
-  int nseg = A->recorded ? 0 : (A->nSteps + A->every - 1) / A->every;
-  for (int sg = nseg - 1; sg >= 0; sg--) {
-    int first = sg * A->every, last = std::min(A->nSteps, first + A->every);
-    if (A->lastKept && sg == nseg - 1) {
-      for (const StepTape& st : A->seg) A->stats[0] += (double)st.outers.size();
-    } else {
-      launch_copy(m.X, A->ckX[sg], (int64_t)V3, s);
-      launch_copy(m.V, A->ckV[sg], (int64_t)V3, s);
-      A->lastKept = false;  // the tape now holds this segment
-      A->tape.reset();
-      A->seg.assign(last - first, StepTape());
-      for (int n = first; n < last; n++)
-        if ((rc = taped_step(h, A->seg[n - first]))) return rc;
-    }
-    double used = 0;
-    for (size_t c = 0; c < A->tape.ci && c < A->tape.chunks.size(); c++) used += (double)A->tape.chunks[c].size;
-    used += (double)A->tape.off;
-    tapeBytes = std::max(tapeBytes, used);
-    for (int n = last - 1; n >= first; n--) {
-      if ((rc = reverse_step(h, A->seg[n - first], xin, vin, xout, vout))) return rc;
-      std::swap(xin, xout);
-      std::swap(vin, vout);
-    }
-    A->stats[2] += 1;
-  }
-  A->stats[1] = tapeBytes;
-  A->stats[3] = A->nSteps;
-  HIPCHK(hipStreamSynchronize(s));
-  if ((rc = check_launch(h))) return rc;
   if (dx0 && (rc = get_soa(h, xin, dx0, m.nSim))) return rc;
   if (dv0 && (rc = get_soa(h, vin, dv0, m.nSim))) return rc;
   if (dk) {

@@ -111,7 +111,8 @@ struct TileMesh {
   uint16_t* loc = nullptr;
   unsigned long long* slots = nullptr;  // two sets of four publication slots
   double* cheb = nullptr;               // W_1 .. of the Chebyshev recurrence
-  int* abort = nullptr;                 // set by a tile that gave up waiting
+  int* abort = nullptr;                 // set by a tile that gave up waiting (abort[1]: in a reverse pass)
+  bool adj = false;                     // the reverse sweeps' kernel fits
   // the local/global loop in one launch (scenes of cloths only, curvCap > 0)
   bool loop32 = false, loop64 = false;
   int curvCap = 0;
@@ -269,6 +270,8 @@ void launch_tile_solve64(const DeviceMesh& m, double w, int iters, int parity, d
 // with rhsOut / itOut (FP64) every pass's rhs and iterates are recorded
 void launch_tile_loop(const DeviceMesh& m, int precision, double w, int passes, int iters, int withCol,
                       double* rhsOut, int64_t rhsStride, double* itOut, int64_t itStride, hipStream_t s);
+struct TileAdj;
+void launch_tile_adj(const DeviceMesh& m, const TileAdj& g, int parity, hipStream_t s);
 // k_solve.hip
 void launch_operators(const DeviceMesh& m, double omega, int precision, hipStream_t s);
 void launch_solve(const DeviceMesh& m, double omega, double rho, int chebIters, int precision, hipStream_t s,
@@ -301,10 +304,20 @@ void launch_solve_taped(const DeviceMesh& m, double omega, double rho, int iters
                         int parity = 0);
 // the whole reverse of one K-sweep solve: u[k] for k = K-1 .. 0 from u[K] (given)
 // and u[K+1] (zero), then one SELL pass adding sum_k W_k u_{k+1} x_k^T to Gbar,
-// with the forward iterates x_0 and x_k = x1 + (k-1) xStride (k >= 1)
+// with the forward iterates x_0 and x_k = x1 + (k-1) xStride (k >= 1).
+// parity: the slot set of a tile solve, which the caller alternates between
+// passes (-1: streamed sweeps)
 constexpr int kMaxCheb = 32;
+// one pass's reverse sweeps: u_0 .. u_K, their weights W_0 .. W_{K-1}, and uc
+struct TileAdj {
+  double* u[kMaxCheb + 1];
+  double w[kMaxCheb];
+  double* uc;
+  int K;
+};
 void launch_adj_pass(const DeviceMesh& m, const AdjMesh& a, const double* W, int K, double* const* u,
-                     const double* x0, const double* x1, int64_t xStride, double* Gbar, double* uc, hipStream_t s);
+                     const double* x0, const double* x1, int64_t xStride, double* Gbar, double* uc, hipStream_t s,
+                     int parity = -1);
 void launch_adj_first(const DeviceMesh& m, double omega, const double* b, const double* uc, double* bbar, double* Dbar,
                       double* R1bar, hipStream_t s);
 // adjoint of the operator update (M^2 from D and R1) as three deterministic

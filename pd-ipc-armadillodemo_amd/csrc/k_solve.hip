@@ -1215,9 +1215,18 @@ __global__ void __launch_bounds__(kBlock, 8) k_adj_spmv_s(int n, int nSlices, in
 
 template <int G>
 void adj_pass_impl(const DeviceMesh& m, const AdjMesh& a, const double* W, int K, double* const* u, const double* x0,
-                   const double* x1, int64_t xStride, double* Gbar, double* uc, hipStream_t s) {
+                   const double* x1, int64_t xStride, double* Gbar, double* uc, hipStream_t s, int parity) {
   const int grid = (m.nSlices * kWave + kBlock - 1) / kBlock;
-  for (int k = K - 1; k >= 0; k--) {
+  const bool tiles = G == 8 && parity >= 0;
+  if (tiles) {
+    TileAdj g;
+    g.K = K;
+    for (int k = 0; k <= K; k++) g.u[k] = u[k];
+    for (int k = 0; k < K; k++) g.w[k] = W[k];
+    g.uc = uc;
+    launch_tile_adj(m, g, parity, s);
+  }
+  for (int k = tiles ? -1 : K - 1; k >= 0; k--) {
     double b = k + 1 <= K - 1 ? 1.0 - W[k + 1] : 0.0;
     bool staged = false;
     if constexpr (G > 1) {
@@ -1431,12 +1440,13 @@ void launch_solve_taped(const DeviceMesh& m, double omega, double rho, int iters
 }
 
 void launch_adj_pass(const DeviceMesh& m, const AdjMesh& a, const double* W, int K, double* const* u,
-                     const double* x0, const double* x1, int64_t xStride, double* Gbar, double* uc, hipStream_t s) {
+                     const double* x0, const double* x1, int64_t xStride, double* Gbar, double* uc, hipStream_t s,
+                     int parity) {
   switch (m.sellLanes) {
-    case 1: adj_pass_impl<1>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s); break;
-    case 2: adj_pass_impl<2>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s); break;
-    case 8: adj_pass_impl<8>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s); break;
-    default: adj_pass_impl<4>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s); break;
+    case 1: adj_pass_impl<1>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s, parity); break;
+    case 2: adj_pass_impl<2>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s, parity); break;
+    case 8: adj_pass_impl<8>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s, parity); break;
+    default: adj_pass_impl<4>(m, a, W, K, u, x0, x1, xStride, Gbar, uc, s, parity); break;
   }
 }
 

@@ -635,6 +635,57 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
     for (int k = 0; k < 3; k++) X[k * a.ld + st.row] = cur[k];
 }
 
+// The reverse sweeps of one pass (the adjoint's recurrence on u = D^{-1} xbar,
+// k_solve.hip): from u_K, u_k = W_k M^2 u_{k+1} + b_k u_{k+2} for k = K - 1 .. 0
+// with b_k = 1 - W_{k+1} (none at K - 1), every u_k stored and
+// uc += W_k u_{k+1}.  128^2 cloth, 15 sweeps: 37.5 us, about 80 as
+// streamed sweeps with their boundaries (4.6 each).
+template <int BT, int TPR, int W, bool LM>
+__global__ void __launch_bounds__(BT) k_tile_adj(TileShape a, const double* __restrict__ val, TileAdj g) {
+  extern __shared__ __attribute__((aligned(16))) char tileLds[];
+  __shared__ int flag;
+  if (tile_aborted(a.abort, &flag)) return;
+  TileState<double, BT, TPR, W, LM, 6, tile_lean<double, TPR, W>()> st;
+  st.template init<true>(a, val, tileLds);
+  const double* u0 = g.u[g.K];
+  for (int q = threadIdx.x; q < st.nHalo; q += BT) {
+    const int h = st.halo[q];
+    st.xy[a.R + q] = make_double2(u0[h], u0[a.ld + h]);
+    st.z[a.R + q] = u0[2 * a.ld + h];
+  }
+  double oth[3] = {0.0, 0.0, 0.0}, cur[3] = {0.0, 0.0, 0.0}, uc[3] = {0.0, 0.0, 0.0};
+  if (st.row >= 0) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      cur[k] = u0[k * a.ld + st.row];
+      uc[k] = g.uc[k * a.ld + st.row];
+    }
+    st.stage_own(st.xy, st.z, cur[0], cur[1], cur[2]);
+  }
+  __syncthreads();
+  const unsigned long long t0 = wall_clock64();
+  for (int k = g.K - 1; k >= 0; k--) {
+    const double w = g.w[k], b = k + 1 <= g.K - 1 ? 1.0 - g.w[k + 1] : 0.0;
+    double acc[3], d[3];
+    st.apply(acc);
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      const double o = b != 0.0 ? b * oth[q] : 0.0;
+      d[q] = fmad(w, acc[q], o);
+      uc[q] = fmad(w, cur[q], uc[q]);
+      oth[q] = cur[q];
+      cur[q] = d[q];
+    }
+    if (k > 0 && !st.exchange(a, g.K - 1 - k, d, 3, &flag, t0, st.xy, st.z)) return;
+    if (st.row >= 0 && st.part == 0)
+#pragma unroll
+      for (int q = 0; q < 3; q++) g.u[k][q * a.ld + st.row] = d[q];
+  }
+  if (st.row >= 0 && st.part == 0)
+#pragma unroll
+    for (int q = 0; q < 3; q++) g.uc[q * a.ld + st.row] = uc[q];
+}
+
 // ---- the whole local/global loop of an outer iteration
 //
 // For scenes of cloths only, one launch runs every local/global pass: the
@@ -986,6 +1037,22 @@ Solve64 solve64_kernel(const TileConfig& c) {
   return nullptr;
 }
 
+using Adj = void (*)(TileShape, const double*, TileAdj);
+Adj adj_kernel(const TileConfig& c) {
+#define PICK(BT, TPR)                                            \
+  if (c.threads == BT && c.tpr == TPR) {                         \
+    if (c.laneMajor) return k_tile_adj<BT, TPR, 8, true>;        \
+    if (c.width == 8) return k_tile_adj<BT, TPR, 8, false>;      \
+    if (c.width == 12 && TPR > 1) return k_tile_adj<BT, TPR, (TPR > 1 ? 12 : 8), false>; \
+  }
+  PICK(256, 4)
+  PICK(512, 4)
+  PICK(512, 2)
+  PICK(512, 1)
+#undef PICK
+  return nullptr;
+}
+
 // Not with one thread per row, nor in FP64 with two: the entries and the passes'
 // other phases would need more registers than a thread has (FP64, 256 rows per
 // tile: 124 us per pass with 100 registers spilled, 92 as separate kernels).
@@ -1047,6 +1114,8 @@ void tile_check(DeviceMesh& m, int cus, int iters) {
   TileConfig& c = m.tile.cfg;
   m.tile.ok32 = fits(solve32_kernel(c), solve32_threads(c), solve32_lds(m.tile, iters), m.tile.nTiles, cus);
   m.tile.ok64 = fits(solve64_kernel(c), c.threads, tile_lds_bytes<double>(m.tile.uCap, iters), m.tile.nTiles, cus);
+  m.tile.adj = m.tile.ok64 &&
+               fits(adj_kernel(c), c.threads, tile_lds_bytes<double>(m.tile.uCap, iters), m.tile.nTiles, cus);
   if (m.tile.curvCap == 0) return;
   m.tile.loop32 = m.tile.ok32 && fits(loop_kernel<float>(c), c.threads,
                                       tile_loop_lds<float>(m.tile.uCap, m.tile.curvCap, iters), m.tile.nTiles, cus);
@@ -1073,6 +1142,13 @@ void launch_tile_solve64(const DeviceMesh& m, double w, int iters, int parity, d
            (uint32_t)tile_lds_bytes<double>(m.tile.uCap, iters), s, shape_of(m, parity, iters), (const double*)m.m2Val, ft,
            m.X, out, outStride);
   if (m.timer) m.timer->weigh(iters - 1);
+}
+
+void launch_tile_adj(const DeviceMesh& m, const TileAdj& g, int parity, hipStream_t s) {
+  TileShape a = shape_of(m, parity, g.K);
+  a.abort = m.tile.abort + 1;  // the forward passes' flag has the host repeat an outer iteration
+  hipLaunchKernelGGL(adj_kernel(m.tile.cfg), dim3(m.tile.nTiles), dim3(m.tile.cfg.threads),
+                     tile_lds_bytes<double>(m.tile.uCap, g.K), s, a, (const double*)m.m2Val, g);
 }
 
 void launch_tile_loop(const DeviceMesh& m, int precision, double w, int passes, int iters, int withCol,

@@ -1074,7 +1074,7 @@ int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort) {
   }
   if (request_abort && t.built) {
     const int one = 1;
-    HIPCHK(hipMemcpyAsync(t.abort, &one, sizeof(int), hipMemcpyHostToDevice, h->stream));
+    HIPCHK(hipMemcpyAsync(t.abort + (request_abort == 2 ? 1 : 0), &one, sizeof(int), hipMemcpyHostToDevice, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
   }
   return PDIPC_OK;

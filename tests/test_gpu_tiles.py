@@ -86,6 +86,13 @@ def test_given_up_solve_repeats_with_streamed_sweeps(prec):
         for u, w in zip(c.backward(dx=g), d.backward(dx=g)):
             assert np.allclose(u, w, rtol=1e-9, atol=1e-12 * max(np.abs(w).max(initial=0.0), 1e-300))
         assert c.tile_solves()["aborts"] == 1
+        # a reverse pass that gives up: the backward is repeated with the streamed sweeps
+        e = pdipc.Simulator.from_scene(sc, precision=prec)
+        e.rollout(3, 2)
+        e.tile_solves(request_abort=2)
+        for u, w in zip(e.backward(dx=g), d.backward(dx=g)):
+            assert np.allclose(u, w, rtol=1e-9, atol=1e-12 * max(np.abs(w).max(initial=0.0), 1e-300))
+        assert e.tile_solves()["aborts"] == 1
 
 
 @pytest.mark.parametrize("n", [2, 11, 40, 150])
