@@ -361,7 +361,8 @@ void launch_toi_init(const DeviceMesh& m, hipStream_t s);
 void launch_ccd(const DeviceMesh& m, int nRecs, double filter, int iters, double step, double gap, int touchPolicy,
                 hipStream_t s);
 // CCD over m.recs on AoS positions; the minimum of workgroup b into blockMin[b]
-// (every entry below the returned count, at most ceil(nRecs / kBlock), is written)
+// (every entry below the returned count, at most kMaxToiBlocks, is written)
+constexpr int kMaxToiBlocks = 2048;
 int launch_ccd_blockmin(const DeviceMesh& m, int nRecs, const double* x0Aos, const double* x1Aos, double filter,
                          int iters, double step, double gap, int touchPolicy, double* blockMin, hipStream_t s);
 // writes colDiag / colRhs of every simulated point (deterministic order)

@@ -41,6 +41,7 @@ struct pdipc_handle {
   DeviceMesh m;
   hipStream_t stream = nullptr;
   int device = 0;  // the HIP device current at pdipc_init
+  int toiSlot = 0;  // part of the device's array that pdipc_toi_noalloc writes
   // local/global loop captured once per (tile solves, collision flag, precision) and replayed
   hipGraphExec_t lgGraph[2][2][2] = {};
   int tileAborts = 0;  // outer iterations repeated with the streamed sweeps
@@ -139,5 +140,5 @@ class TileTurn {
 constexpr int kTileAborted = 1000;
 int tile_recover(pdipc_handle* h, int outer);
 int adjoint_refresh_values(pdipc_handle* h);  // adjoint.hip: after a stiffness change
-int noalloc_setup(int device);                 // noalloc.hip: with `device` current
+int noalloc_setup(int device, int* slot);      // noalloc.hip: with `device` current
 }  // namespace pdipc

@@ -26,6 +26,7 @@ constexpr int kBlock = 256;
 constexpr int kManyRecs = 1 << 21;
 // the same where nothing is packed (k_ccd_blockmin, 3 M records: 54 -> 41 us)
 constexpr int kManyRecsAos = 1 << 18;
+static_assert(kManyRecsAos / kBlock <= kMaxToiBlocks, "one workgroup minimum each");
 
 template <class T>
 struct P3T { T v[3]; };
@@ -378,7 +379,7 @@ __device__ __forceinline__ bool surely_inactive(int type, const P3f (&x)[4], flo
 // every lane has one (or the records end), so the costly part runs with full
 // wavefronts.  Two wavefronts of records at a time, whose loads overlap, and
 // 1,024 or 4,096 workgroups measured the same: the gathers bound it.
-constexpr int kShareBlocks = 2048;
+constexpr int kShareBlocks = kMaxToiBlocks;
 struct WaveQueue {
   int rec[kBlock / kWave][2 * kWave];
 };

@@ -3,7 +3,8 @@
 // allocate device memory -- code under HIP graph capture, tight serving loops.
 // Positions and the result stay on the device, the work is only enqueued, and
 // the per-workgroup minima live in `scratch`, a file-scope device array each
-// GPU holds for the life of the process.  Its device address comes from
+// GPU holds for the life of the process, in slots that handles take in turn (a
+// call writes at most 2,048 minima).  Its device address comes from
 // hipGetSymbolAddress once per device (pdipc_init, with the handle's device
 // current); host code passes that address, never the array's name.
 #include <hip/hip_runtime.h>
@@ -17,15 +18,16 @@ namespace pdipc {
 
 namespace {
 
-constexpr int kRecsPerBlock = 256;     // k_ccd_blockmin's workgroup size
-constexpr int kMaxBlocks = 65536;      // 512 KiB of minima: at most 16,777,216 candidate records
+constexpr int kMaxRecs = 1 << 24;      // candidate records a call takes
+constexpr int kSlots = 32;             // handles whose calls may overlap
 constexpr int kMaxDevices = 64;
 constexpr int kReduceThreads = 1024;
 
-static __device__ __align__(256) double scratch[kMaxBlocks];
+static __device__ __align__(256) double scratch[kSlots * kMaxToiBlocks];
 
 std::mutex g_mu;
 double* g_scratch[kMaxDevices] = {};  // device address of `scratch`, per device
+unsigned g_next[kMaxDevices] = {};    // handles set up so far
 
 // one workgroup: min over the n block minima, then the reference's safety
 // scale (getImpactOfTimeHost, PdIpcGpuFunc.cu:2698-2699): t < 1 -> t * scale
@@ -52,9 +54,10 @@ __global__ void __launch_bounds__(kReduceThreads) k_toi_reduce(const double* __r
 }  // namespace
 
 // With `device` current: looks up this device's copy of `scratch` once.
-int noalloc_setup(int device) {
+int noalloc_setup(int device, int* slot) {
   if (device < 0 || device >= kMaxDevices) return fail(PDIPC_E_ARG, "device ordinal out of range");
   std::lock_guard<std::mutex> lock(g_mu);
+  *slot = g_next[device]++ % kSlots;
   if (g_scratch[device]) return PDIPC_OK;
   void* p = nullptr;
   hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
@@ -73,8 +76,7 @@ int pdipc_toi_noalloc(pdipc_handle* h, const double* x0, const double* x1, doubl
   if (rc) return rc;
   if (!x0 || !x1 || !toi) return fail(PDIPC_E_ARG, "null argument");
   const int nRecs = h->lastRecs;
-  const int nBlocks = (nRecs + kRecsPerBlock - 1) / kRecsPerBlock;
-  if (nBlocks > kMaxBlocks)
+  if (nRecs > kMaxRecs)
     return fail(PDIPC_E_CAPACITY, "pdipc_toi_noalloc: " + std::to_string(nRecs) +
                                       " candidate records exceed its limit of 16777216 (use pdipc_debug_toi)");
   double* scr;
@@ -83,6 +85,7 @@ int pdipc_toi_noalloc(pdipc_handle* h, const double* x0, const double* x1, doubl
     scr = g_scratch[h->device];
   }
   if (!scr) return fail(PDIPC_E_ARG, "pdipc_toi_noalloc: no scratch address for the handle's device");
+  scr += (size_t)(h->toiSlot % kSlots) * kMaxToiBlocks;
   hipStream_t s = stream ? (hipStream_t)stream : h->stream;
   const pdipc_params& p = h->prm;
   const int minima = launch_ccd_blockmin(h->m, nRecs, x0, x1, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
