@@ -450,7 +450,8 @@ template <class Quick, class Moves>
 __device__ __forceinline__ double share_toi(int nRecs, const int4* __restrict__ recs, const Quick& quick, const Moves& mv,
                                             const AccdParams& p) {
   __shared__ WaveQueue queue;
-  const float step = 0.9999f * (float)p.step;
+  // (without a first ACCD step no record may return 1 from it)
+  const float step = p.iters > 0 ? 0.9999f * (float)p.step : 0.f;
   double toi = 1.0;
   for_kept_records(
       nRecs, recs, queue,

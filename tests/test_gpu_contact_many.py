@@ -44,3 +44,16 @@ def test_many_records_match_the_oracle(pair, noise, offset, tol):
     assert ng == no
     assert np.abs(dg - do).max() <= tol * np.abs(do).max()
     assert np.abs(rg - ro).max() <= tol * np.abs(ro).max()
+
+
+def test_no_accd_steps(pair):
+    """Without a step of ACCD every record that passes the filter returns 0, and
+    none may be settled by its first step."""
+    sc, ref, _ = pair
+    none = dict(sc, params=dict(sc["params"], ccd_iters=0))
+    sim, x0 = pdipc.Simulator.from_scene(none), ref.x()
+    x1 = x0.copy()
+    x1[: ref.sim] += np.random.default_rng(0).normal(0, 1e-5, (ref.sim, 3))
+    print("case: no ACCD steps", flush=True)
+    assert len(sim.debug_broad_phase(x0, x1 - x0)) >= 1 << 21
+    assert sim.debug_toi(x0, x1) == 0.0
