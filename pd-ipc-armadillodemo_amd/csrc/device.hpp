@@ -256,6 +256,9 @@ void launch_copy(double* dst, const double* src, int64_t n, hipStream_t s);
 // residualOmega >= 0 (FP32-split): also the first pass of the solve's FP64
 // residual (into xa0 / cA, for the current X and D); the solve is then
 // launched with residualReady
+// pinned host points (AoS) to [3][ld] and back; clearRest: zero the rows past npts
+void launch_points_in(const double* host, int npts, int ld, bool clearRest, double* dst, hipStream_t s);
+void launch_points_out(const double* src, int npts, int ld, double* host, hipStream_t s);
 void launch_local(const DeviceMesh& m, int precision, double sigLo, double sigHi, int withCollision, hipStream_t s,
                   double residualOmega = -1.0);
 // k_tiles.hip: one launch per Chebyshev solve (launch_solve picks them while

@@ -47,9 +47,9 @@ struct pdipc_handle {
   int tileAborts = 0;  // outer iterations repeated with the streamed sweeps
   std::vector<void*> allocs;
   // host mirrors
-  void* scalHost = nullptr;  // pinned: residual, toiBits, counters[12], the tile solves' abort flag
+  void* scalHost = nullptr;  // pinned, after `stage`: residual, toiBits, counters[12], the tile solves' abort flag
   void* scalDev = nullptr;
-  std::vector<double> stage;
+  double* stage = nullptr;   // pinned: 3 * ld doubles, arrays of points on their way in or out
   pdipc_counters cnt;
   int lastRecs = 0, lastPairs = 0;
   double* trackToi = nullptr;  // per-record TOIs when track_toi_argmin is on
@@ -89,7 +89,7 @@ struct pdipc_handle {
     delete m.timer;
     pdipc::adjoint_free(adj);
     for (void* p : allocs) (void)hipFree(p);
-    if (scalHost) (void)hipHostFree(scalHost);
+    if (stage) (void)hipHostFree(stage);
     if (stream) (void)hipStreamDestroy(stream);
   }
   void drop_graphs() {

@@ -32,31 +32,26 @@ int fail(int code, const std::string& msg) {
 namespace pdipc {
 
 // AoS xyz (npoints) -> SoA [3][ld] device
-int put_soa(pdipc_handle* h, double* dst, const double* aos, int npts) {
-  h->stage.assign(3 * (size_t)h->m.ld, 0.0);
-  for (int i = 0; i < npts; i++)
-    for (int k = 0; k < 3; k++) h->stage[(size_t)k * h->m.ld + i] = aos[3 * (size_t)i + k];
-  HIPCHK(hipMemcpyAsync(dst, h->stage.data(), 3 * (size_t)h->m.ld * sizeof(double), hipMemcpyHostToDevice, h->stream));
+// Arrays of points cross the boundary through the handle's pinned buffer: the
+// host copies them straight through it and a kernel turns them into the [3][ld]
+// layout as it reads (or writes) that buffer.
+static int put_points(pdipc_handle* h, double* dst, const double* aos, int npts, bool clearRest) {
+  memcpy(h->stage, aos, 3 * (size_t)npts * sizeof(double));
+  launch_points_in(h->stage, npts, h->m.ld, clearRest, dst, h->stream);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));
   return PDIPC_OK;
 }
+int put_soa(pdipc_handle* h, double* dst, const double* aos, int npts) { return put_points(h, dst, aos, npts, true); }
 // partial overwrite: only the first npts points of each component
 int put_soa_prefix(pdipc_handle* h, double* dst, const double* aos, int npts) {
-  h->stage.assign(3 * (size_t)h->m.ld, 0.0);
-  HIPCHK(hipMemcpyAsync(h->stage.data(), dst, 3 * (size_t)h->m.ld * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  for (int i = 0; i < npts; i++)
-    for (int k = 0; k < 3; k++) h->stage[(size_t)k * h->m.ld + i] = aos[3 * (size_t)i + k];
-  HIPCHK(hipMemcpyAsync(dst, h->stage.data(), 3 * (size_t)h->m.ld * sizeof(double), hipMemcpyHostToDevice, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  return PDIPC_OK;
+  return put_points(h, dst, aos, npts, false);
 }
 int get_soa(pdipc_handle* h, const double* src, double* aos, int npts) {
-  h->stage.assign(3 * (size_t)h->m.ld, 0.0);
-  HIPCHK(hipMemcpyAsync(h->stage.data(), src, 3 * (size_t)h->m.ld * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  launch_points_out(src, npts, h->m.ld, h->stage, h->stream);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));
-  for (int i = 0; i < npts; i++)
-    for (int k = 0; k < 3; k++) aos[3 * (size_t)i + k] = h->stage[(size_t)k * h->m.ld + i];
+  memcpy(aos, h->stage, 3 * (size_t)npts * sizeof(double));
   return PDIPC_OK;
 }
 
@@ -314,7 +309,8 @@ int upload_all(pdipc_handle* h) {
   m.residual = (double*)sd;
   m.toiBits = (unsigned long long*)((char*)sd + 8);
   m.counters = (int*)((char*)sd + 16);
-  HIPCHK(hipHostMalloc(&h->scalHost, kScalarBytes, hipHostMallocDefault));
+  HIPCHK(hipHostMalloc((void**)&h->stage, V3 * sizeof(double) + kScalarBytes, hipHostMallocDefault));
+  h->scalHost = h->stage + V3;
   memset(h->scalHost, 0, kScalarBytes);
   // initial positions
   {

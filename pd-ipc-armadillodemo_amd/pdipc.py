@@ -261,7 +261,7 @@ class Simulator:
 
     # --- postRun / state
     def x(self):
-        out = np.zeros((self.total, 3))
+        out = np.empty((self.total, 3))
         _check(lib().pdipc_get_x(self.h, _dp(out), self.total))
         return out
 
@@ -272,7 +272,7 @@ class Simulator:
         _check(lib().pdipc_set_x(self.h, _dp(x), len(x)))
 
     def v(self):
-        out = np.zeros((self.sim, 3))
+        out = np.empty((self.sim, 3))
         _check(lib().pdipc_get_v(self.h, _dp(out), self.sim))
         return out
 
