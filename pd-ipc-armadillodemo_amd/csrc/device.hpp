@@ -128,7 +128,8 @@ struct DeviceMesh {
   int ld = 0;  // leading dimension of SoA vectors (>= nTotal, multiple of 64)
   // state and work vectors, SoA [3][ld] doubles
   double *X = nullptr, *Xold = nullptr, *X0 = nullptr, *Dir = nullptr, *Pre = nullptr, *Next = nullptr, *V = nullptr;
-  double *initRhs = nullptr, *sysRhs = nullptr, *firstTerm = nullptr, *colRhs = nullptr, *clothA = nullptr, *Xrest = nullptr;
+  double *initRhs = nullptr, *sysRhs = nullptr, *firstTerm = nullptr, *colRhs = nullptr, *Xrest = nullptr;
+  Row64 *xRows = nullptr, *aRows = nullptr;  // of the local step: positions and curvature vectors, a row per point
   // FP64 sweep work vectors, one Row64 per row (ld rows): three iterates and c
   Row64 *xa0 = nullptr, *xa1 = nullptr, *xa2 = nullptr, *cA = nullptr;
   // FP32-split work vectors, one float4 (x, y, z, 0) per row (ld rows): a

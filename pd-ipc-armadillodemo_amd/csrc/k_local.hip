@@ -1,9 +1,9 @@
 // The PD local step (doLocalProjection, Simulator/PD-IPC/PdIpcSimulator.cpp:1624-1681)
 // as two gathers instead of the reference's float atomics:
-//   1. k_cloth_curvature: per cloth vertex, the Laplace-Beltrami vector a_i,
-//      rescaled to the rest mean-curvature norm (PdIpcGpuFunc.cu:668-707);
-//      k_tet_project: per tet, the corotational strain projection
-//      w * U clamp(S) V^T Dm^{-T} G (PdIpcGpuFunc.cu:439-599) into 12 outputs.
+//   1. k_project: per cloth vertex, the Laplace-Beltrami vector a_i, rescaled
+//      to the rest mean-curvature norm (PdIpcGpuFunc.cu:668-707); per tet, the
+//      corotational strain projection w * U clamp(S) V^T Dm^{-T} G
+//      (PdIpcGpuFunc.cu:439-599) into 12 outputs.
 //   2. k_rhs: per point, rhs = rhs0 + tet outputs + springs + bending gathered
 //      from the 1-ring + collision rhs + position term.
 // Every point's sum is formed by a few lanes (entries dealt round-robin)
@@ -120,39 +120,50 @@ __device__ inline void svd3(const T F[9], T U[9], T sig[3], T V[9]) {
   sig[0] = s0; sig[1] = s1; sig[2] = s2;
 }
 
+struct ProjectArgs {
+  int nSim, ld, nT;
+  const double* X;
+  const int *clothOfPoint, *cOff, *cNbr;
+  const double *cLbo, *cH0;
+  Row64 *xr, *ar;
+  const int4* tets;
+  const double *dminv, *w;
+  double* tetOut;
+};
+
+// a point's row of X and, for a cloth point, of the curvature vector
 template <class T>
-__global__ void k_cloth_curvature(int nCloth, int ld, const int* __restrict__ cCenter, const int* __restrict__ cOff,
-                                  const int* __restrict__ cNbr, const double* __restrict__ cLbo,
-                                  const double* __restrict__ cH0, const double* __restrict__ X,
-                                  double* __restrict__ A) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nCloth) return;
-  int i = cCenter[c];
-  int o = cOff[c], e = cOff[c + 1];
+__device__ __forceinline__ void point_rows(const ProjectArgs& p, int i) {
+  if (i >= p.nSim) return;
+  const double* X = p.X;
+  const int ld = p.ld;
   double xi[3] = {X[i], X[ld + i], X[2 * ld + i]};
+  p.xr[i] = Row64{xi[0], xi[1], xi[2], 0.0};
+  const int c = p.clothOfPoint[i];
+  if (c < 0) return;
+  int o = p.cOff[c], e = p.cOff[c + 1];
   // a = sum_s L_s x_s = sum_{s>0} L_s (x_s - x_i) + (sum_s L_s) x_i  (the row sum is ~0)
-  double lsum = cLbo[o];
+  double lsum = p.cLbo[o];
   T a[3] = {0, 0, 0};
   for (int s = o + 1; s < e; s++) {
-    int j = cNbr[s];
-    T l = (T)cLbo[s];
-    lsum += cLbo[s];
+    int j = p.cNbr[s];
+    T l = (T)p.cLbo[s];
+    lsum += p.cLbo[s];
 #pragma unroll
     for (int k = 0; k < 3; k++) a[k] += l * (T)(X[k * ld + j] - xi[k]);
   }
   double ad[3];
-  curvature_rescale(a, lsum, xi, cH0[c], ad);
-#pragma unroll
-  for (int k = 0; k < 3; k++) A[k * ld + i] = ad[k];
+  curvature_rescale(a, lsum, xi, p.cH0[c], ad);
+  p.ar[i] = Row64{ad[0], ad[1], ad[2], 0.0};
 }
 
 template <class T>
-__global__ void k_tet_project(int nT, int ld, T sigLo, T sigHi, const int4* __restrict__ tets,
-                              const double* __restrict__ dminv, const double* __restrict__ w,
-                              const double* __restrict__ X, double* __restrict__ out) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void tet_project(const ProjectArgs& p, T sigLo, T sigHi, int t) {
+  const int nT = p.nT, ld = p.ld;
+  const double *X = p.X, *dminv = p.dminv, *w = p.w;
+  double* out = p.tetOut;
   if (t >= nT) return;
-  int4 q = tets[t];
+  int4 q = p.tets[t];
   int id[4] = {q.x, q.y, q.z, q.w};
   T Ds[9];
 #pragma unroll
@@ -204,6 +215,23 @@ __global__ void k_tet_project(int nT, int ld, T sigLo, T sigHi, const int4* __re
   }
 }
 
+// Curvature and strain projections in one launch (TETS: the first tetBlocks
+// workgroups take the tets, whose Jacobi chains are the longer ones).  Both are
+// latency-bound on scenes that leave the chip idle, and each launch costs its
+// 4 us floor: 24^3-cell block under a cloth 4.9 + 9.0 us apart, 9.0 together.
+// The rows of X and of the curvature that it writes let k_rhs gather a point as
+// one 32-byte row instead of three lines (512^2 cloth: k_rhs<float, true> 49.4
+// -> 43.8 us, of which 28 are its 147 MB of tables and results; 2.3 us more here).
+template <class T, bool TETS>
+__global__ void __launch_bounds__(kBlock) k_project(ProjectArgs p, int tetBlocks, T sigLo, T sigHi) {
+  if constexpr (TETS)
+    if ((int)blockIdx.x < tetBlocks) {
+      tet_project<T>(p, sigLo, sigHi, blockIdx.x * kBlock + threadIdx.x);
+      return;
+    }
+  point_rows<T>(p, ((int)blockIdx.x - (TETS ? tetBlocks : 0)) * kBlock + (int)threadIdx.x);
+}
+
 // RES (FP32-split): also the first pass of the solve's FP64 residual for the
 // current X and D (as k_res_a in k_solve.hip: v = M x + w D^{-1} b and the
 // pointwise part (1 - w) M x + (2 - w) w D^{-1} b - x), saving a launch.
@@ -245,7 +273,7 @@ __global__ void k_rhs(int nSim, int ld, int nT, int withCol, ResidualArgs ra, co
                       const int* __restrict__ vtOff, const int* __restrict__ vtList, const double* __restrict__ tetOut,
                       const int2* __restrict__ ringRange, const int* __restrict__ cNbr,
                       const double* __restrict__ cRest, const double* __restrict__ cStrain,
-                      const double* __restrict__ cBendIn, const double* __restrict__ A, const double* __restrict__ X,
+                      const double* __restrict__ cBendIn, const Row64* __restrict__ ar, const Row64* __restrict__ xr,
                       const double* __restrict__ colRhs, const double* __restrict__ fixK,
                       const double* __restrict__ Xrest, double* __restrict__ rhs) {
   int gt = blockIdx.x * blockDim.x + threadIdx.x;
@@ -256,7 +284,8 @@ __global__ void k_rhs(int nSim, int ld, int nT, int withCol, ResidualArgs ra, co
   const int2 ring = ringRange[ii];  // the point's cloth ring slots (empty for tet points)
   const int q0 = live ? vtOff[ii] : 0, q1 = live ? vtOff[ii + 1] : 0;
   const int r0 = RES ? ra.off[ii] : 0, r1 = RES && live ? ra.off[ii + 1] : 0;
-  const double xi[3] = {X[ii], X[ld + ii], X[2 * ld + ii]};
+  const Row64 xii = xr[ii];
+  const double xi[3] = {xii.x, xii.y, xii.z};
   double init[3] = {0, 0, 0}, col[3] = {0, 0, 0}, kf = 0.0, di = 1.0;
   if (sub == 0) {
 #pragma unroll
@@ -302,12 +331,11 @@ __global__ void k_rhs(int nSim, int ld, int nT, int withCol, ResidualArgs ra, co
       stiff[b] = in && sl > o ? cStrain[sl] : 0.0;
     }
 #pragma unroll
-    for (int b = 0; b < kRingBatch; b++)
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        xj[b][k] = X[k * ld + j[b]];
-        aj[b][k] = A[k * ld + j[b]];
-      }
+    for (int b = 0; b < kRingBatch; b++) {
+      const Row64 x = xr[j[b]], a = ar[j[b]];
+      xj[b][0] = x.x, xj[b][1] = x.y, xj[b][2] = x.z;
+      aj[b][0] = a.x, aj[b][1] = a.y, aj[b][2] = a.z;
+    }
 #pragma unroll
     for (int b = 0; b < kRingBatch; b++) {
       const int sl = s0 + b * kRhsLanes;
@@ -334,9 +362,10 @@ __global__ void k_rhs(int nSim, int ld, int nT, int withCol, ResidualArgs ra, co
         a[b] = in ? ra.val[q + b * kRhsLanes] : 0.0;
       }
 #pragma unroll
-      for (int b = 0; b < kResBatch; b++)
-#pragma unroll
-        for (int k = 0; k < 3; k++) xv[b][k] = X[k * ld + j[b]];
+      for (int b = 0; b < kResBatch; b++) {
+        const Row64 x = xr[j[b]];
+        xv[b][0] = x.x, xv[b][1] = x.y, xv[b][2] = x.z;
+      }
 #pragma unroll
       for (int b = 0; b < kResBatch; b++)
         if (q + b * kRhsLanes < r1)
@@ -377,17 +406,16 @@ __global__ void k_rhs(int nSim, int ld, int nT, int withCol, ResidualArgs ra, co
 
 template <class T>
 void local_impl(const DeviceMesh& m, T lo, T hi, int withCol, double resW, hipStream_t s) {
-  if (m.nCloth > 0)
-    launch_t(m.timer, TC_PROJECT, k_cloth_curvature<T>, dim3(grid_for(m.nCloth)), dim3(kBlock), 0, s, m.nCloth, m.ld,
-             m.cCenter, m.cOff, m.cNbr, m.cLbo, m.cH0, m.X, m.clothA);
-  if (m.nTets > 0)
-    launch_t(m.timer, TC_PROJECT, k_tet_project<T>, dim3(grid_for(m.nTets)), dim3(kBlock), 0, s, m.nTets, m.ld, lo, hi,
-             m.tetIdx, m.tetDminv, m.tetW, m.X, m.tetOut);
+  const ProjectArgs pa{m.nSim, m.ld,    m.nTets, m.X,    m.clothOfPoint, m.cOff,     m.cNbr, m.cLbo,
+                       m.cH0,  m.xRows, m.aRows, m.tetIdx, m.tetDminv,   m.tetW, m.tetOut};
+  const int tetBlocks = grid_for(m.nTets);
+  launch_t(m.timer, TC_PROJECT, m.nTets > 0 ? k_project<T, true> : k_project<T, false>,
+           dim3(grid_for(m.nSim) + tetBlocks), dim3(kBlock), 0, s, pa, tetBlocks, lo, hi);
   const ResidualArgs ra{resW, m.r1Off, m.r1Col, m.r1Val, m.sysDiag, m.xa0, m.cA};
   const dim3 grid(grid_for((int64_t)m.nSim * kRhsLanes));
   launch_t(m.timer, TC_RHS, resW >= 0.0 ? k_rhs<T, true> : k_rhs<T, false>, grid, dim3(kBlock), 0, s, m.nSim, m.ld,
            m.nTets, withCol, ra, m.initRhs, m.vtOff, m.vtList, m.tetOut, m.ringRange, m.cNbr, m.cRest, m.cStrain,
-           m.cBendIn, m.clothA, m.X, m.colRhs, m.fixK, m.Xrest, m.sysRhs);
+           m.cBendIn, m.aRows, m.xRows, m.colRhs, m.fixK, m.Xrest, m.sysRhs);
 }
 
 // ---- adjoint of the local step (FP64), evaluated at the recorded x

@@ -164,11 +164,12 @@ int upload_all(pdipc_handle* h) {
 #define UP(field, vec) if ((rc = h->upload(&m.field, vec))) return rc
 #define AL(field, n) if ((rc = h->alloc(&m.field, n))) return rc
   AL(X, V3); AL(Xold, V3); AL(X0, V3); AL(Dir, V3); AL(Pre, V3); AL(Next, V3); AL(V, V3);
-  AL(initRhs, V3); AL(sysRhs, V3); AL(firstTerm, V3); AL(colRhs, V3); AL(clothA, V3); AL(Xrest, V3);
+  AL(initRhs, V3); AL(sysRhs, V3); AL(firstTerm, V3); AL(colRhs, V3); AL(Xrest, V3);
+  AL(xRows, m.ld); AL(aRows, m.ld);
   AL(dPre, m.ld); AL(dCur, m.ld); AL(dNext, m.ld); AL(r0, m.ld);
   AL(xa0, m.ld); AL(xa1, m.ld); AL(xa2, m.ld); AL(cA, m.ld);
   for (Row64* p : {m.xa0, m.xa1, m.xa2, m.cA}) HIPCHK(hipMemsetAsync(p, 0, m.ld * sizeof(Row64), h->stream));
-  for (double* p : {m.X, m.Xold, m.X0, m.Dir, m.Pre, m.Next, m.V, m.initRhs, m.sysRhs, m.firstTerm, m.colRhs, m.clothA,
+  for (double* p : {m.X, m.Xold, m.X0, m.Dir, m.Pre, m.Next, m.V, m.initRhs, m.sysRhs, m.firstTerm, m.colRhs,
                     m.Xrest})
     HIPCHK(hipMemsetAsync(p, 0, V3 * sizeof(double), h->stream));
   for (float4* p : {m.dPre, m.dCur, m.dNext, m.r0}) HIPCHK(hipMemsetAsync(p, 0, m.ld * sizeof(float4), h->stream));
