@@ -241,6 +241,108 @@ __global__ void k_radix_scatter(int n, int shift, const uint32_t* __restrict__ k
   }
 }
 
+// The sort of up to kSortSmall codes, and their keys, in one workgroup: there
+// the launches of the sort above (three per digit, four digits, then the keys)
+// cost their floor, about 72 us whatever the size.  One workgroup: 24 us for
+// 4,124 patches, 40 for 9,244, 61 for 16,157, and its LDS ends soon after.
+// The codes live in LDS, an item's 16-bit patch beside it.  Per digit a wave takes
+// its run of them to registers and counts its digits, the counts are scanned
+// (digit by digit, wave by wave), and the wave puts its items in order at their
+// places, equal digits ranked by ballots (what bounds it): the same stable order.
+constexpr int kSortThreads = 1024, kSortWaves = kSortThreads / kWave, kSortRounds = 16;
+constexpr int kSortSmall = kSortThreads * kSortRounds;
+constexpr size_t sort_small_lds(int rounds) { return (size_t)kSortThreads * rounds * 6 + kSortWaves * 256 * 4; }
+
+__global__ void __launch_bounds__(kSortThreads) k_sort_small(int P, uint32_t* __restrict__ code,
+                                                             int* __restrict__ idx, uint64_t* __restrict__ keys) {
+  extern __shared__ __attribute__((aligned(16))) char sortLds[];
+  __shared__ int digitBase[256], waveSum[256 / kWave];
+  const int t = threadIdx.x, lane = t % kWave, w = t / kWave;
+  const int rounds = (P + kSortThreads - 1) / kSortThreads;  // at most kSortRounds
+  int(*cnt)[256] = (int(*)[256])sortLds;
+  uint32_t* k = (uint32_t*)(sortLds + kSortWaves * 256 * 4);
+  uint16_t* v = (uint16_t*)(k + kSortThreads * rounds);
+  const int base = w * rounds * kWave + lane;
+  const unsigned long long lt = (1ull << lane) - 1ull;
+  uint32_t key[kSortRounds];
+  int val[kSortRounds];
+#pragma unroll
+  for (int r = 0; r < kSortRounds; r++) {
+    const int i = base + r * kWave;
+    val[r] = i;
+    key[r] = r < rounds && i < P ? code[i] : 0u;
+  }
+  for (int shift = 0; shift < 30; shift += 8) {
+#pragma unroll
+    for (int q = 0; q < kSortWaves * 256 / kSortThreads; q++) (&cnt[0][0])[t + q * kSortThreads] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRounds; r++)
+      if (r < rounds && base + r * kWave < P) atomicAdd(&cnt[w][(key[r] >> shift) & 255u], 1);
+    __syncthreads();
+    int sum = 0, inc = 0;
+    if (t < 256) {  // (whole waves)
+#pragma unroll
+      for (int q = 0; q < kSortWaves; q++) {
+        const int c = cnt[q][t];
+        cnt[q][t] = sum;
+        sum += c;
+      }
+      inc = sum;
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        const int y = __shfl_up(inc, o, kWave);
+        if (lane >= o) inc += y;
+      }
+      if (lane == kWave - 1) waveSum[w] = inc;
+    }
+    __syncthreads();
+    if (t < 256) {
+      int b = inc - sum;
+      for (int q = 0; q < w; q++) b += waveSum[q];
+      digitBase[t] = b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRounds; r++) {
+      if (r >= rounds) break;
+      const bool in = base + r * kWave < P;
+      const int d = (int)((key[r] >> shift) & 255u);
+      unsigned long long peers = __ballot(in);
+#pragma unroll
+      for (int b = 0; b < 8; b++) {
+        const unsigned long long bb = __ballot((d >> b) & 1);
+        peers &= ((d >> b) & 1) ? bb : ~bb;
+      }
+      if (in) {
+        const int pos = digitBase[d] + cnt[w][d] + (int)__popcll(peers & lt);
+        k[pos] = key[r];
+        v[pos] = (uint16_t)val[r];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the counts are the wave's own
+      if (in && lane == __ffsll((long long)peers) - 1) cnt[w][d] += (int)__popcll(peers);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRounds; r++) {
+      const int i = base + r * kWave;
+      if (r < rounds && i < P) {
+        key[r] = k[i];
+        val[r] = v[i];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kSortRounds; r++) {
+    const int i = base + r * kWave;
+    if (r >= rounds || i >= P) continue;
+    code[i] = key[r];
+    idx[i] = val[r];
+    keys[i] = ((uint64_t)key[r] << 32) | (uint32_t)val[r];
+  }
+}
+
 // ---------------- exclusive scan of int counts ----------------
 __device__ inline int block_exclusive_scan(int v, int* sh, int* total) {
   // inclusive scan within waves via shuffles, then across waves
@@ -971,15 +1073,22 @@ void launch_patch_boxes(const DeviceMesh& m, const double* x, const double* dx, 
                      m.ld, m.pfOff, m.pfList, m.bFaces, x, dx, m.nSim, inflation, m.patchBox);
 }
 
-void launch_lbvh(DeviceMesh& m, hipStream_t s) {
-  int P = m.nPatches;
-  if (P <= 0) return;
-  int nPart = std::min(256, (P + kBlock - 1) / kBlock);
-  hipLaunchKernelGGL(k_scene_partial, dim3(nPart), dim3(kBlock), 0, s, P, m.patchBox, m.sceneBoxPart);
-  hipLaunchKernelGGL(k_scene_final, dim3(1), dim3(kBlock), 0, s, nPart, m.sceneBoxPart, m.sceneBox);
-  hipLaunchKernelGGL(k_morton, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, m.sceneBox, m.patchBox,
-                     m.mortonA, m.idxA);
-  int nb = (P + kRadixTile - 1) / kRadixTile;
+// the one-workgroup sort, when the patches are few enough for it
+static bool sort_small(const DeviceMesh& m, hipStream_t s) {
+  const int P = m.nPatches;
+  if (P > kSortSmall) return false;
+  const size_t lds = sort_small_lds((P + kSortThreads - 1) / kSortThreads);
+  if (lds > (60 << 10) && hipFuncSetAttribute((const void*)k_sort_small, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              (int)lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kSortThreads), lds, s, P, m.mortonA, m.idxA, m.keys);
+  return true;
+}
+
+static void sort_patches(const DeviceMesh& m, hipStream_t s) {
+  const int P = m.nPatches, nb = (P + kRadixTile - 1) / kRadixTile;
   uint32_t *kin = m.mortonA, *kout = m.mortonB;
   int *iin = m.idxA, *iout = m.idxB;
   for (int shift = 0; shift < 30; shift += 8) {
@@ -989,12 +1098,23 @@ void launch_lbvh(DeviceMesh& m, hipStream_t s) {
     std::swap(kin, kout);
     std::swap(iin, iout);
   }
-  // 4 passes: the sorted data is back in the A buffers
   hipLaunchKernelGGL(k_make_keys, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, kin, iin, m.keys);
+}
+
+void launch_lbvh(DeviceMesh& m, hipStream_t s) {
+  int P = m.nPatches;
+  if (P <= 0) return;
+  int nPart = std::min(256, (P + kBlock - 1) / kBlock);
+  hipLaunchKernelGGL(k_scene_partial, dim3(nPart), dim3(kBlock), 0, s, P, m.patchBox, m.sceneBoxPart);
+  hipLaunchKernelGGL(k_scene_final, dim3(1), dim3(kBlock), 0, s, nPart, m.sceneBoxPart, m.sceneBox);
+  hipLaunchKernelGGL(k_morton, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, m.sceneBox, m.patchBox,
+                     m.mortonA, m.idxA);
+  // (the sorted patches end in idxA on either path)
+  if (!sort_small(m, s)) sort_patches(m, s);
   if (P > 1)
     hipLaunchKernelGGL(k_karras, dim3((P - 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, m.keys, m.nodeLeft,
                        m.nodeRight, m.nodeParent, m.nodeRange);
-  hipLaunchKernelGGL(k_table_level0, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, iin, m.patchBox,
+  hipLaunchKernelGGL(k_table_level0, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, m.idxA, m.patchBox,
                      m.nodeTable);
   int top = 0;  // the highest level: 2^top <= P
   while ((2 << top) <= P) top++;
@@ -1003,7 +1123,7 @@ void launch_lbvh(DeviceMesh& m, hipStream_t s) {
     hipLaunchKernelGGL(k_table_levels, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, j,
                        std::min(per, top - j + 1), m.nodeTable);
   hipLaunchKernelGGL(k_node_boxes, dim3((2 * P - 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, m.nodeRange,
-                     m.nodeTable, m.nodeLeft, m.nodeRight, m.nodeParent, iin, m.nodes);
+                     m.nodeTable, m.nodeLeft, m.nodeRight, m.nodeParent, m.idxA, m.nodes);
 }
 
 int traverse_top_waves(int P) { return ((P + kBlock - 1) / kBlock) * (kBlock / kWave); }
