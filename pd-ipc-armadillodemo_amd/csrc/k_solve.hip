@@ -189,6 +189,11 @@ __global__ void __launch_bounds__(kBlock) k_res_a(int n, int ld, double w, const
   pt[row] = Row64{pp[0], pp[1], pp[2], 0.0};
 }
 
+// The second residual pass: r0 = pt + (w / D) R1 v, and the streamed sweeps' first
+// two iterates where dpreF is given.  A lane's R1 entries are fetched six at a
+// time (a cloth row's 19 over 4 lanes in one batch), since on small scenes the
+// round trips bound it and on large ones the bytes: @RESB@.
+constexpr int kResRowBatch = 6;
 template <int G>
 __global__ void __launch_bounds__(kBlock) k_res_b(int n, double w, const int* __restrict__ off,
                                                   const int* __restrict__ col, const double* __restrict__ val,
@@ -202,19 +207,33 @@ __global__ void __launch_bounds__(kBlock) k_res_b(int n, double w, const int* __
   const double dr = D[rr];
   const Row64 p = pt[rr];
   double sv[3] = {0.0, 0.0, 0.0};
-  if (row < n)
-    for (int q = off[row] + sub; q < off[row + 1]; q += G) {
-      double a = val[q];
-      Row64 vj = v[col[q]];
-      sv[0] += a * vj.x;
-      sv[1] += a * vj.y;
-      sv[2] += a * vj.z;
+  const int q0 = off[rr], q1 = row < n ? off[rr + 1] : q0;
+  for (int q = q0 + sub; q < q1; q += kResRowBatch * G) {
+    int j[kResRowBatch];
+    double a[kResRowBatch];
+    Row64 vj[kResRowBatch];
+#pragma unroll
+    for (int b = 0; b < kResRowBatch; b++) {
+      const bool in = q + b * G < q1;
+      j[b] = in ? col[q + b * G] : rr;
+      a[b] = in ? val[q + b * G] : 0.0;
     }
+#pragma unroll
+    for (int b = 0; b < kResRowBatch; b++) vj[b] = v[j[b]];
+#pragma unroll
+    for (int b = 0; b < kResRowBatch; b++)
+      if (q + b * G < q1) {
+        sv[0] += a[b] * vj[b].x;
+        sv[1] += a[b] * vj[b].y;
+        sv[2] += a[b] * vj[b].z;
+      }
+  }
   group_reduce<G>(sv);
   if (sub != 0 || row >= n) return;
   double f = w / dr;
   float4 rv = make_float4((float)(p.x + f * sv[0]), (float)(p.y + f * sv[1]), (float)(p.z + f * sv[2]), 0.0f);
   r0F[row] = rv;
+  if (!dpreF) return;
   dpreF[row] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   dnextF[row] = rv;
 }
@@ -1016,13 +1035,12 @@ void solve_impl(const DeviceMesh& m, double w, double rho, int iters, int precis
   if (!residualReady)  // else the local step's k_rhs wrote v and pt
     launch_t(m.timer, TC_FIRST, k_res_a<GR>, dim3(gridR), dim3(kBlock), 0, s, m.nSim, m.ld, w, m.r1Off, m.r1Col,
              m.r1Val, m.sysDiag, m.X, m.sysRhs, m.xa0, m.cA);
+  const bool tiles = G == 8 && m.tile.use(1);
   launch_t(m.timer, TC_FIRST, k_res_b<GR>, dim3(gridR), dim3(kBlock), 0, s, m.nSim, w, m.r1Off, m.r1Col, m.r1Val,
-           m.sysDiag, m.xa0, m.cA, pre, cur, m.r0);
-  if constexpr (G == 8) {
-    if (m.tile.use(1)) {
-      launch_tile_solve32(m, iters, parity, s);
-      return;
-    }
+           m.sysDiag, m.xa0, m.cA, tiles ? nullptr : pre, cur, m.r0);
+  if (tiles) {
+    launch_tile_solve32(m, iters, parity, s);
+    return;
   }
   if (iters <= 1) {
     hipLaunchKernelGGL(k_apply_delta, dim3((m.nSim + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nSim, m.ld, cur,
