@@ -387,8 +387,8 @@ int taped_step(pdipc_handle* h, StepTape& st) {
       if ((rc = run_captured(h, A->fwdGraph[m.tile.use(PDIPC_FP64) ? 1 : 0][ot.withCol], [&]() { enqueue_taped_lg(h, ot.withCol); }))) return rc;
       if ((rc = A->tape.alloc(A->lay.bytes(), (void**)&ot.blob))) return rc;
       HIPCHK(hipMemcpyAsync(ot.blob, A->stage, A->lay.bytes(), hipMemcpyDeviceToDevice, s));
-      launch_direction(m, s);
       if (outer == 0) {
+        launch_direction(m, s);
         if ((rc = broad_phase(h, m.Xold, m.Dir))) return rc;
         st.nRecs = h->lastRecs;
         if ((rc = A->tape.alloc((size_t)std::max(1, st.nRecs) * sizeof(int4), (void**)&st.recs))) return rc;
@@ -403,7 +403,7 @@ int taped_step(pdipc_handle* h, StepTape& st) {
           if ((rc = dalloc(A, &A->recToi, (size_t)A->recToiCap))) return rc;
         }
       }
-      HIPCHK(hipMemsetAsync(m.counters + 4, 0x7f, sizeof(int), s));  // (launch_direction reset the TOI minimum)
+      HIPCHK(hipMemsetAsync(m.counters + 4, 0x7f, sizeof(int), s));  // (launch_diag reset the TOI minimum)
       launch_ccd_records(m, m.recs, h->lastRecs, m.Xold, m.X, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
                          p.touch_policy, A->recToi, m.counters + 4, s);
       launch_clamp_residual(m, p.toi_scale, s);

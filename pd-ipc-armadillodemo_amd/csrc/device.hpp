@@ -249,7 +249,9 @@ struct DeviceMesh {
 void launch_predict(const DeviceMesh& m, double dt, hipStream_t s);
 void launch_diag(const DeviceMesh& m, int withCollision, hipStream_t s);
 void launch_direction(const DeviceMesh& m, hipStream_t s);  // also sets the TOI minimum to 1
+// leaves partial sums of the residual; launch_collision adds them up
 void launch_clamp_residual(const DeviceMesh& m, double toiScale, hipStream_t s);
+int residual_partials(const DeviceMesh& m);
 void launch_velocity(const DeviceMesh& m, double dt, hipStream_t s);
 void launch_zero(double* p, int64_t n, hipStream_t s);
 void launch_copy(double* dst, const double* src, int64_t n, hipStream_t s);

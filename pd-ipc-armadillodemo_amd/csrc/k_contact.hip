@@ -13,6 +13,7 @@
 
 #include "device.hpp"
 #include "dual.hpp"
+#include "local_ops.hpp"
 
 namespace pdipc {
 namespace {
@@ -677,9 +678,16 @@ __global__ void __launch_bounds__(kBlock) k_col_terms_few(int nRecs, ColTerms c)
 
 // zeroes the pass's counters (counters[2]: active records, counters[5]: list
 // overflow) and the per-point counts and cursors: one launch instead of four
-// memsets
-__global__ void k_col_clear(int nSim, int* __restrict__ counters, int* __restrict__ ptCount,
-                            int* __restrict__ ptCursor) {
+// memsets.  The last workgroup adds up the residual's partial sums that the
+// clamp before it left.
+__global__ void __launch_bounds__(kBlock) k_col_clear(int nSim, int* __restrict__ counters, int* __restrict__ ptCount,
+                                                      int* __restrict__ ptCursor, int nPart,
+                                                      const double* __restrict__ partials,
+                                                      double* __restrict__ residual) {
+  if (blockIdx.x == gridDim.x - 1) {
+    sum_partials<kBlock>(nPart, partials, residual);
+    return;
+  }
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     counters[2] = 0;
@@ -994,8 +1002,8 @@ void launch_adj_ccd(const DeviceMesh& m, const int4* recs, int argmin, const dou
 }
 
 int launch_collision(DeviceMesh& m, int nRecs, double dhat, double kappa, double dt, hipStream_t s) {
-  hipLaunchKernelGGL(k_col_clear, dim3((m.nSim + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nSim, m.counters,
-                     m.ptCount, m.ptCursor);
+  hipLaunchKernelGGL(k_col_clear, dim3((m.nSim + 1 + kBlock - 1) / kBlock + 1), dim3(kBlock), 0, s, m.nSim, m.counters,
+                     m.ptCount, m.ptCursor, residual_partials(m), m.partials, m.residual);
   const ColTerms c{m.ld,    m.nSim, m.actCap, m.recs, m.X,       m.colMass, dhat,
                    kappa, dt,     m.actRec, m.actW, m.actT, m.ptCount, m.counters};
   if (nRecs >= kManyRecs) {

@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "device.hpp"
+#include "local_ops.hpp"
 
 namespace pdipc {
 
@@ -53,10 +54,14 @@ void launch_predict(const DeviceMesh& m, double dt, hipStream_t s) {
 // LocalGlobalIteration diagonal (PdIpcSimulator.cpp:1557-1560): D = elastic + inertial
 // (+ collision).  Also records which rows changed since the last operator update
 // (or were marked stale by the host), so the M^2 update can skip untouched rows.
+// Thread 0 also resets the device-resident TOI minimum to 1 for the CCD pass of
+// this outer iteration.
 __global__ void k_diag(int n, const double* __restrict__ e, const double* __restrict__ in,
                        const double* __restrict__ col, int withCol, double* __restrict__ D,
-                       uint8_t* __restrict__ stale, uint8_t* __restrict__ changed) {
+                       uint8_t* __restrict__ stale, uint8_t* __restrict__ changed,
+                       unsigned long long* __restrict__ toiBits) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *toiBits = (unsigned long long)__double_as_longlong(1.0);
   if (i >= n) return;
   double d = e[i] + in[i];
   if (withCol) d += col[i];
@@ -68,16 +73,13 @@ __global__ void k_diag(int n, const double* __restrict__ e, const double* __rest
 
 void launch_diag(const DeviceMesh& m, int withCollision, hipStream_t s) {
   hipLaunchKernelGGL(k_diag, dim3(grid_for(m.nSim)), dim3(kBlock), 0, s, m.nSim, m.elasticDiag, m.inertialDiag,
-                     m.colDiag, withCollision, m.sysDiag, m.dStale, m.dChanged);
+                     m.colDiag, withCollision, m.sysDiag, m.dStale, m.dChanged, m.toiBits);
 }
 
-// computeDirectionKernel (PdIpcGpuFunc.cu:185-200); thread 0 also resets the
-// device-resident TOI minimum to 1 for the CCD pass that follows (a launch
-// fewer per outer iteration)
+// computeDirectionKernel (PdIpcGpuFunc.cu:185-200), for the broad phase
 __global__ void k_direction(int n, int ld, const double* __restrict__ X, const double* __restrict__ Xold,
-                            double* __restrict__ D, unsigned long long* __restrict__ toiBits) {
+                            double* __restrict__ D) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) *toiBits = (unsigned long long)__double_as_longlong(1.0);
   if (i >= n) return;
 #pragma unroll
   for (int c = 0; c < 3; c++) D[c * ld + i] = X[c * ld + i] - Xold[c * ld + i];
@@ -85,15 +87,18 @@ __global__ void k_direction(int n, int ld, const double* __restrict__ X, const d
 
 void launch_direction(const DeviceMesh& m, hipStream_t s) {
   hipLaunchKernelGGL(k_direction, dim3(grid_for(std::max(1, m.nSim))), dim3(kBlock), 0, s, m.nSim, m.ld, m.X, m.Xold,
-                     m.Dir, m.toiBits);
+                     m.Dir);
 }
 
 // clampDirectionKernel (PdIpcGpuFunc.cu:222-238) reading the device-resident TOI,
-// fused with the block partial sums of |d|^2 (the residual of PdIpcSimulator.cpp:1774).
+// fused with the block partial sums of |d|^2 (the residual of PdIpcSimulator.cpp:1774),
+// which the barrier pass's first kernel adds up: a launch of 4.5 us less per outer
+// iteration; and it forms d itself, so only the first iteration, whose broad phase
+// reads d, runs k_direction (4.8 us).
 // The TOI minimum over all records, scaled by toi_scale when below 1, equals the
 // reference's per-block scaling followed by the global minimum (the scaling is monotone).
 __global__ void k_clamp_residual(int n, int ld, double toiScale, const unsigned long long* __restrict__ toiBits,
-                                 const double* __restrict__ Xold, const double* __restrict__ D, double* __restrict__ X,
+                                 const double* __restrict__ Xold, double* __restrict__ X,
                                  double* __restrict__ partials) {
   __shared__ double red[kBlock / kWave];
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -103,8 +108,8 @@ __global__ void k_clamp_residual(int n, int ld, double toiScale, const unsigned 
   if (i < n) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      double d = D[c * ld + i];
-      X[c * ld + i] = Xold[c * ld + i] + toi * d;
+      const double xo = Xold[c * ld + i], d = X[c * ld + i] - xo;
+      X[c * ld + i] = xo + toi * d;
       acc += d * d;
     }
   }
@@ -120,26 +125,15 @@ __global__ void k_clamp_residual(int n, int ld, double toiScale, const unsigned 
 }
 
 __global__ void k_sum_partials(int n, const double* __restrict__ partials, double* __restrict__ out) {
-  __shared__ double red[kBlock / kWave];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) acc += partials[i];
-  for (int off = kWave / 2; off > 0; off >>= 1) acc += __shfl_down(acc, off, kWave);
-  int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
-  if (lane == 0) red[wv] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < kBlock / kWave; w++) t += red[w];
-    *out = t;
-  }
+  sum_partials<kBlock>(n, partials, out);
 }
 
 void launch_clamp_residual(const DeviceMesh& m, double toiScale, hipStream_t s) {
   int g = grid_for(m.nSim);
-  hipLaunchKernelGGL(k_clamp_residual, dim3(g), dim3(kBlock), 0, s, m.nSim, m.ld, toiScale, m.toiBits, m.Xold, m.Dir,
+  hipLaunchKernelGGL(k_clamp_residual, dim3(g), dim3(kBlock), 0, s, m.nSim, m.ld, toiScale, m.toiBits, m.Xold,
                      m.X, m.partials);
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kBlock), 0, s, g, m.partials, m.residual);
 }
+int residual_partials(const DeviceMesh& m) { return grid_for(m.nSim); }
 
 // updateVelocityKernel (PdIpcGpuFunc.cu:262-280) with damping 1 - dt (PdIpcSimulator.cpp:1789)
 __global__ void k_velocity(int n, int ld, double invt, const double* __restrict__ X, const double* __restrict__ X0,

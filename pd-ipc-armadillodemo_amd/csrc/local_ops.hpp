@@ -59,4 +59,21 @@ __device__ __forceinline__ void add_spring(const T (&d)[3], double stiff, double
   for (int k = 0; k < 3; k++) sp[k] = fmad(rc, d[k], sp[k]);
 }
 
+// One workgroup of BT threads: the sum of n partials in a fixed order
+template <int BT>
+__device__ __forceinline__ void sum_partials(int n, const double* __restrict__ partials, double* __restrict__ out) {
+  constexpr int kW = 64;
+  __shared__ double red[BT / kW];
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < n; i += BT) acc += partials[i];
+  for (int off = kW / 2; off > 0; off >>= 1) acc += __shfl_down(acc, off, kW);
+  if (threadIdx.x % kW == 0) red[threadIdx.x / kW] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < BT / kW; w++) t += red[w];
+    *out = t;
+  }
+}
+
 }  // namespace pdipc

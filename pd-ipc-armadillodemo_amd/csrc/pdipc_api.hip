@@ -495,15 +495,15 @@ int outer_iteration(pdipc_handle* h, int outer, bool activeCol, bool* tracked) {
   hipStream_t s = h->stream;
   int rc;
   if ((rc = local_global(h, activeCol ? 1 : 0))) return rc;
-  launch_direction(m, s);
   if (outer == 0) {
+    launch_direction(m, s);
     hipEvent_t b0 = nullptr, b1 = nullptr;
     if (m.timer && m.timer->take(TC_BROAD, &b0, &b1)) HIPCHK(hipEventRecord(b0, s));
     rc = broad_phase(h, m.Xold, m.Dir);
     if (b1) HIPCHK(hipEventRecord(b1, s));
     if (rc) return rc;
   }
-  const bool track = p.track_toi_argmin && h->lastRecs > 0;  // (launch_direction reset the TOI minimum)
+  const bool track = p.track_toi_argmin && h->lastRecs > 0;  // (launch_diag reset the TOI minimum)
   *tracked = track;
   if (track) {  // per-record TOIs, then the first record attaining the minimum
     if (h->trackCap < h->lastRecs) {
