@@ -1037,28 +1037,28 @@ void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, S
     for (int s = hs.cOff[c]; s < hs.cOff[c + 1]; s++) fn(s, hs.cNbr[s]);
   };
   parallel_ranges(T.nTiles, nt, [&](int64_t t0, int64_t t1, int) {
+    std::vector<int> inH(n, -1), inG(n, -1);  // the last tile that listed the point
     for (int t = (int)t0; t < (int)t1; t++) {
       std::vector<int>&H = halo[t], &G = ringHalo[t];
-      auto read = [&](int c) {
-        if (owner[c] != t) H.push_back(c);
+      auto list = [&](int c, std::vector<int>& in, std::vector<int>& to) {
+        if (owner[c] == t || in[c] == t) return;
+        in[c] = t;
+        to.push_back(c);
       };
+      auto read = [&](int c) { list(c, inH, H); };
       for (int r = 0; r < R; r++)
         if (const int row = T.rows[(size_t)t * R + r]; row >= 0) {
           for (int q = hs.m2Off[row]; q < hs.m2Off[row + 1]; q++) read(hs.m2Col[q]);
           if (!cloths) continue;
           for (int q = hs.r1Off[row]; q < hs.r1Off[row + 1]; q++) read(hs.r1Col[q]);
-          ring_of(row, [&](int, int c) {
-            if (owner[c] != t) G.push_back(c);
-          });
+          ring_of(row, [&](int, int c) { list(c, inG, G); });
         }
       std::sort(G.begin(), G.end());
-      G.erase(std::unique(G.begin(), G.end()), G.end());
       for (int c : G) {
         read(c);
         ring_of(c, [&](int, int b) { read(b); });
       }
       std::sort(H.begin(), H.end());
-      H.erase(std::unique(H.begin(), H.end()), H.end());
     }
   }, 8);
   // The exchange needs a symmetric neighbour relation.  M^2's pattern is

@@ -192,7 +192,9 @@ __global__ void __launch_bounds__(kBlock) k_res_a(int n, int ld, double w, const
 // The second residual pass: r0 = pt + (w / D) R1 v, and the streamed sweeps' first
 // two iterates where dpreF is given.  A lane's R1 entries are fetched six at a
 // time (a cloth row's 19 over 4 lanes in one batch), since on small scenes the
-// round trips bound it and on large ones the bytes: @RESB@.
+// round trips bound it and on large ones the bytes.  One entry at a
+// time, with the first iterates written for the tile solves too, against now: 24^3-cell
+// tet block 5.3 -> 4.8 us, 512^2 cloth 22.3 -> 18.6 (about 80 MB).
 constexpr int kResRowBatch = 6;
 template <int G>
 __global__ void __launch_bounds__(kBlock) k_res_b(int n, double w, const int* __restrict__ off,
