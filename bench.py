@@ -569,10 +569,23 @@ def main():
     step_bytes, spmv_bytes = algorithmic_step_bytes(c, slots, outer32, recs32, 4, scene["params"]["lg_iters"],
                                                scene["params"]["cheb_iters"])
     sweep = kt["fp32_split"]["sweep_fp32"]
-    ach = spmv_bytes / (sweep["mean_us"] * 1e-6) / 1e9
     staging = sims["fp32_split"].sweep_staging()
     kname, slot_bytes = SWEEP32_KERNELS[staging]
+    bytes_formula = "8 B per M^2 entry (FP32 value + int32 column) + 4 vectors x 3N x 4 B"
     stored = c["nnz_r2"] * slot_bytes + 3 * c["sim_points"] * 4.0 * 4
+    bytes64 = 8 * c["nnz_r2"] + 4 * 3 * c["sim_points"] * 8
+    # a tile solve reads the matrix once for all its sweeps; times are per sweep
+    sweeps = scene["params"]["cheb_iters"] - 1
+    tiles = sims["fp32_split"].tile_solves()
+    if tiles["fp32"] and sweeps > 0:
+        kname = "k_tile_solve32 (a whole FP32 solve per launch, M^2 in registers, iterates exchanged), per sweep"
+        slot_bytes = 6.0
+        spmv_bytes = stored = (6.0 * c["sell_entries"] + 64.0 * c["sim_points"]) / sweeps
+        bytes_formula = ("per solve 6 B per stored M^2 entry (FP32 value + 16-bit LDS index) and 64 B per point (r0, X "
+                         "in and out), over its sweeps; bound by the exchange between tiles, not by these bytes")
+    if tiles["fp64"]:
+        bytes64 = (10.0 * c["sell_entries"] + 96.0 * c["sim_points"]) / (sweeps + 1)
+    ach = spmv_bytes / (sweep["mean_us"] * 1e-6) / 1e9
     matrix_bytes = c["sell_entries"] * slot_bytes
     out = {
         "metric": METRIC,
@@ -612,12 +625,12 @@ def main():
         },
         "roofline": {
             "kernel": kname,
-            "bound": "hbm",
+            "bound": "latency" if tiles["fp32"] else "hbm",
             "achieved": ach,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": ach / HBM_PEAK_GBS,
-            "traffic": None if workload else
+            "traffic": None if workload or tiles["fp32"] else
                        SWEEP32_TRAFFIC_BYTES.get((args.n, args.subdiv, args.sell_lanes, staging)),
             "traffic_source": "profiles/k_sweep_config1_hbm_traffic.md: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE "
                               "per launch, scaled by a 1 GiB copy; a recorded constant, not measured in this run",
@@ -625,7 +638,7 @@ def main():
             "avg_us_source": f"mean of {sweep['launches']} in-step launches, HIP events on each launch "
                              "(pdipc_kernel_timing, the timed window with direct launches)",
             "bytes_per_launch": spmv_bytes,
-            "bytes_formula": "8 B per M^2 entry (FP32 value + int32 column) + 4 vectors x 3N x 4 B",
+            "bytes_formula": bytes_formula,
             "bytes_stored_format": stored,
             "frac_stored_format": stored / (sweep["mean_us"] * 1e-6) / 1e9 / HBM_PEAK_GBS,
             "mall_resident": matrix_bytes < 256e6,
@@ -637,7 +650,7 @@ def main():
                           f"{matrix_bytes / 1e6:.1f} MB) exceeds the 256 MB Infinity Cache: every sweep streams it "
                           "from HBM"),
             "fp64_sweep": {"avg_us": kt["fp64"]["sweep_fp64"]["mean_us"],
-                           "achieved": (8 * c["nnz_r2"] + 4 * 3 * c["sim_points"] * 8)
+                           "achieved": bytes64
                            / (kt["fp64"]["sweep_fp64"]["mean_us"] * 1e-6) / 1e9},
             "replay": replay,
         },
