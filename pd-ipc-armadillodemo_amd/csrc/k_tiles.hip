@@ -884,7 +884,8 @@ __global__ void __launch_bounds__(BT) k_tile_loop(TileShape a, TileLoop g, const
         }
       }
       if constexpr (F32) {
-        if (!st.exchange(a, j, vv, 2, &flag, t0, Vxy, Vz)) return;
+        // (publication j - 2: a correction of two words, or with one sweep the last pass's v)
+        if (!st.exchange(a, j, vv, a.iters == 1 ? 3 : 2, &flag, t0, Vxy, Vz)) return;
         j++;
 #pragma unroll
         for (int k = 0; k < 3; k++) r[k] = pt[k];

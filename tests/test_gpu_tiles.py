@@ -133,3 +133,21 @@ def test_handles_stepping_from_several_threads():
     for p, q in zip(alone, together):
         assert np.array_equal(p[0], q[0]) and np.array_equal(p[1], q[1])
         assert p[2] == 0 and q[2] == 0
+
+
+# Few sweeps leave few publications between two of the same slot: whole steps,
+# whose passes follow each other in one launch (cloths) or in alternating sets.
+# 32 and 88 rows per tile, the latter with four threads per row; several models.
+@pytest.mark.parametrize("iters", [1, 2, 3])
+@pytest.mark.parametrize("which", ["20", "150", "layers"])
+def test_fp32_steps_of_few_sweeps_match_streamed_sweeps(which, iters):
+    sc = scenes.config4(n=40, side=80.0 / 1024) if which == "layers" else _cloth(int(which))
+    sc["params"]["cheb_iters"] = iters
+    print(f"case: {which}, FP32 steps of {iters} sweeps", flush=True)
+    a, b = (pdipc.Simulator.from_scene(sc, precision=pdipc.FP32_SPLIT, sell_stage=st) for st in (1, 2))
+    assert a.tile_solves()["fp32"] == 1 and a.tile_solves()["tiles"] > 1 and b.tile_solves()["built"] == 0
+    for k in range(4):
+        a.step(1)
+        b.step(1)
+        assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v()), k
+    assert a.tile_solves()["aborts"] == 0
