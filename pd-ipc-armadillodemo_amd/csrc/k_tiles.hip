@@ -625,7 +625,9 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
       pre[k] = cur[k];
       cur[k] = d[k];
     }
-    if (it < a.iters - 1 && !st.exchange(a, it, d, 3, &flag, t0, st.xy, st.z)) return;
+    // (a single sweep's iterate is exchanged too: a tile writes its rows of X only
+    // when its neighbours have staged their halos from it)
+    if ((it == 0 || it < a.iters - 1) && !st.exchange(a, it, d, 3, &flag, t0, st.xy, st.z)) return;
     if (out && st.row >= 0 && st.part == 0)
 #pragma unroll
       for (int k = 0; k < 3; k++) out[it * outStride + k * a.ld + st.row] = d[k];

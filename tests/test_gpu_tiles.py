@@ -151,3 +151,43 @@ def test_fp32_steps_of_few_sweeps_match_streamed_sweeps(which, iters):
         b.step(1)
         assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v()), k
     assert a.tile_solves()["aborts"] == 0
+
+
+# the same in FP64: cloths in one launch per outer iteration and, over 128 rows
+# per tile, in separate solves that read their neighbours' rows of X and write
+# their own; tet scenes have only those
+@pytest.mark.parametrize("iters", [1, 2, 3])
+@pytest.mark.parametrize("which", ["20", "200", "tets6", "tets20"])
+def test_fp64_steps_of_few_sweeps_match_streamed_sweeps(which, iters):
+    sc = scenes.config2(cells=int(which[4:]), cloth_n=20) if which.startswith("tets") else _cloth(int(which))
+    sc["params"]["cheb_iters"] = iters
+    print(f"case: {which}, FP64 steps of {iters} sweeps", flush=True)
+    a, b = (pdipc.Simulator.from_scene(sc, sell_stage=st) for st in (1, 2))
+    assert a.tile_solves()["fp64"] == 1 and a.tile_solves()["tiles"] > 1 and b.tile_solves()["built"] == 0
+    for k in range(4):
+        a.step(1)
+        b.step(1)
+        assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v()), k
+    for s in (a, b):
+        s.rollout(2, 0)
+    assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v())
+    assert a.tile_solves()["aborts"] == 0
+    if which.startswith("tets"):
+        return
+    g = np.random.default_rng(iters).normal(size=(a.sim, 3))  # the bound of the 15-sweep rollouts above
+    for u, w in zip(a.backward(dx=g, dv=g), b.backward(dx=g, dv=g)):
+        assert np.allclose(u, w, rtol=1e-9, atol=1e-12 * max(np.abs(w).max(initial=0.0), 1e-300))
+
+
+@pytest.mark.parametrize("which", ["tets6", "tets20", "layers"])
+def test_fp32_tet_steps_of_few_sweeps_match_streamed_sweeps(which):
+    sc = scenes.config4(n=40, side=80.0 / 1024) if which == "layers" else scenes.config2(cells=int(which[4:]), cloth_n=20)
+    for iters in (1, 2, 3):
+        for timed in (False, True):  # with kernel timing the passes run as separate launches
+            sc["params"]["cheb_iters"] = iters
+            print(f"case: {which}, FP32 steps of {iters} sweeps, timed {timed}", flush=True)
+            a, b = (pdipc.Simulator.from_scene(sc, precision=pdipc.FP32_SPLIT, sell_stage=st) for st in (1, 2))
+            a.kernel_timing(timed)
+            a.step(3)
+            b.step(3)
+            assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v())
