@@ -245,10 +245,11 @@ int pdipc_debug_tile_layout(pdipc_handle* h, int max_tiles, long long* sizes, in
  * total points doubles each), written to the device double *toi.  The work is
  * only enqueued on `stream` (NULL: the handle's stream); nothing is allocated
  * and the simulation state is untouched; at most 16,777,216 candidate records
- * (more: PDIPC_E_CAPACITY).  Per-workgroup minima go to a library-wide device
- * array of 512 KiB per GPU, held until the process ends, in 32 slots that
- * handles take in turn at pdipc_init: overlapping calls of one handle (other
- * streams or threads) race, and so do those of handles that share a slot. */
+ * (more: PDIPC_E_CAPACITY).  Per-workgroup minima go to the handle's own place,
+ * from pdipc_init to pdipc_destroy: one of 32 slots of a library-wide device
+ * array of 512 KiB per GPU, or while other handles have them all a buffer of 16
+ * KiB.  Calls of different handles may overlap; overlapping calls of one handle
+ * (other streams or threads) race. */
 int pdipc_toi_noalloc(pdipc_handle* h, const double* x0, const double* x1, double* toi, void* stream);
 
 /* --- measurement support (no counterpart in the reference): replays one

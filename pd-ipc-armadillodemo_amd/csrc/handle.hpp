@@ -28,6 +28,11 @@ void adjoint_free(AdjointState* a);  // releases its device memory
 
 using pdipc::fail;
 
+struct pdipc_handle;
+namespace pdipc {
+void noalloc_release(pdipc_handle* h);  // noalloc.hip: gives the slot of its minima back
+}
+
 struct pdipc_handle {
   using HostSetup = pdipc::HostSetup;
   using SellLayout = pdipc::SellLayout;
@@ -41,7 +46,8 @@ struct pdipc_handle {
   DeviceMesh m;
   hipStream_t stream = nullptr;
   int device = 0;  // the HIP device current at pdipc_init
-  int toiSlot = 0;  // part of the device's array that pdipc_toi_noalloc writes
+  double* toiMinima = nullptr;  // where pdipc_toi_noalloc keeps its workgroup minima,
+  int toiSlot = -1;             // and the slot of the device's array it is (-1: the handle's own buffer)
   // local/global loop captured once per (tile solves, collision flag, precision) and replayed
   hipGraphExec_t lgGraph[2][2][2] = {};
   int tileAborts = 0;  // outer iterations repeated with the streamed sweeps
@@ -89,6 +95,7 @@ struct pdipc_handle {
     delete m.timer;
     pdipc::adjoint_free(adj);
     for (void* p : allocs) (void)hipFree(p);
+    pdipc::noalloc_release(this);  // (the frees have waited for the device)
     if (stage) (void)hipHostFree(stage);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -140,5 +147,5 @@ class TileTurn {
 constexpr int kTileAborted = 1000;
 int tile_recover(pdipc_handle* h, int outer);
 int adjoint_refresh_values(pdipc_handle* h);  // adjoint.hip: after a stiffness change
-int noalloc_setup(int device, int* slot);      // noalloc.hip: with `device` current
+int noalloc_setup(pdipc_handle* h);            // noalloc.hip: with the handle's device current
 }  // namespace pdipc

@@ -3,12 +3,15 @@
 // allocate device memory -- code under HIP graph capture, tight serving loops.
 // Positions and the result stay on the device, the work is only enqueued, and
 // the per-workgroup minima live in `scratch`, a file-scope device array each
-// GPU holds for the life of the process, in slots that handles take in turn (a
-// call writes at most 2,048 minima).  Its device address comes from
-// hipGetSymbolAddress once per device (pdipc_init, with the handle's device
-// current); host code passes that address, never the array's name.
+// GPU holds for the life of the process: a handle has a slot of it from
+// pdipc_init to pdipc_destroy (a call writes at most 2,048 minima), or, while
+// 32 others have them all, a buffer of its own allocated at pdipc_init.  The
+// array's device address comes from hipGetSymbolAddress once per device
+// (pdipc_init, with the handle's device current); host code passes that
+// address, never the array's name.
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <mutex>
 #include <string>
 
@@ -19,15 +22,16 @@ namespace pdipc {
 namespace {
 
 constexpr int kMaxRecs = 1 << 24;      // candidate records a call takes
-constexpr int kSlots = 32;             // handles whose calls may overlap
+constexpr int kSlots = 32;             // handles that have a part of `scratch` at a time
 constexpr int kMaxDevices = 64;
 constexpr int kReduceThreads = 1024;
 
+static_assert(kSlots == 32, "one bit of g_taken each");
 static __device__ __align__(256) double scratch[kSlots * kMaxToiBlocks];
 
 std::mutex g_mu;
 double* g_scratch[kMaxDevices] = {};  // device address of `scratch`, per device
-unsigned g_next[kMaxDevices] = {};    // handles set up so far
+uint32_t g_taken[kMaxDevices] = {};   // bit per slot: some handle has it
 
 // one workgroup: min over the n block minima, then the reference's safety
 // scale (getImpactOfTimeHost, PdIpcGpuFunc.cu:2698-2699): t < 1 -> t * scale
@@ -53,18 +57,32 @@ __global__ void __launch_bounds__(kReduceThreads) k_toi_reduce(const double* __r
 
 }  // namespace
 
-// With `device` current: looks up this device's copy of `scratch` once.
-int noalloc_setup(int device, int* slot) {
+// With the handle's device current: its place for the minima.  This device's
+// copy of `scratch` is looked up once.
+int noalloc_setup(pdipc_handle* h) {
+  const int device = h->device;
   if (device < 0 || device >= kMaxDevices) return fail(PDIPC_E_ARG, "device ordinal out of range");
+  if (h->toiMinima) return PDIPC_OK;
   std::lock_guard<std::mutex> lock(g_mu);
-  *slot = g_next[device]++ % kSlots;
-  if (g_scratch[device]) return PDIPC_OK;
-  void* p = nullptr;
-  hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-  if (e != hipSuccess || !p)
-    return fail(PDIPC_E_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-  g_scratch[device] = (double*)p;
+  if (!g_scratch[device]) {
+    void* p = nullptr;
+    hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+    if (e != hipSuccess || !p)
+      return fail(PDIPC_E_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
+    g_scratch[device] = (double*)p;
+  }
+  if (g_taken[device] == ~0u) return h->alloc(&h->toiMinima, kMaxToiBlocks);
+  h->toiSlot = __builtin_ctz(~g_taken[device]);
+  g_taken[device] |= 1u << h->toiSlot;
+  h->toiMinima = g_scratch[device] + (size_t)h->toiSlot * kMaxToiBlocks;
   return PDIPC_OK;
+}
+
+void noalloc_release(pdipc_handle* h) {
+  if (h->toiSlot < 0) return;
+  std::lock_guard<std::mutex> lock(g_mu);
+  g_taken[h->device] &= ~(1u << h->toiSlot);
+  h->toiSlot = -1;
 }
 
 }  // namespace pdipc
@@ -79,17 +97,10 @@ int pdipc_toi_noalloc(pdipc_handle* h, const double* x0, const double* x1, doubl
   if (nRecs > kMaxRecs)
     return fail(PDIPC_E_CAPACITY, "pdipc_toi_noalloc: " + std::to_string(nRecs) +
                                       " candidate records exceed its limit of 16777216 (use pdipc_debug_toi)");
-  double* scr;
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    scr = g_scratch[h->device];
-  }
-  if (!scr) return fail(PDIPC_E_ARG, "pdipc_toi_noalloc: no scratch address for the handle's device");
-  scr += (size_t)(h->toiSlot % kSlots) * kMaxToiBlocks;
   hipStream_t s = stream ? (hipStream_t)stream : h->stream;
   const pdipc_params& p = h->prm;
   const int minima = launch_ccd_blockmin(h->m, nRecs, x0, x1, p.ccd_filter, p.ccd_iters, p.ccd_step, p.ccd_gap,
-                                         p.touch_policy, scr, s);
-  hipLaunchKernelGGL(k_toi_reduce, dim3(1), dim3(kReduceThreads), 0, s, scr, minima, p.toi_scale, toi);
+                                         p.touch_policy, h->toiMinima, s);
+  hipLaunchKernelGGL(k_toi_reduce, dim3(1), dim3(kReduceThreads), 0, s, h->toiMinima, minima, p.toi_scale, toi);
   return check_launch(h);
 }

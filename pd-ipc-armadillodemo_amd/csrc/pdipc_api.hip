@@ -767,7 +767,7 @@ int pdipc_init(pdipc_handle* h) {
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return fail(PDIPC_E_NODEVICE, "no HIP device");
   HIPCHK(hipGetDevice(&h->device));
-  if ((rc = pdipc::noalloc_setup(h->device, &h->toiSlot))) return rc;
+  if ((rc = pdipc::noalloc_setup(h))) return rc;
   HIPCHK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
   if ((rc = upload_all(h)) || (rc = upload_tiles(h))) return rc;
   h->cnt.sell_entries = h->m.sellEntries;
