@@ -336,7 +336,9 @@ __host__ __device__ inline bool record_ids(int4 r, int id[4]) {  // false for sh
 // The two primitives' separation along the line n between their centres: their
 // distance is at least gap / |n|, less the rounding of FP32 coordinates,
 // differences, products and roots: under 16 * 2^-24 of the largest coordinate,
-// and so of `size`, their sum (both sides have twice that).
+// and so of `size`, their sum (both sides have twice that).  Where |n|^2 is near
+// the smallest FP32 numbers (centres that coincide) its root says nothing: gap 0,
+// which certifies nothing.
 struct Separation {
   float gap, len, size;
 };
@@ -347,8 +349,9 @@ __device__ __forceinline__ Separation separation(int type, const P3f (&x)[4]) {
   P3f n;
 #pragma unroll
   for (int k = 0; k < 3; k++) n.v[k] = b.v[k] + c.v[k] + sa * a.v[k];
-  const float pa = dot(n, a), lo = fminf(dot(n, b), dot(n, c));
-  return {type == 0 ? fminf(pa, lo) : lo - fmaxf(pa, 0.f), __builtin_amdgcn_sqrtf(dot(n, n)),
+  const float pa = dot(n, a), lo = fminf(dot(n, b), dot(n, c)), nn = dot(n, n);
+  const float gap = type == 0 ? fminf(pa, lo) : lo - fmaxf(pa, 0.f);
+  return {nn > 1e-30f ? gap : 0.f, __builtin_amdgcn_sqrtf(nn),
           (sum_abs(x[0]) + sum_abs(x[1])) + (sum_abs(x[2]) + sum_abs(x[3]))};
 }
 constexpr float kRound = 2e-6f;    // 32 * 2^-24

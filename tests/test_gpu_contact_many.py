@@ -6,6 +6,7 @@ the certificate's rounding allowance settles fewer records)."""
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 import pdipc
@@ -57,3 +58,35 @@ def test_no_accd_steps(pair):
     print("case: no ACCD steps", flush=True)
     assert len(sim.debug_broad_phase(x0, x1 - x0)) >= 1 << 21
     assert sim.debug_toi(x0, x1) == 0.0
+
+
+def test_crossing_edges_of_vanishing_normal():
+    """Two edges whose centres lie 1e-21 apart, in coordinates so small that the
+    square of that line's length is no FP32 number: no bound of their distance
+    follows, so the record takes the full path although all around it are
+    settled (2^18 records and more on caller's positions) -- the same time of
+    impact as one record per thread finds."""
+    cl = scenes.cloth_over_sphere(96, 4, ground=False, seed=3, patch_dim=96, sphere_patch_dim=32, height=0.1505)
+    sc = dict(cl, cloths=list(cl["cloths"]))
+    s = 0.01
+    v = s * np.array([[-1.0, 0, 0], [1, 0, 0], [0, -1, 0.25]])
+    w = s * np.array([[0.0, 1e-21 / s, -1], [0, 1e-21 / s, 1], [0.25, 1, 0]])
+    for q in (v, w):
+        sc["cloths"].append(dict(cl["cloths"][0], v=q, f=np.array([[0, 1, 2]], np.int32), patch_dim=2))
+    sc["cloths"][0] = dict(cl["cloths"][0], v=np.asarray(cl["cloths"][0]["v"]) + [0.0, 2.0, 0.0])
+    sc["statics"] = [dict(t, v=np.asarray(t["v"]) + [0.0, 2.0, 0.0]) for t in cl["statics"]]
+    sim = pdipc.Simulator.from_scene(sc)
+    x0 = sim.x()
+    x1 = x0.copy()
+    x1[sim.sim - 3: sim.sim, 1] -= 1e-6  # the second triangle's edge passes through the first's
+    recs = sim.debug_broad_phase(x0, x1 - x0)
+    print(f"case: vanishing normal, {len(recs)} records", flush=True)
+    assert 1 << 18 <= len(recs) < 1 << 21
+    want = sim.debug_toi(x0, x1)
+    assert want < 1.0
+    a, b = (torch.tensor(x.reshape(-1), dtype=torch.float64, device="cuda") for x in (x0, x1))
+    out = torch.full((1,), -1.0, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    sim.toi_noalloc(a.data_ptr(), b.data_ptr(), out.data_ptr())
+    torch.cuda.synchronize()
+    assert out.item() == want
