@@ -1078,8 +1078,10 @@ static bool sort_small(const DeviceMesh& m, hipStream_t s) {
   const int P = m.nPatches;
   if (P > kSortSmall) return false;
   const size_t lds = sort_small_lds((P + kSortThreads - 1) / kSortThreads);
+  // (the attribute is the process's: always the same value, so that no handle
+  // lowers it under another one's launch)
   if (lds > (60 << 10) && hipFuncSetAttribute((const void*)k_sort_small, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              (int)lds) != hipSuccess) {
+                                              (int)sort_small_lds(kSortRounds)) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }

@@ -1095,11 +1095,21 @@ TileShape shape_of(const DeviceMesh& m, int parity, int iters) {
   return a;
 }
 
+// A kernel's dynamic LDS limit belongs to the process, and handles of other
+// tilings share the kernels: always the whole of what its static LDS leaves of
+// a compute unit's 160 KB, so that no handle lowers it under another one.
+constexpr size_t kLdsBytes = 160 << 10;
+bool allow_lds(const void* kernel, size_t lds) {
+  hipFuncAttributes at;
+  return hipFuncGetAttributes(&at, kernel) == hipSuccess && at.sharedSizeBytes + lds <= kLdsBytes &&
+         hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)(kLdsBytes - at.sharedSizeBytes)) == hipSuccess;
+}
+
 template <class K>
 bool fits(K kernel, int threads, size_t lds, int tiles, int cus) {
   if (!kernel) return false;
-  if (lds > (64 << 10) &&
-      hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+  if (lds > (64 << 10) && !allow_lds((const void*)kernel, lds)) {
     (void)hipGetLastError();
     return false;
   }

@@ -3,6 +3,8 @@
 each patch once, equal codes in patch order; and the tree's candidates are the
 oracle's."""
 
+import threading
+
 import numpy as np
 import pytest
 
@@ -31,3 +33,30 @@ def test_sorted_keys(n):
         print(f"  {len(keys)} patches, {len(got)} records", flush=True)
         assert np.array_equal(keys, np.sort(keys))
         assert np.array_equal(np.sort(keys & np.uint64(0xFFFFFFFF)), np.arange(len(keys), dtype=np.uint64))
+
+
+def test_sorts_of_two_handles_in_two_threads():
+    """About 11,000 and 16,300 patches: both need more LDS than the default limit, which
+    is the process's and must never be lowered between another thread's raising
+    it and its launch."""
+    print("case: two handles sorting in two threads", flush=True)
+    sims = [pdipc.Simulator.from_scene(scenes.cloth_over_sphere(n, 1, ground=False, seed=5, patch_dim=n,
+                                                                sphere_patch_dim=8, height=0.166)) for n in (105, 127)]
+    xs = [s.x() for s in sims]
+    want = [s.debug_broad_phase(x, np.zeros_like(x)) for s, x in zip(sims, xs)]
+    bad = []
+
+    def go(i):
+        try:
+            for _ in range(30):
+                if not np.array_equal(sims[i].debug_broad_phase(xs[i], np.zeros_like(xs[i])), want[i]):
+                    bad.append(i)
+        except Exception as e:  # a refused launch
+            bad.append(e)
+
+    ts = [threading.Thread(target=go, args=(i,)) for i in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
