@@ -38,9 +38,9 @@
 // launch stay; launches alternate between two sets of slots, each emptying the
 // other set.
 //
-// Every wait is bounded (kTileWaitTicks): a tile whose neighbours do not
-// arrive -- another process's kernels hold compute units for good -- raises
-// the abort flag, every tile leaves, X keeps a finite value, and the host
+// Every wait is bounded (kTileWaitRounds of polling): a tile whose
+// neighbours do not arrive -- other kernels hold compute units for long --
+// raises the abort flag, every tile leaves, and the host, which restores X,
 // repeats the outer iteration with the streamed kernels.
 #include <algorithm>
 
@@ -51,7 +51,9 @@ namespace pdipc {
 namespace {
 
 constexpr unsigned long long kTileEmpty = 0xfff5a5a5fff5a5a5ull;
-constexpr unsigned long long kTileWaitTicks = 1000000ull;  // 10 ms of the 100 MHz wall clock
+// polling rounds per wait: about 10 ms (2^14 rounds of a 40^2 to 300^2 cloth's
+// solve took 3.8); counted, so that a wait takes no registers for the clock
+constexpr int kTileWaitRounds = 44 << 10;
 constexpr int kRowWords = 3;   // words per row in a publication slot (FP32 vectors use two)
 
 __device__ __forceinline__ void publish(unsigned long long* p, unsigned long long v) {
@@ -290,7 +292,7 @@ struct TileState {
   // polls the words at off[] (-1: none) until all have arrived, then stages them
   template <class U, class U2>
   __device__ __forceinline__ bool poll(const TileShape& a, const unsigned long long* s, const int (&off)[PB],
-                                       int i0, unsigned long long t0, U2* pxy, U* pz) const {
+                                       int i0, U2* pxy, U* pz) const {
     constexpr int N = TileWords<U>::N;
     unsigned long long w[PB];
     for (int spin = 1;; spin++) {
@@ -300,7 +302,7 @@ struct TileState {
 #pragma unroll
       for (int q = 0; q < PB; q++) ready = ready && w[q] != kTileEmpty;
       if (ready) break;
-      if ((spin & 63) == 0 && (wall_clock64() - t0 > kTileWaitTicks ||
+      if ((spin & 63) == 0 && (spin >= kTileWaitRounds ||
                                __hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
         return false;
     }
@@ -313,7 +315,7 @@ struct TileState {
   }
   // stages publication j of the neighbours' rows; false: gave up waiting
   template <class U, class U2>
-  __device__ __forceinline__ bool receive(const TileShape& a, int j, unsigned long long t0, U2* pxy, U* pz) const {
+  __device__ __forceinline__ bool receive(const TileShape& a, int j, U2* pxy, U* pz) const {
     constexpr int N = TileWords<U>::N;
     const int items = nHalo * N;
     if (items == 0) return true;
@@ -325,7 +327,7 @@ struct TileState {
     bool ok = true;
     int i0 = threadIdx.x;
     if constexpr (N == NW) {  // the words of the solve's own type are listed at the start
-      ok = poll(a, s, hw, i0, t0, pxy, pz);
+      ok = poll(a, s, hw, i0, pxy, pz);
       i0 += PB * BT;
     }
     for (; i0 < items; i0 += PB * BT) {
@@ -335,7 +337,7 @@ struct TileState {
         const int i = i0 + q * BT;
         off[q] = i < items ? halo[i / N] * kRowWords + i % N : -1;
       }
-      ok = poll(a, s, off, i0, t0, pxy, pz) && ok;
+      ok = poll(a, s, off, i0, pxy, pz) && ok;
     }
     return ok;
   }
@@ -343,11 +345,11 @@ struct TileState {
   // into LDS; false (for the whole workgroup): some wait was given up
   template <class U, class U2>
   __device__ __forceinline__ bool exchange(const TileShape& a, int j, const U (&d)[3], int old, int* flag,
-                                           unsigned long long t0, U2* pxy, U* pz) const {
+                                           U2* pxy, U* pz) const {
     send(a, j, d, old);
     __syncthreads();  // every row of the tile has read the old vector
     stage_own(pxy, pz, d[0], d[1], d[2]);
-    if (!receive(a, j, t0, pxy, pz)) {
+    if (!receive(a, j, pxy, pz)) {
       *flag = 1;
       __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -400,7 +402,6 @@ __global__ void __launch_bounds__(BT) k_tile_solve32(TileShape a, const float* _
     st.stage_own(st.xy, st.z, q.x, q.y, q.z);
   }
   __syncthreads();
-  const unsigned long long t0 = wall_clock64();
   for (int it = 1; it < a.iters; it++) {
     const float Wc = (float)st.cheb[it - 1];
     float acc[3];
@@ -412,7 +413,7 @@ __global__ void __launch_bounds__(BT) k_tile_solve32(TileShape a, const float* _
       pre[k] = cur[k];
       cur[k] = d[k];
     }
-    if (it < a.iters - 1 && !st.exchange(a, it - 1, d, 2, &flag, t0, st.xy, st.z)) return;
+    if (it < a.iters - 1 && !st.exchange(a, it - 1, d, 2, &flag, st.xy, st.z)) return;
   }
   if (st.row >= 0 && st.part == 0)
 #pragma unroll
@@ -473,7 +474,6 @@ __global__ void __launch_bounds__(kTwoThreads) k_tile_solve32_two(TileShape a, c
     st.z[a.R + u] = q.z;
   }
   __syncthreads();
-  const unsigned long long t0 = wall_clock64();
   for (int it = 1; it < a.iters; it++) {
     const float Wc = (float)st.cheb[it - 1];
     float d[2][3];
@@ -524,7 +524,7 @@ __global__ void __launch_bounds__(kTwoThreads) k_tile_solve32_two(TileShape a, c
         st.xy[r] = make_float2(d[q][0], d[q][1]);
         st.z[r] = d[q][2];
       }
-    if (!st.receive(a, j, t0, st.xy, st.z)) {
+    if (!st.receive(a, j, st.xy, st.z)) {
       flag = 1;
       __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -608,7 +608,6 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
   }
   if constexpr (TPR == 1) st.load(a, ri, val);
   __syncthreads();
-  const unsigned long long t0 = wall_clock64();
   for (int it = 0; it < a.iters; it++) {
     const double Wc = it > 0 ? st.cheb[it - 1] : 0.0;
     double acc[3], d[3];
@@ -627,7 +626,7 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
     }
     // (a single sweep's iterate is exchanged too: a tile writes its rows of X only
     // when its neighbours have staged their halos from it)
-    if ((it == 0 || it < a.iters - 1) && !st.exchange(a, it, d, 3, &flag, t0, st.xy, st.z)) return;
+    if ((it == 0 || it < a.iters - 1) && !st.exchange(a, it, d, 3, &flag, st.xy, st.z)) return;
     if (out && st.row >= 0 && st.part == 0)
 #pragma unroll
       for (int k = 0; k < 3; k++) out[it * outStride + k * a.ld + st.row] = d[k];
@@ -665,7 +664,6 @@ __global__ void __launch_bounds__(BT) k_tile_adj(TileShape a, const double* __re
     st.stage_own(st.xy, st.z, cur[0], cur[1], cur[2]);
   }
   __syncthreads();
-  const unsigned long long t0 = wall_clock64();
   for (int k = g.K - 1; k >= 0; k--) {
     const double w = g.w[k], b = k + 1 <= g.K - 1 ? 1.0 - g.w[k + 1] : 0.0;
     double acc[3], d[3];
@@ -678,7 +676,7 @@ __global__ void __launch_bounds__(BT) k_tile_adj(TileShape a, const double* __re
       oth[q] = cur[q];
       cur[q] = d[q];
     }
-    if (k > 0 && !st.exchange(a, g.K - 1 - k, d, 3, &flag, t0, st.xy, st.z)) return;
+    if (k > 0 && !st.exchange(a, g.K - 1 - k, d, 3, &flag, st.xy, st.z)) return;
     if (st.row >= 0 && st.part == 0)
 #pragma unroll
       for (int q = 0; q < 3; q++) g.u[k][q * a.ld + st.row] = d[q];
@@ -799,8 +797,7 @@ __global__ void __launch_bounds__(BT) k_tile_loop(TileShape a, TileLoop g, const
   int j = 0;  // publications so far
   for (int pass = 0; pass < g.passes; pass++) {
     const bool last = pass == g.passes - 1;
-    const unsigned long long t0 = wall_clock64();
-    // curvature
+      // curvature
     for (int i = t; i < g.curvCap; i += BT) {
       const int4 it = g.curvItems[(size_t)blockIdx.x * g.curvCap + i];
       if (it.y == 0) continue;
@@ -887,12 +884,12 @@ __global__ void __launch_bounds__(BT) k_tile_loop(TileShape a, TileLoop g, const
       }
       if constexpr (F32) {
         // (publication j - 2: a correction of two words, or with one sweep the last pass's v)
-        if (!st.exchange(a, j, vv, a.iters == 1 ? 3 : 2, &flag, t0, Vxy, Vz)) return;
+        if (!st.exchange(a, j, vv, a.iters == 1 ? 3 : 2, &flag, Vxy, Vz)) return;
         j++;
 #pragma unroll
         for (int k = 0; k < 3; k++) r[k] = pt[k];
       } else {
-        if (!st.exchange(a, j, r, 3, &flag, t0, Vxy, Vz)) return;
+        if (!st.exchange(a, j, r, 3, &flag, Vxy, Vz)) return;
         j++;
         if (g.rhsOut && live && st.part == 0)
 #pragma unroll
@@ -924,7 +921,7 @@ __global__ void __launch_bounds__(BT) k_tile_loop(TileShape a, TileLoop g, const
         const bool done = it == a.iters - 1;
         if (done && last) break;
         // (publication j - 2 was v, of three words, at it = 1)
-        if (!st.exchange(a, j, cur, it == 1 ? 3 : 2, &flag, t0, (float2*)st.xy, (float*)st.z)) return;
+        if (!st.exchange(a, j, cur, it == 1 ? 3 : 2, &flag, (float2*)st.xy, (float*)st.z)) return;
         j++;
         if (done) break;
         const float Wc = (float)st.cheb[it];
@@ -979,7 +976,7 @@ __global__ void __launch_bounds__(BT) k_tile_loop(TileShape a, TileLoop g, const
           xi[k] = d[k];
         }
         if (!(last && it == a.iters - 1)) {
-          if (!st.exchange(a, j, d, 3, &flag, t0, (double2*)st.xy, (double*)st.z)) return;
+          if (!st.exchange(a, j, d, 3, &flag, (double2*)st.xy, (double*)st.z)) return;
           j++;
         }
         if (g.itOut && live && st.part == 0)
