@@ -225,7 +225,8 @@ int pdipc_sweep_staging(pdipc_handle* h, int* path);
  * [1] / [2] 1 if its FP32 / FP64 solves run as tiles, [3] tiles, [4] rows per
  * tile, [5] outer iterations repeated with the streamed sweeps because a tile
  * gave up waiting for its neighbours (a backward pass repeated so counts as
- * one).  request_abort makes the next tile solve of a step (1) or of a backward
+ * one).  After two within a minute [1] and [2] are 0 for 2 s, in which the
+ * handle's steps stream; each further one doubles that, up to 32 s.  request_abort makes the next tile solve of a step (1) or of a backward
  * pass (2) give up (tests). */
 int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort);
 /* The tile tables for at most max_tiles tiles from the host precompute alone

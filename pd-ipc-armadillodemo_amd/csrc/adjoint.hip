@@ -676,8 +676,7 @@ int pdipc_backward(pdipc_handle* h, const double* dx, const double* dv, double* 
     int gaveUp = 0;  // a tile of some reverse pass gave up waiting: once more, with the streamed sweeps
     HIPCHK(h->copy(&gaveUp, m.tile.abort + 1, sizeof gaveUp, hipMemcpyDeviceToHost));
     if (gaveUp) {
-      h->tileAborts++;
-      m.tile.on = false;
+      tile_gave_up(h);
       HIPCHK(hipMemsetAsync(m.tile.abort + 1, 0, sizeof gaveUp, s));
       if ((rc = reverse_rollout(h, dx, dv, &xin, &vin))) return rc;
     }

@@ -50,7 +50,9 @@ struct pdipc_handle {
   int toiSlot = -1;             // and the slot of the device's array it is (-1: the handle's own buffer)
   // local/global loop captured once per (tile solves, collision flag, precision) and replayed
   hipGraphExec_t lgGraph[2][2][2] = {};
-  int tileAborts = 0;  // outer iterations repeated with the streamed sweeps
+  int tileAborts = 0;  // outer iterations repeated with the streamed sweeps,
+  int tileStreak = 0;  // of them the last in a row less than a minute apart,
+  double tileLastAbort = 0.0, tileRest = 0.0;  // when the last one was, and until when no tile solve is tried
   std::vector<void*> allocs;
   // host mirrors
   void* scalHost = nullptr;  // pinned, after `stage`: residual, toiBits, counters[12], the tile solves' abort flag
@@ -133,6 +135,7 @@ class TileTurn {
  public:
   explicit TileTurn(pdipc_handle* h);
   ~TileTurn();
+  void renew();  // before each step of the call: tile solves may run, or again
   TileTurn(const TileTurn&) = delete;
   TileTurn& operator=(const TileTurn&) = delete;
 
@@ -142,10 +145,11 @@ class TileTurn {
 };
 // returned by read_scalars (and what calls it) when a tile solve gave up
 // waiting; tile_recover clears the flag, switches the handle to the streamed
-// sweeps for the rest of the call and restores X as the outer iteration
+// sweeps until the turn is renewed and restores X as the outer iteration
 // found it
 constexpr int kTileAborted = 1000;
 int tile_recover(pdipc_handle* h, int outer);
+void tile_gave_up(pdipc_handle* h);  // counts it, and may have the handle rest from tile solves
 int adjoint_refresh_values(pdipc_handle* h);  // adjoint.hip: after a stiffness change
 int noalloc_setup(pdipc_handle* h);            // noalloc.hip: with the handle's device current
 }  // namespace pdipc

@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -73,16 +74,26 @@ int read_scalars(pdipc_handle* h) {
 // ---- tile solves
 namespace {
 std::atomic<int> g_tileTurn[64];  // per device: 1 while a handle may launch tile solves
-constexpr int kTileMaxAborts = 2;  // a handle that gave up this often keeps to the streamed sweeps
+// A handle whose tile solves gave up twice within a minute (long kernels of
+// others hold the device) keeps to the streamed sweeps for 2 s, then 4 and up
+// to 32: an attempt that fails costs its 10 ms and one outer iteration, so at
+// most about 1 % of the time is lost to attempts.
+constexpr double kTileForget = 60.0, kTileRestMin = 2.0, kTileRestMax = 32.0;
+double seconds_now() {
+  return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+bool tiles_may(const pdipc_handle* h) {
+  return h->m.tile.built && (h->tileStreak < 2 || seconds_now() >= h->tileRest);
+}
 }  // namespace
 
-TileTurn::TileTurn(pdipc_handle* h) : h_(h) {
-  TileMesh& t = h->m.tile;
-  t.on = false;
-  if (!t.built || h->tileAborts >= kTileMaxAborts || h->device < 0 || h->device >= 64) return;
+TileTurn::TileTurn(pdipc_handle* h) : h_(h) { renew(); }
+void TileTurn::renew() {
+  const bool may = tiles_may(h_) && h_->device >= 0 && h_->device < 64;
+  if (held_ && !may) g_tileTurn[h_->device].store(0);  // (what gave up has left the device)
   int free = 0;
-  held_ = g_tileTurn[h->device].compare_exchange_strong(free, 1);
-  t.on = held_;
+  held_ = may && (held_ || g_tileTurn[h_->device].compare_exchange_strong(free, 1));
+  h_->m.tile.on = held_;
 }
 TileTurn::~TileTurn() {
   h_->m.tile.on = false;
@@ -91,10 +102,18 @@ TileTurn::~TileTurn() {
   g_tileTurn[h_->device].store(0);
 }
 
+void tile_gave_up(pdipc_handle* h) {
+  const double now = seconds_now();
+  h->tileAborts++;
+  h->tileStreak = h->tileStreak > 0 && now - h->tileLastAbort < kTileForget ? h->tileStreak + 1 : 1;
+  h->tileLastAbort = now;
+  if (h->tileStreak >= 2) h->tileRest = now + std::min(kTileRestMax, std::ldexp(kTileRestMin, std::min(h->tileStreak - 2, 8)));
+  h->m.tile.on = false;
+}
+
 int tile_recover(pdipc_handle* h, int outer) {
   DeviceMesh& m = h->m;
-  h->tileAborts++;
-  m.tile.on = false;
+  tile_gave_up(h);
   HIPCHK(hipMemsetAsync(m.tile.abort, 0, sizeof(int), h->stream));
   launch_copy(m.X, outer == 0 ? m.X0 : m.Xold, 3 * (int64_t)m.ld, h->stream);
   if (outer == 0) launch_predict(m, h->prm.dt, h->stream);
@@ -795,6 +814,7 @@ int pdipc_step(pdipc_handle* h, int nsteps) {
   if (rc) return rc;
   pdipc::TileTurn turn(h);
   for (int i = 0; i < nsteps; i++) {
+    if (i > 0) turn.renew();
     if ((rc = advance(h))) return rc;
     if ((rc = fold_timer(h))) return rc;
   }
@@ -1061,7 +1081,7 @@ int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort) {
   if (rc) return rc;
   const TileMesh& t = h->m.tile;
   if (info) {
-    const bool may = t.built && h->tileAborts < kTileMaxAborts;
+    const bool may = tiles_may(h);
     info[0] = t.built ? 1 : 0;
     info[1] = may && t.ok32 ? 1 : 0;
     info[2] = may && t.ok64 ? 1 : 0;

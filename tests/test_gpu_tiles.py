@@ -4,6 +4,7 @@ sweeps; when a tile gives up waiting; and with several handles stepping at
 once from different threads."""
 
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -191,3 +192,28 @@ def test_fp32_tet_steps_of_few_sweeps_match_streamed_sweeps(which):
             a.step(3)
             b.step(3)
             assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v())
+
+
+def test_handle_that_gave_up_twice_tries_again():
+    """It rests from tile solves for two seconds, with the same bits meanwhile."""
+    print("case: two tile aborts, then a rest", flush=True)
+    a, b = (pdipc.Simulator.from_scene(_cloth(40), use_graphs=1) for _ in range(2))
+    for k in range(2):
+        a.tile_solves(request_abort=True)
+        a.step(2)
+        b.step(2)
+    assert a.tile_solves()["aborts"] == 2 and a.tile_solves()["fp64"] == 0
+    a.step(1)
+    b.step(1)
+    time.sleep(2.1)
+    assert a.tile_solves()["fp64"] == 1
+    a.step(2)
+    b.step(2)
+    assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v())
+    assert a.tile_solves()["aborts"] == 2
+    a.tile_solves(request_abort=True)  # the tiles ran: the next request is seen, and the rest is longer
+    a.step(1)
+    b.step(1)
+    time.sleep(2.1)
+    assert a.tile_solves()["aborts"] == 3 and a.tile_solves()["fp64"] == 0
+    assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v())
