@@ -226,8 +226,10 @@ int pdipc_sweep_staging(pdipc_handle* h, int* path);
  * tile, [5] outer iterations repeated with the streamed sweeps because a tile
  * gave up waiting for its neighbours (a backward pass repeated so counts as
  * one).  After two within a minute [1] and [2] are 0 for 2 s, in which the
- * handle's steps stream; each further one doubles that, up to 32 s.  request_abort makes the next tile solve of a step (1) or of a backward
- * pass (2) give up (tests). */
+ * handle's steps stream; each further one doubles that, up to 32 s.
+ * request_abort (tests): the next tile solve of a step (1) or of a backward pass
+ * (2) gives up before it begins; 65536 + j, 131072 + j: the first tile of the
+ * first one that comes to a publication j of iterates (from 0) does so there. */
 int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort);
 /* The tile tables for at most max_tiles tiles from the host precompute alone
  * (after pdipc_host_setup; no device).  sizes: [0] 1 if the scene tiles, [1]

@@ -678,6 +678,7 @@ int pdipc_backward(pdipc_handle* h, const double* dx, const double* dv, double* 
     if (gaveUp) {
       tile_gave_up(h);
       HIPCHK(hipMemsetAsync(m.tile.abort + 1, 0, sizeof gaveUp, s));
+      HIPCHK(hipMemsetAsync(m.tile.abort + 3, 0, sizeof gaveUp, s));
       if ((rc = reverse_rollout(h, dx, dv, &xin, &vin))) return rc;
     }
   }

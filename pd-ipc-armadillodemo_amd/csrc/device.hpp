@@ -111,7 +111,9 @@ struct TileMesh {
   uint16_t* loc = nullptr;
   unsigned long long* slots = nullptr;  // two sets of four publication slots
   double* cheb = nullptr;               // W_1 .. of the Chebyshev recurrence
-  int* abort = nullptr;                 // set by a tile that gave up waiting (abort[1]: in a reverse pass)
+  // set by a tile that gave up waiting (abort[1]: in a reverse pass); abort[2] and
+  // [3]: the publication, + 1, at which tile 0 of the same gives up (tests; 0: none)
+  int* abort = nullptr;
   bool adj = false;                     // the reverse sweeps' kernel fits
   // the local/global loop in one launch (scenes of cloths only, curvCap > 0)
   bool loop32 = false, loop64 = false;

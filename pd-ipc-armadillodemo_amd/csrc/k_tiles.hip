@@ -115,7 +115,7 @@ struct TileShape {  // what one launch works on (device pointers of DeviceMesh)
   unsigned long long* slots;  // this launch's four publication slots
   unsigned long long* other;  // the other set, emptied here
   size_t slotStride;          // words per slot
-  int* abort;
+  int* abort;                 // and, two words on, where tile 0 gives up (tests): a publication + 1
   const double* cheb;         // W_1 .. W_{iters-1}
   int iters;
 };
@@ -136,6 +136,7 @@ struct TileState {
   T* z;
   double* cheb;        // LDS: the sweeps' weights
   int hw[PB];  // word offset of the thread's first polled words (-1: none)
+  int stop;    // this tile gives up at that publication (-1: none)
 
   // a row's LDS indices (tables of `threads` threads per tile, here thread t's)
   static __device__ __forceinline__ void load_loc(const TileShape& a, int threads, int t, unsigned (&li)[E / 2]) {
@@ -178,7 +179,8 @@ struct TileState {
     }
   }
   // LDS pointers, weights, halo and the first polled words
-  __device__ __forceinline__ void setup(const TileShape& a, char* lds) {
+  __device__ __forceinline__ void setup(const TileShape& a, char* lds, int stopAt) {
+    stop = __builtin_amdgcn_readfirstlane(stopAt);
     const int t = threadIdx.x, tile = blockIdx.x;
     xy = (V2*)lds;
     z = (T*)(lds + (size_t)a.uCap * sizeof(V2));
@@ -204,8 +206,8 @@ struct TileState {
     load_val(ri, part, val, v);
   }
   template <bool EMPTY_OTHER, bool LOAD = true>
-  __device__ __forceinline__ int4 init(const TileShape& a, const T* __restrict__ val, char* lds) {
-    setup(a, lds);
+  __device__ __forceinline__ int4 init(const TileShape& a, const T* __restrict__ val, char* lds, int stopAt) {
+    setup(a, lds, stopAt);
     const int t = threadIdx.x, ln = t % kWave;
     rl = (t / kWave) * RW + ln % RW;
     part = ln / RW;
@@ -349,7 +351,7 @@ struct TileState {
     send(a, j, d, old);
     __syncthreads();  // every row of the tile has read the old vector
     stage_own(pxy, pz, d[0], d[1], d[2]);
-    if (!receive(a, j, pxy, pz)) {
+    if (!receive(a, j, pxy, pz) || j == stop) {
       *flag = 1;
       __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -371,9 +373,13 @@ template <class T, int TPR, int W>
 constexpr bool tile_lean() { return 8 / TPR * W * (2 + (int)sizeof(T) / 4) > 100; }
 
 // leaves the kernel at its start when an earlier launch gave up (the same
-// answer for the whole workgroup)
-__device__ __forceinline__ bool tile_aborted(const int* abort, int* flag) {
-  if (threadIdx.x == 0) *flag = __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// answer for the whole workgroup); stop: the publication at which this tile does
+__device__ __forceinline__ bool tile_aborted(const int* abort, int* flag, int* stop) {
+  if (threadIdx.x == 0) {
+    const int f = __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *stop = (blockIdx.x == 0 ? __hip_atomic_load(abort + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0) - 1;
+    *flag = f;
+  }
   __syncthreads();
   return *flag != 0;
 }
@@ -384,10 +390,10 @@ template <int BT, int TPR, int W, bool LM>
 __global__ void __launch_bounds__(BT) k_tile_solve32(TileShape a, const float* __restrict__ val,
                                                      const float4* __restrict__ r0, double* __restrict__ X) {
   extern __shared__ __attribute__((aligned(16))) char tileLds[];
-  __shared__ int flag;
-  if (tile_aborted(a.abort, &flag)) return;
+  __shared__ int flag, stop;
+  if (tile_aborted(a.abort, &flag, &stop)) return;
   TileState<float, BT, TPR, W, LM, 6, tile_lean<float, TPR, W>()> st;
-  st.template init<true>(a, val, tileLds);
+  st.template init<true>(a, val, tileLds, stop);
   for (int u = threadIdx.x; u < st.nHalo; u += BT) {
     const float4 q = r0[st.halo[u]];
     st.xy[a.R + u] = make_float2(q.x, q.y);
@@ -438,10 +444,10 @@ __global__ void __launch_bounds__(kTwoThreads) k_tile_solve32_two(TileShape a, c
   constexpr int BT = kTwoThreads;
   using St = TileState<float, BT, 1, 8, LM, 4, true>;
   extern __shared__ __attribute__((aligned(16))) char tileLds[];
-  __shared__ int flag;
-  if (tile_aborted(a.abort, &flag)) return;
+  __shared__ int flag, stop;
+  if (tile_aborted(a.abort, &flag, &stop)) return;
   St st;
-  st.setup(a, tileLds);
+  st.setup(a, tileLds, stop);
   st.part = 0;
   float* rs = (float*)(tileLds + tile_lds_bytes<float>(a.uCap, a.iters));  // r0, then delta_{k-1}, of the own rows
   float* ps = rs + 3 * 2 * BT;
@@ -524,7 +530,7 @@ __global__ void __launch_bounds__(kTwoThreads) k_tile_solve32_two(TileShape a, c
         st.xy[r] = make_float2(d[q][0], d[q][1]);
         st.z[r] = d[q][2];
       }
-    if (!st.receive(a, j, st.xy, st.z)) {
+    if (!st.receive(a, j, st.xy, st.z) || j == st.stop) {
       flag = 1;
       __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -554,13 +560,13 @@ template <int BT, int TPR, int W, bool LM>
 __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* __restrict__ val, TileFirst ft,
                                                      double* X, double* __restrict__ out, int64_t outStride) {
   extern __shared__ __attribute__((aligned(16))) char tileLds[];
-  __shared__ int flag;
-  if (tile_aborted(a.abort, &flag)) return;
+  __shared__ int flag, stop;
+  if (tile_aborted(a.abort, &flag, &stop)) return;
   using State = TileState<double, BT, TPR, W, LM, 6, tile_lean<double, TPR, W>()>;
   constexpr int SUBS = State::SUBS;
   State st;
   // (one thread per row: the entries' registers are not free before c is formed)
-  const int4 ri = st.template init<true, (TPR > 1)>(a, val, tileLds);
+  const int4 ri = st.template init<true, (TPR > 1)>(a, val, tileLds, stop);
   for (int u = threadIdx.x; u < st.nHalo; u += BT) {
     const int h = st.halo[u];
     st.xy[a.R + u] = make_double2(X[h], X[a.ld + h]);
@@ -644,10 +650,10 @@ __global__ void __launch_bounds__(BT) k_tile_solve64(TileShape a, const double* 
 template <int BT, int TPR, int W, bool LM>
 __global__ void __launch_bounds__(BT) k_tile_adj(TileShape a, const double* __restrict__ val, TileAdj g) {
   extern __shared__ __attribute__((aligned(16))) char tileLds[];
-  __shared__ int flag;
-  if (tile_aborted(a.abort, &flag)) return;
+  __shared__ int flag, stop;
+  if (tile_aborted(a.abort, &flag, &stop)) return;
   TileState<double, BT, TPR, W, LM, 6, tile_lean<double, TPR, W>()> st;
-  st.template init<true>(a, val, tileLds);
+  st.template init<true>(a, val, tileLds, stop);
   const double* u0 = g.u[g.K];
   for (int q = threadIdx.x; q < st.nHalo; q += BT) {
     const int h = st.halo[q];
@@ -754,13 +760,13 @@ constexpr size_t tile_loop_lds(int uCap, int aCap, int iters) {
 template <class T, int BT, int TPR, int W, bool LM>
 __global__ void __launch_bounds__(BT) k_tile_loop(TileShape a, TileLoop g, const T* __restrict__ val) {
   extern __shared__ __attribute__((aligned(16))) char tileLds[];
-  __shared__ int flag;
-  if (tile_aborted(a.abort, &flag)) return;
+  __shared__ int flag, stop;
+  if (tile_aborted(a.abort, &flag, &stop)) return;
   constexpr bool F32 = sizeof(T) == 4;
   using State = TileState<T, BT, TPR, W, LM, 3, tile_lean<T, TPR, W>()>;
   constexpr int SUBS = State::SUBS, QL = 4 / TPR;
   State st;
-  st.template init<false>(a, val, tileLds);
+  st.template init<false>(a, val, tileLds, stop);
   const int t = threadIdx.x, U = a.uCap, ld = a.ld;
   // LDS arrays after the iterate and the weights
   char* p = tileLds + ((tile_lds_bytes<T>(U, a.iters) + 15) & ~(size_t)15);

@@ -73,6 +73,7 @@ int read_scalars(pdipc_handle* h) {
 
 // ---- tile solves
 namespace {
+constexpr int kAbortAt = 1 << 16;  // pdipc_tile_solves: give up at a publication
 std::atomic<int> g_tileTurn[64];  // per device: 1 while a handle may launch tile solves
 // A handle whose tile solves gave up twice within a minute (long kernels of
 // others hold the device) keeps to the streamed sweeps for 2 s, then 4 and up
@@ -115,6 +116,7 @@ int tile_recover(pdipc_handle* h, int outer) {
   DeviceMesh& m = h->m;
   tile_gave_up(h);
   HIPCHK(hipMemsetAsync(m.tile.abort, 0, sizeof(int), h->stream));
+  HIPCHK(hipMemsetAsync(m.tile.abort + 2, 0, sizeof(int), h->stream));
   launch_copy(m.X, outer == 0 ? m.X0 : m.Xold, 3 * (int64_t)m.ld, h->stream);
   if (outer == 0) launch_predict(m, h->prm.dt, h->stream);
   return check_launch(h);
@@ -1090,9 +1092,10 @@ int pdipc_tile_solves(pdipc_handle* h, int* info, int request_abort) {
     info[5] = h->tileAborts;
   }
   if (request_abort && t.built) {
-    const int one = 1;
-    HIPCHK(hipMemcpyAsync(t.abort + (request_abort == 2 ? 1 : 0), &one, sizeof(int), hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
+    // 1, 2: at its start; kAbortAt (twice: backward) + j: tile 0 at publication j
+    const bool at = request_abort >= kAbortAt, back = at ? request_abort >= 2 * kAbortAt : request_abort == 2;
+    const int value = at ? request_abort % kAbortAt + 1 : 1;
+    HIPCHK(h->copy(t.abort + (back ? 1 : 0) + (at ? 2 : 0), &value, sizeof(int), hipMemcpyHostToDevice));
   }
   return PDIPC_OK;
 }

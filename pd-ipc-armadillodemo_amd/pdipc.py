@@ -378,7 +378,8 @@ class Simulator:
     def tile_solves(self, request_abort=False):
         """Whether this handle's Chebyshev solves run as tiles (one launch per
         solve), the tiling, and how often a tile gave up waiting; request_abort
-        makes the next one of a step (1) or a backward pass (2) give up."""
+        makes the next one of a step (1) or a backward pass (2) give up (65536 +
+        j, 131072 + j: its first tile, at its publication j)."""
         info = np.zeros(6, np.int32)
         _check(lib().pdipc_tile_solves(self.h, _ip(info), int(request_abort)))
         return dict(zip(("built", "fp32", "fp64", "tiles", "rows_per_tile", "aborts"), (int(v) for v in info)))

@@ -217,3 +217,52 @@ def test_handle_that_gave_up_twice_tries_again():
     time.sleep(2.1)
     assert a.tile_solves()["aborts"] == 3 and a.tile_solves()["fp64"] == 0
     assert np.array_equal(a.x(), b.x()) and np.array_equal(a.v(), b.v())
+
+
+# (scene, precision): the loop in one launch in both precisions; separate solves
+# of one and two rows per thread and of tets.  One tile gives up when the others
+# are under way: some have written X, others have not.
+@pytest.mark.parametrize("which,prec", [("40", pdipc.FP64), ("40", pdipc.FP32_SPLIT), ("150", pdipc.FP32_SPLIT),
+                                        ("200", pdipc.FP64), ("300", pdipc.FP32_SPLIT), ("380", pdipc.FP32_SPLIT),
+                                        ("tets6", pdipc.FP64), ("tets6", pdipc.FP32_SPLIT)])
+def test_solve_given_up_under_way_repeats_with_streamed_sweeps(which, prec):
+    sc = scenes.config2(cells=6, cloth_n=20) if which == "tets6" else _cloth(int(which))
+    ref = pdipc.Simulator.from_scene(sc, precision=prec, sell_stage=2)
+    xs = []
+    for _ in range(3):
+        ref.step(1)
+        xs.append((ref.x(), ref.v(), ref.counters()))
+    for j in (0, 1, 5, 12):
+        print(f"case: {which}, precision {prec}, first tile gives up at publication {j}", flush=True)
+        a = pdipc.Simulator.from_scene(sc, precision=prec, use_graphs=j % 2)
+        assert a.tile_solves()["tiles"] > 1
+        for k in range(3):
+            if k == 1:
+                a.tile_solves(request_abort=65536 + j)
+            a.step(1)
+            assert np.array_equal(a.x(), xs[k][0]) and np.array_equal(a.v(), xs[k][1]), k
+            assert a.counters()["outer_iters"] == xs[k][2]["outer_iters"]
+        assert a.tile_solves()["aborts"] == 1
+
+
+def test_passes_given_up_under_way_repeat_with_streamed_sweeps():
+    """Recorded passes (their iterates are recorded again) and reverse sweeps."""
+    sc = _cloth(40)
+    d = pdipc.Simulator.from_scene(sc)
+    g = np.random.default_rng(0).normal(size=(d.sim, 3))
+    d.rollout(3, 2)
+    want = d.backward(dx=g)
+    for every in (0, 2):
+        for j in (0, 7, 13):
+            for back in (0, 1):
+                print(f"case: checkpoints every {every}, {'backward' if back else 'rollout'} publication {j}", flush=True)
+                c = pdipc.Simulator.from_scene(sc)
+                if not back:
+                    c.tile_solves(request_abort=65536 + j)
+                c.rollout(3, every)
+                assert np.array_equal(c.x(), d.x()) and c.tile_solves()["aborts"] == 1 - back
+                if back:
+                    c.tile_solves(request_abort=131072 + j)
+                for u, w in zip(c.backward(dx=g), want):
+                    assert np.allclose(u, w, rtol=1e-9, atol=1e-12 * max(np.abs(w).max(initial=0.0), 1e-300))
+                assert c.tile_solves()["aborts"] == 1
