@@ -275,7 +275,11 @@ int pdipc_time_kernel(pdipc_handle* h, int which, int reps, double* avg_us, doub
  * 0 FP64 sweeps, 1 FP32-split sweeps, 2 local-step rhs gather, 3 cloth
  * curvature and tet projection, 4 first FP64 sweep and FP32-split residual
  * passes, 5 M^2 operator update, 6 time of impact, 7 barrier terms, 8 broad
- * phase (one span per broad phase, its host waits included). */
+ * phase (one span per broad phase, its host waits included), 9 the launches
+ * that run all local/global passes of an outer iteration (only after
+ * pdipc_kernel_timing(h, 2): after 1 such a scene's passes run as the kernels of
+ * classes 0 to 4, which its untimed steps do not launch).  A tile solve counts
+ * as its sweeps.  6 and 7 include the packing of the points. */
 int pdipc_kernel_timing(pdipc_handle* h, int enable);
 int pdipc_get_kernel_times(pdipc_handle* h, double* us, long long* counts, int nclasses);
 

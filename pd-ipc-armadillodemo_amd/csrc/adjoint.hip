@@ -345,7 +345,7 @@ void enqueue_taped_lg(pdipc_handle* h, int withCol) {
   launch_copy(L.D(b), m.sysDiag, m.nSim, s);
   launch_operators(m, p.omega, PDIPC_FP64, s);
   if (m.tile.use(PDIPC_FP64)) launch_tile_reset(m, s);
-  if (m.tile.loop(PDIPC_FP64) && !m.timer) {
+  if (m.tile.loop(PDIPC_FP64, m.timer)) {
     launch_tile_loop(m, PDIPC_FP64, p.omega, p.lg_iters, p.cheb_iters, withCol, L.rhs(b, 0), (int64_t)L.V3,
                      L.it(b, 0, 1), (int64_t)L.V3, s);
     return;

@@ -44,18 +44,22 @@ enum TimerClass {
   TC_CCD,          // time of impact
   TC_BARRIER,      // barrier projection terms
   TC_BROAD,        // broad phase (span, host waits included)
+  TC_LOOP,         // all local/global passes of an outer iteration in one launch
   TC_COUNT
 };
 
 struct KernelTimer {
   std::vector<hipEvent_t> pool;  // (start, stop) pairs
   std::vector<int> cls;          // class of each pair in use
-  std::vector<int> weight;       // launches each pair counts as (a tile solve: its sweeps)
+  std::vector<int> weight;       // launches each pair counts as (a tile solve: its sweeps; a kernel that
+                                 // prepares another's operands: 0)
+  bool perPass = true;           // scenes whose passes run in one launch: the passes' kernels one by one instead
   size_t used = 0;
   double us[TC_COUNT] = {};
   long long count[TC_COUNT] = {};
-  // a (start, stop) pair for one launch of class c (false: no event available)
-  bool take(int c, hipEvent_t* e0, hipEvent_t* e1) {
+  // a (start, stop) pair for one launch of class c that counts as `launches` of
+  // them (false: no event available)
+  bool take(int c, hipEvent_t* e0, hipEvent_t* e1, int launches = 1) {
     if (2 * used + 2 > pool.size()) {
       hipEvent_t a = nullptr, b = nullptr;
       if (hipEventCreate(&a) != hipSuccess) return false;
@@ -70,27 +74,30 @@ struct KernelTimer {
     *e1 = pool[2 * used + 1];
     if (cls.size() <= used) cls.resize(used + 1);
     if (weight.size() <= used) weight.resize(used + 1);
-    weight[used] = 1;
+    weight[used] = launches;
     cls[used++] = c;
     return true;
-  }
-  void weigh(int launches) {  // the last pair taken stands for this many launches
-    if (used) weight[used - 1] = launches;
   }
   ~KernelTimer() {
     for (hipEvent_t e : pool) (void)hipEventDestroy(e);
   }
 };
 
-// a kernel launch, timed when a timer is attached
+// a kernel launch, timed when a timer is attached; `launches`: how many of its
+// class it counts as
 template <class... KA, class... A>
-inline void launch_t(KernelTimer* t, int cls, void (*kernel)(KA...), dim3 grid, dim3 block, uint32_t shm,
+inline void launch_n(KernelTimer* t, int cls, int launches, void (*kernel)(KA...), dim3 grid, dim3 block, uint32_t shm,
                      hipStream_t s, A... args) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  if (t && t->take(cls, &e0, &e1))
+  if (t && t->take(cls, &e0, &e1, launches))
     hipExtLaunchKernelGGL(kernel, grid, block, shm, s, e0, e1, 0, args...);
   else
     hipLaunchKernelGGL(kernel, grid, block, shm, s, args...);
+}
+template <class... KA, class... A>
+inline void launch_t(KernelTimer* t, int cls, void (*kernel)(KA...), dim3 grid, dim3 block, uint32_t shm,
+                     hipStream_t s, A... args) {
+  launch_n(t, cls, 1, kernel, grid, block, shm, s, args...);
 }
 
 // How the tile solves (k_tiles.hip) map a tile's rows to a workgroup: `tpr`
@@ -120,7 +127,9 @@ struct TileMesh {
   int curvCap = 0;
   int4* curvItems = nullptr;
   uint16_t *curvLoc = nullptr, *ringLoc = nullptr, *ringItem = nullptr, *r1Loc = nullptr;
-  bool loop(int precision) const { return on && (precision == 0 ? loop64 : loop32); }
+  bool loop(int precision, const KernelTimer* t) const {
+    return on && (precision == 0 ? loop64 : loop32) && !(t && t->perPass);
+  }
   bool use(int precision) const { return on && (precision == 0 ? ok64 : ok32); }
 };
 

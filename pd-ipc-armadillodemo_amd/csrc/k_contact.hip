@@ -954,7 +954,8 @@ void launch_ccd(const DeviceMesh& m, int nRecs, double filter, int iters, double
              m.toiBits);
     return;
   }
-  hipLaunchKernelGGL(k_pack_moves, dim3((m.nTotal + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nTotal, mv, m.packed);
+  launch_n(m.timer, TC_CCD, 0, k_pack_moves, dim3((m.nTotal + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nTotal, mv,
+           m.packed);
   launch_t(m.timer, TC_CCD, k_ccd, dim3(share_blocks(nRecs)), dim3(kBlock), 0, s, nRecs, m.recs, PackedMoves{m.packed},
            mv, p, m.toiBits);
 }
@@ -1010,8 +1011,8 @@ int launch_collision(DeviceMesh& m, int nRecs, double dhat, double kappa, double
   const ColTerms c{m.ld,    m.nSim, m.actCap, m.recs, m.X,       m.colMass, dhat,
                    kappa, dt,     m.actRec, m.actW, m.actT, m.ptCount, m.counters};
   if (nRecs >= kManyRecs) {
-    hipLaunchKernelGGL(k_pack_points, dim3((m.nTotal + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nTotal, m.ld, m.X,
-                       m.packed);
+    launch_n(m.timer, TC_BARRIER, 0, k_pack_points, dim3((m.nTotal + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m.nTotal,
+             m.ld, m.X, m.packed);
     launch_t(m.timer, TC_BARRIER, k_col_terms, dim3(share_blocks(nRecs)), dim3(kBlock), 0, s, nRecs, m.packed, c);
   } else if (nRecs > 0) {
     launch_t(m.timer, TC_BARRIER, k_col_terms_few, dim3((nRecs + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nRecs, c);

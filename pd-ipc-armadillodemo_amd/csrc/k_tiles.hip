@@ -1145,19 +1145,17 @@ void launch_tile_reset(const DeviceMesh& m, hipStream_t s) {
 }
 
 void launch_tile_solve32(const DeviceMesh& m, int iters, int parity, hipStream_t s) {
-  launch_t(m.timer, TC_SWEEP32, solve32_kernel(m.tile.cfg), dim3(m.tile.nTiles),
+  launch_n(m.timer, TC_SWEEP32, iters - 1, solve32_kernel(m.tile.cfg), dim3(m.tile.nTiles),
            dim3(solve32_threads(m.tile.cfg)), (uint32_t)solve32_lds(m.tile, iters), s, shape_of(m, parity, iters), (const float*)m.m2ValF,
            (const float4*)m.r0, m.X);
-  if (m.timer) m.timer->weigh(iters - 1);
 }
 
 void launch_tile_solve64(const DeviceMesh& m, double w, int iters, int parity, double* out, int64_t outStride,
                          hipStream_t s) {
   const TileFirst ft{m.r1Off, m.r1Col, m.r1Val, m.sysDiag, m.sysRhs, w};
-  launch_t(m.timer, TC_SWEEP64, solve64_kernel(m.tile.cfg), dim3(m.tile.nTiles), dim3(m.tile.cfg.threads),
+  launch_n(m.timer, TC_SWEEP64, iters - 1, solve64_kernel(m.tile.cfg), dim3(m.tile.nTiles), dim3(m.tile.cfg.threads),
            (uint32_t)tile_lds_bytes<double>(m.tile.uCap, iters), s, shape_of(m, parity, iters), (const double*)m.m2Val, ft,
            m.X, out, outStride);
-  if (m.timer) m.timer->weigh(iters - 1);
 }
 
 void launch_tile_adj(const DeviceMesh& m, const TileAdj& g, int parity, hipStream_t s) {
@@ -1200,11 +1198,11 @@ void launch_tile_loop(const DeviceMesh& m, int precision, double w, int passes, 
   g.itStride = itStride;
   const TileShape a = shape_of(m, 0, iters);
   if (precision == 0)
-    hipLaunchKernelGGL(loop_kernel<double>(t.cfg), dim3(t.nTiles), dim3(t.cfg.threads),
-                       tile_loop_lds<double>(t.uCap, t.curvCap, iters), s, a, g, (const double*)m.m2Val);
+    launch_t(m.timer, TC_LOOP, loop_kernel<double>(t.cfg), dim3(t.nTiles), dim3(t.cfg.threads),
+             (uint32_t)tile_loop_lds<double>(t.uCap, t.curvCap, iters), s, a, g, (const double*)m.m2Val);
   else
-    hipLaunchKernelGGL(loop_kernel<float>(t.cfg), dim3(t.nTiles), dim3(t.cfg.threads),
-                       tile_loop_lds<float>(t.uCap, t.curvCap, iters), s, a, g, (const float*)m.m2ValF);
+    launch_t(m.timer, TC_LOOP, loop_kernel<float>(t.cfg), dim3(t.nTiles), dim3(t.cfg.threads),
+             (uint32_t)tile_loop_lds<float>(t.uCap, t.curvCap, iters), s, a, g, (const float*)m.m2ValF);
 }
 
 }  // namespace pdipc

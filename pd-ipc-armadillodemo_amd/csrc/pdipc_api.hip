@@ -470,7 +470,7 @@ void enqueue_local_global(pdipc_handle* h, int withCol) {
   launch_diag(m, withCol, s);
   launch_operators(m, p.omega, p.precision, s);
   if (m.tile.use(p.precision)) launch_tile_reset(m, s);
-  if (m.tile.loop(p.precision) && !m.timer) {  // kernel timing times the passes' kernels one by one
+  if (m.tile.loop(p.precision, m.timer)) {
     launch_tile_loop(m, p.precision, p.omega, p.lg_iters, p.cheb_iters, withCol, nullptr, 0, nullptr, 0, s);
     return;
   }
@@ -831,6 +831,7 @@ int pdipc_kernel_timing(pdipc_handle* h, int enable) {
   delete h->m.timer;  // a new timer starts from zero
   h->m.timer = nullptr;
   if (enable) h->m.timer = new pdipc::KernelTimer();
+  if (enable == 2) h->m.timer->perPass = false;
   return PDIPC_OK;
 }
 

@@ -110,7 +110,7 @@ SIGNATURES = {
 KERNEL_IDS = {"sweep_fp64": 0, "sweep_fp32": 1, "local": 2, "ccd": 3, "operators": 4}
 # classes of pdipc_get_kernel_times, in order
 TIMER_CLASSES = ["sweep_fp64", "sweep_fp32", "rhs", "project", "first_residual", "operators", "ccd", "barrier",
-                 "broad_phase"]
+                 "broad_phase", "lg_loop"]
 
 _lib = None
 
@@ -453,8 +453,10 @@ class Simulator:
 
     def kernel_timing(self, enable=True):
         """In-step kernel timing on (direct launches, each timed kernel's own
-        start/stop recorded) or off; turning it on again starts from zero."""
-        _check(lib().pdipc_kernel_timing(self.h, 1 if enable else 0))
+        start/stop recorded) or off; turning it on again starts from zero.  With
+        2 the passes of a scene that runs them in one launch stay in it (class
+        lg_loop) instead of running as the kernels of the other classes."""
+        _check(lib().pdipc_kernel_timing(self.h, 2 if enable == 2 else 1 if enable else 0))
 
     def kernel_times(self):
         """{class: (summed microseconds, launches)} since timing was enabled."""

@@ -73,3 +73,30 @@ def test_toi_argmin_tracking_changes_nothing():
             active += 1
             assert cb["active_sets"] != 0, k
     assert clamped > 0 and active > 0
+
+
+@pytest.mark.parametrize("prec", [pdipc.FP64, pdipc.FP32_SPLIT])
+def test_timing_of_the_kernels_that_plain_steps_launch(prec):
+    """Timing mode 2 of a cloth scene: one launch per outer iteration for all
+    local/global passes, none of the passes' own kernels; the same bits.  A tet
+    scene's passes run as separate kernels in either mode."""
+    sc = scenes.cloth_over_sphere(24, 2, ground=True, seed=4, patch_dim=24, sphere_patch_dim=12, height=0.16)
+    print(f"case: kernel timing of the passes' launch, precision {prec}", flush=True)
+    a, b = (pdipc.Simulator.from_scene(sc, precision=prec) for _ in range(2))
+    b.kernel_timing(2)
+    outer = 0
+    for _ in range(3):
+        a.step(1)
+        b.step(1)
+        outer += b.counters()["outer_iters"]
+        assert np.array_equal(a.x(), b.x())
+    t = b.kernel_times()
+    assert t["lg_loop"][1] == outer and t["lg_loop"][0] > 0.0
+    assert all(t[k] == (0.0, 0) for k in ("sweep_fp64", "sweep_fp32", "rhs", "project", "first_residual"))
+    b.kernel_timing(True)
+    b.step(1)
+    assert b.kernel_times()["lg_loop"] == (0.0, 0) and b.kernel_times()["rhs"][1] > 0
+    c = pdipc.Simulator.from_scene(scenes.config2(cells=5, cloth_n=12), precision=prec)
+    c.kernel_timing(2)
+    c.step(1)
+    assert c.kernel_times()["lg_loop"] == (0.0, 0) and c.kernel_times()["rhs"][1] == c.counters()["lg_iters"]
