@@ -15,9 +15,10 @@ Measured, each precision from the same state:
     sphere (the outer iterations per step, hence the cost, roughly double);
   * the per-step error of FP32-split against FP64 from identical states;
   * in-step kernel durations (HIP events on every launch, over the timed
-    window re-run with direct launches): the roofline of the FP32 sweep uses
-    the algorithmic bytes (8 B per M^2 entry: an FP32 value and a 32-bit
-    column, plus the row vectors) over that mean.
+    window re-run with direct launches): the roofline is that of the kernel
+    that runs the FP32 sweeps -- all passes of an outer iteration in one launch
+    or a solve per launch where the scene's matrix fits the registers, else the
+    streamed sweep -- and uses its algorithmic bytes over that mean.
 
 Prints one JSON line.  --gpus above 1 exits: the step runs on one GPU.
 """
@@ -89,13 +90,27 @@ def cloth_ring_slots(scene):
     return n
 
 
-def algorithmic_step_bytes(c, ring_slots, outer_per_step, recs_per_step, p_vec, lg=10, cheb=15):
+def tile_bytes(c, ring_slots, loop):
+    """Bytes an FP32 launch of the tile solves cannot do without, each read or
+    written once: per stored M^2 entry its FP32 value and 16-bit LDS index, per
+    point r0 and X in and out; with all passes in one launch (`loop`) the ring
+    and R1 tables (their values and LDS places) and per point X in and out, the
+    inertial and collision rhs, D and the position weight instead."""
+    entries = 6.0 * c["sell_entries"]
+    if not loop:
+        return entries + 64.0 * c["sim_points"]
+    return entries + ring_slots * 38.0 + c["nnz_r1"] * 10.0 + 112.0 * c["sim_points"]
+
+
+def algorithmic_step_bytes(c, ring_slots, outer_per_step, recs_per_step, p_vec, lg=10, cheb=15, tiles=None):
     """Algorithmic HBM bytes of one step (FP32 values,
     int32 indices, p_vec bytes per vector element in the solve and local step,
     FP64 CCD and barrier): per outer iteration the operator update, lg x
     (local step + cheb sweeps), CCD and barrier over the step's candidate
     records K, plus prediction and velocity (4 and 3 vector passes; the broad
-    phase is left out)."""
+    phase is left out).  tiles: None where the sweeps stream the matrix, "solve"
+    where a launch reads it once for the sweeps of a pass, "loop" once for all
+    passes."""
     N, nnz1, nnz2, n2p = c["sim_points"], c["nnz_r1"], c["nnz_r2"], c["n_2paths"]
     D, tot, K = 3 * N, c["total_points"], recs_per_step
     b_spmv = 8 * nnz2 + 4 * D * p_vec
@@ -103,20 +118,32 @@ def algorithmic_step_bytes(c, ring_slots, outer_per_step, recs_per_step, p_vec, 
     b_ops = nnz1 * 12 + n2p * 16 + nnz2 * 16 + N * p_vec
     b_ccd = K * (20 + 24 * 8)
     b_bar = K * (20 + 12 * 8) + 2 * (tot * 8 + 3 * tot * 8)
-    per_outer = b_ops + lg * (b_local + cheb * b_spmv) + b_ccd + b_bar
+    passes = (tile_bytes(c, ring_slots, True) if tiles == "loop" else
+              lg * (b_local + (tile_bytes(c, ring_slots, False) if tiles else cheb * b_spmv)))
+    per_outer = b_ops + passes + b_ccd + b_bar
     return outer_per_step * per_outer + 7 * D * p_vec, b_spmv
 
 
 def kernel_means(sim, x, v, steps):
     """Mean in-step duration (us) and launches per timed class over `steps`
-    steps from (x, v), every launch timed with HIP events (direct launches)."""
-    sim.set_x(x)
-    sim.set_v(v)
-    sim.kernel_timing(True)
-    sim.step(steps)
-    t = sim.kernel_times()
-    sim.kernel_timing(False)
-    return {k: {"mean_us": us / n, "launches": n} for k, (us, n) in t.items() if n}
+    steps from (x, v), every launch timed with HIP events (direct launches).
+    Where the plain steps run all passes of an outer iteration in one launch
+    (lg_loop), the passes' own kernels are timed in a second run that launches
+    them one by one."""
+    res = {}
+    for mode in (2, 1):
+        sim.set_x(x)
+        sim.set_v(v)
+        sim.kernel_timing(mode)
+        sim.step(steps)
+        t = sim.kernel_times()
+        sim.kernel_timing(False)
+        for k, (us, n) in t.items():
+            if n and k not in res:
+                res[k] = {"mean_us": us / n, "launches": n}
+        if "lg_loop" not in res:
+            break
+    return res
 
 
 def stacked_bench(args):
@@ -566,25 +593,43 @@ def main():
     outer32 = res["fp32_split"]["outer"] / steps
     recs32 = float(np.mean(res["fp32_split"]["recs"]))
     slots = cloth_ring_slots(scene)
+    tiles = sims["fp32_split"].tile_solves()
+    form = "loop" if "lg_loop" in kt["fp32_split"] else "solve" if tiles["fp32"] else None
     step_bytes, spmv_bytes = algorithmic_step_bytes(c, slots, outer32, recs32, 4, scene["params"]["lg_iters"],
-                                               scene["params"]["cheb_iters"])
+                                               scene["params"]["cheb_iters"], form)
     sweep = kt["fp32_split"]["sweep_fp32"]
+    timing = (f"mean of {sweep['launches']} in-step launches, HIP events on each launch (pdipc_kernel_timing, the "
+              "timed window with direct launches)")
     staging = sims["fp32_split"].sweep_staging()
     kname, slot_bytes = SWEEP32_KERNELS[staging]
     bytes_formula = "8 B per M^2 entry (FP32 value + int32 column) + 4 vectors x 3N x 4 B"
     stored = c["nnz_r2"] * slot_bytes + 3 * c["sim_points"] * 4.0 * 4
     bytes64 = 8 * c["nnz_r2"] + 4 * 3 * c["sim_points"] * 8
-    # a tile solve reads the matrix once for all its sweeps; times are per sweep
+    # a tile solve reads the matrix once for all its sweeps (its time is given per sweep), a launch of all
+    # passes once for them all
     sweeps = scene["params"]["cheb_iters"] - 1
-    tiles = sims["fp32_split"].tile_solves()
-    if tiles["fp32"] and sweeps > 0:
+    if form == "loop":
+        sweep = kt["fp32_split"]["lg_loop"]
+        kname = ("k_tile_loop (all local/global passes of an outer iteration per launch, M^2 in registers, iterates "
+                 "exchanged)")
+        slot_bytes = 6.0
+        spmv_bytes = stored = tile_bytes(c, slots, True)
+        bytes_formula = ("6 B per stored M^2 entry (FP32 value + 16-bit LDS index), 38 B per ring slot, 10 B per R1 "
+                         "entry and 112 B per point, once per launch; bound by the exchange between tiles, not by "
+                         "these bytes")
+        timing = (f"mean of {sweep['launches']} in-step launches, HIP events on each launch (pdipc_kernel_timing with "
+                  "2, the timed window with direct launches); the sweep and local-step classes of kernel_means_us "
+                  "are of a second run that launches the passes' kernels one by one, as the timed steps do not")
+    elif form == "solve" and sweeps > 0:
         kname = "k_tile_solve32 (a whole FP32 solve per launch, M^2 in registers, iterates exchanged), per sweep"
         slot_bytes = 6.0
-        spmv_bytes = stored = (6.0 * c["sell_entries"] + 64.0 * c["sim_points"]) / sweeps
+        spmv_bytes = stored = tile_bytes(c, slots, False) / sweeps
         bytes_formula = ("per solve 6 B per stored M^2 entry (FP32 value + 16-bit LDS index) and 64 B per point (r0, X "
                          "in and out), over its sweeps; bound by the exchange between tiles, not by these bytes")
-    if tiles["fp64"]:
-        bytes64 = (10.0 * c["sell_entries"] + 96.0 * c["sim_points"]) / (sweeps + 1)
+        timing = (f"in-step solves, HIP events on each launch (pdipc_kernel_timing, the timed window with direct "
+                  f"launches), over their {sweep['launches']} sweeps")
+    if tiles["fp64"] and sweeps > 0:
+        bytes64 = (10.0 * c["sell_entries"] + 96.0 * c["sim_points"]) / sweeps
     ach = spmv_bytes / (sweep["mean_us"] * 1e-6) / 1e9
     matrix_bytes = c["sell_entries"] * slot_bytes
     out = {
@@ -635,20 +680,19 @@ def main():
             "traffic_source": "profiles/k_sweep_config1_hbm_traffic.md: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE "
                               "per launch, scaled by a 1 GiB copy; a recorded constant, not measured in this run",
             "avg_us": sweep["mean_us"],
-            "avg_us_source": f"mean of {sweep['launches']} in-step launches, HIP events on each launch "
-                             "(pdipc_kernel_timing, the timed window with direct launches)",
+            "avg_us_source": timing,
             "bytes_per_launch": spmv_bytes,
             "bytes_formula": bytes_formula,
             "bytes_stored_format": stored,
             "frac_stored_format": stored / (sweep["mean_us"] * 1e-6) / 1e9 / HBM_PEAK_GBS,
             "mall_resident": matrix_bytes < 256e6,
             "mall_note": (f"the M^2 matrix (FP32 values + {int(slot_bytes - 4) * 8}-bit indices, "
-                          f"{matrix_bytes / 1e6:.1f} MB) fits the 256 MB Infinity Cache: after the first sweep it is "
+                          f"{matrix_bytes / 1e6:.1f} MB) fits the 256 MB Infinity Cache: after its first read it is "
                           "served from MALL, so this fraction of HBM peak is not evidence of HBM-bound execution")
                          if matrix_bytes < 256e6 else
                          (f"the M^2 matrix (FP32 values + {int(slot_bytes - 4) * 8}-bit indices, "
-                          f"{matrix_bytes / 1e6:.1f} MB) exceeds the 256 MB Infinity Cache: every sweep streams it "
-                          "from HBM"),
+                          f"{matrix_bytes / 1e6:.1f} MB) exceeds the 256 MB Infinity Cache: every "
+                          f"{'launch' if form else 'sweep'} streams it from HBM"),
             "fp64_sweep": {"avg_us": kt["fp64"]["sweep_fp64"]["mean_us"],
                            "achieved": bytes64
                            / (kt["fp64"]["sweep_fp64"]["mean_us"] * 1e-6) / 1e9},
