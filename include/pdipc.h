@@ -219,7 +219,9 @@ int pdipc_debug_narrow_stage_layout(pdipc_handle* h, long long* sizes, int* tile
 int pdipc_sweep_staging(pdipc_handle* h, int* path);
 
 /* Tile solves: where a scene's system fits the registers of the device (8 lanes
- * per row, sell_stage 1, about 130,000 rows at most) a whole Chebyshev solve is
+ * per row, sell_stage 1; FP32-split up to 262,144 rows on 256 compute units,
+ * FP64 up to 131,072, with more than 64 entries per row up to 131,072 and
+ * 65,536) a whole Chebyshev solve is
  * one launch whose workgroups exchange the iterates; the results are those of
  * the streamed sweeps bit for bit.  info: [0] 1 if this handle has the tables,
  * [1] / [2] 1 if its FP32 / FP64 solves run as tiles, [3] tiles, [4] rows per

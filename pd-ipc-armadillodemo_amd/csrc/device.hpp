@@ -258,8 +258,8 @@ struct DeviceMesh {
 // ---- kernel launch wrappers (all asynchronous on `s`) -------------------------
 // k_step.hip
 void launch_predict(const DeviceMesh& m, double dt, hipStream_t s);
-void launch_diag(const DeviceMesh& m, int withCollision, hipStream_t s);
-void launch_direction(const DeviceMesh& m, hipStream_t s);  // also sets the TOI minimum to 1
+void launch_diag(const DeviceMesh& m, int withCollision, hipStream_t s);  // also sets the TOI minimum to 1
+void launch_direction(const DeviceMesh& m, hipStream_t s);
 // leaves partial sums of the residual; launch_collision adds them up
 void launch_clamp_residual(const DeviceMesh& m, double toiScale, hipStream_t s);
 int residual_partials(const DeviceMesh& m);

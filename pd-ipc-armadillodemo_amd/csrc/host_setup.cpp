@@ -1001,8 +1001,9 @@ void build_solve_tiles(const HostSetup& hs, const SellLayout& L, int maxTiles, S
   T = SolveTiles();
   const int n = hs.nSim;
   if (L.lanes != 8 || n < 1 || maxTiles < 1 || L.sliceOff.back() > INT32_MAX) return;
-  // One tile while a workgroup's own LDS reads cost less than an exchange
-  // (per pass, FP32 / FP64: 144 rows 23 / 39 us, as five tiles 28 / 31); then
+  // One tile while a workgroup's own LDS reads cost less than an exchange in both
+  // precisions, which share the tables (per pass, FP32 / FP64: 144 rows 23 / 39 us,
+  // as five tiles 28 / 31, so FP32 gives 5 us away for FP64's 8); then
   // small tiles until every compute unit has one (rows per tile 32 / 64 / 128,
   // FP64 solves: 64^2 cloth 38 / 40 / 45 us, 13^3-cell tet block 51 / 55 / 58 us),
   // then as many rows as that takes.

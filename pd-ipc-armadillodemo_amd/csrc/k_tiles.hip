@@ -8,8 +8,8 @@
 // of the chip (512 KB per compute unit) hold such a matrix, so here it is read
 // once per solve, and a sweep is LDS reads and FMAs on the tile plus one
 // exchange of the iterate over the Infinity Cache.  Per sweep of a 256^2
-// cloth (256 tiles of 256 rows): about 1 us of LDS reads and 1 us of exchange
-// against 4.7 us (FP32) and 8.6 us (FP64) for the streamed kernels.
+// cloth (256 tiles of 256 rows), loads and launch included: 2.8 us (FP32) and
+// 5.1 (FP64) against 4.7 and 8.6 for the streamed kernels.
 //
 // Tiles: compact in space (recursive bisection of the rest positions, model by
 // model), at most one per compute unit, so that all of them are resident
